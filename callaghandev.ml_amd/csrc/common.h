@@ -61,6 +61,76 @@ __device__ __forceinline__ floatx16 mfma32x32x2(float a, float b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+// fp32 products on the bf16 matrix cores.  An fp32 value is the sum of three
+// bf16 values, h = bf16(x), m = bf16(x - h), l = x - h - m, each rounded to
+// nearest: 8 + 8 + 8 significant bits hold all 24, so the split loses nothing
+// (for |x| above 2^-110; below it l underflows).  Of the nine products of two
+// split operands, hh + hm + mh + mm + hl + lh are summed in fp32; ml, lm and ll
+// are below 2^-24 of |a b| together.  Six bf16 products take 6/16 of one fp32
+// product's matrix-core cycles.
+//
+// The bf16 MFMA adds eight products at a time to its accumulator, one rounding
+// each: with all six products in one accumulator a K of 16 takes 12 roundings
+// of the whole sum, where the fp32 MFMA takes 16, and fewer where operands are
+// zero (behind a ReLU the single-accumulator form came out 8% worse than fp32,
+// so it was not kept).  hh has an accumulator of its own and the five
+// corrections, 2^-8 and less of it, another: two roundings of the whole sum per
+// 16.  Error against float64 (2-norm, N(0, 1) operands, 256 x 256 outputs): K =
+// 64 0.5e-7, 1024 1.9e-7, 8192 5.8e-7, where the fp32 MFMA has 1.4e-7, 5.7e-7 and
+// 16e-7 (positive operands, K = 8192: 4.2e-7 against 11.9e-7).
+//
+// The bf16 MFMA aligns its addends to the largest of them and drops the bits
+// below by rounding down, so a long sum drifts towards minus infinity by about
+// 1e-8 of its size: nothing next to an element's own rounding error, but the
+// same sign in every element, which a column sum over many rows collects (a
+// bias gradient over 130816 rows had 5.8e-6 instead of 4.5e-7).  The kernels
+// therefore compute every other row and column of a product negated (rows and
+// columns of the operands change their sign as they are split, at no cost),
+// which turns the drift round, and undo the sign at the end.
+//
+// An infinity, a NaN or a value above the largest bf16 leaves inf - inf in m,
+// so every result that it reaches comes out non-finite; the kernels test their
+// results for that (any_nonfinite) and recompute such blocks with
+// mfma32x32x2, whose infinities and NaNs are those of the fp32 sum.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t vu2 __attribute__((ext_vector_type(2)));
+typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
+constexpr int kSplitProducts = 6;
+constexpr int kSplitA[kSplitProducts] = {2, 0, 1, 1, 0, 0};  // piece of A (0 = h, 1 = m, 2 = l)
+constexpr int kSplitB[kSplitProducts] = {0, 2, 1, 0, 1, 0};  // piece of B
+constexpr int kSplitMain = 5;                                // hh; the others are its corrections
+
+// (bf16(a), bf16(b)) in the low and high half, rounded to nearest even.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  typedef float vf2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((vf2{a, b}), bf16x2));
+}
+
+// The three pieces of a (low halves) and b (high halves).
+__device__ __forceinline__ void split_bf16x3(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+  h = pack_bf16(a, b);
+  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+  m = pack_bf16(ra, rb);
+  l = pack_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+}
+
+// bf16 MFMA 32x32x16: D = A(32x16) * B(16x32) + C.  Lane l holds eight
+// consecutive k, 8 * (l / 32) + 0..7, of row (A) or column (B) l % 32; D as
+// mfma32x32x2.
+__device__ __forceinline__ floatx16 mfma32x32x16(bf16x8 a, bf16x8 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// 0 when every value of v is finite, NaN otherwise (summed into s).
+__device__ __forceinline__ float nonfinite_sum(const floatx16 &v, float s) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s = fmaf(v[r], 0.f, s);
+  return s;
+}
+// Whether any lane's nonfinite_sum found one (wave-uniform).
+__device__ __forceinline__ bool any_nonfinite(float s) { return __builtin_amdgcn_ballot_w64(s != s) != 0; }
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // The forward attention launcher (flash_attn.hip) for callers that have

@@ -1,5 +1,5 @@
-// fp32 MFMA GEMM for the projections of the attention path and their
-// gradients:
+// fp32 GEMM on the matrix cores for the projections of the attention path and
+// their gradients:
 //   C[m, n] = act(sum_k opA[m, k] * opB[k, n] + bias[n])  (+ C[m, n] when beta)
 // opA is A [M, K] (row stride lda) or, transposed, A stored [K, M]; opB is the
 // weight W [N, K] ([out, in], the reference's layout: y = x W^T) or, for
@@ -12,13 +12,13 @@
 //   bias gradient (row sums of opA = column sums of dY) folded into the
 //   staging of opA.
 //
-// The MFMA inner loop is the same for every layout: both operand tiles sit in
-// LDS as [rows][k] with row pitch BK + 4 floats, and every lane reads its A
-// and B operands as 16-byte LDS reads that feed four v_mfma_f32_32x32x2_f32
-// each.  The reduction index k is visited in the permuted order
-// kappa(s, h) = 8*(s/4) + 4*h + s%4 on both operands, which leaves the sum
-// unchanged.  A transposed operand is transposed on its way into LDS.
+// The main kernel (gemm_tile_kernel) multiplies three bf16 pieces per operand
+// (common.h) and is the same for every layout; a transposed operand is
+// transposed on its way into LDS.  Small and odd shapes have kernels of their
+// own, and gemm_f32_kernel keeps the fp32 MFMA for the pre-activations of ReLU
+// layers.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -28,9 +28,6 @@ namespace {
 constexpr int BM = 128, BN = 128, BK = 32, LDSK = BK + 4;
 constexpr int NTHREADS = 256;
 constexpr int GROUP_M = 8;
-// Epilogue selector of the tiled kernel beyond the activations: no
-// activation, rotary embedding on problems 0 and 1.
-constexpr int kActRope = 100;
 
 struct GemmProblem {
   const float *a;     // opA source
@@ -82,6 +79,7 @@ struct GemmArgs {
   float *pre;
   const float *dz, *add;
   int ldpre, lddz, ldadd, dact;
+  int f32;  // forward: keep the fp32 MFMA (gemm_f32_kernel)
 };
 
 // The value of lane l ^ 1 (a DPP quad permutation [1, 0, 3, 2]).
@@ -180,103 +178,10 @@ __device__ __forceinline__ void store_rope(const GemmArgs &args, const GemmProbl
   }
 }
 
-// The same epilogue with the (cos, sin) table staged through LDS, for full
-// row tiles inside one position segment and head dims 2^(LP+1) (8 .. 64).
-// The k-loop ends on a barrier, so the operand tiles in `tab` (As) are free.
-// Phase i covers block i of every wave row: the workgroup copies the table
-// rows of those WM x 32 output rows into tab[pair * RS + row] with coalesced
-// loads (a thread keeps one pair for all its fetches, so every fetch and LDS
-// write is its base plus a constant), and each lane then reads its (cos, sin)
-// from LDS, which never waits on the stores (a global load issued after a
-// store waits for it: one round trip per group of rows in store_rope).
-// Same arithmetic, same bits as store_rope.
-template <int TM, int WM, int NT, int BI, int BJ, int LP>
-__device__ __forceinline__ void store_rope_lds(const GemmArgs &args, const GemmProblem &P,
-                                               const floatx16 (&acc)[BI][BJ], int mseg, int wm, int mw, int nw,
-                                               int li, int hf, float2 *tab) {
-#pragma clang fp contract(off)
-  constexpr int PAIRS = 1 << LP;
-  constexpr int ROWS = WM * 32;             // table rows per phase
-  constexpr int RS = ROWS + 2;              // pitch of one pair's column (float2)
-  constexpr int STEP = NT / PAIRS;          // rows between a thread's fetches
-  constexpr int KN = ROWS * PAIRS / NT;     // fetches per thread and phase
-  constexpr int WR = TM / WM;               // tile rows per wave row
-  static_assert(KN >= 1 && KN * NT == ROWS * PAIRS && (STEP % 32 == 0 || 32 % STEP == 0), "fetch shape");
-  const int t = threadIdx.x;
-  const int p = t & (PAIRS - 1), q0 = t >> LP;
-  // table row q of a phase is tile row (q / 32) * WR + q % 32 (+ 32 i); for
-  // q = q0 + k * STEP that is the lane's base row plus a constant
-  const int ro0 = STEP <= 32 ? q0 : (q0 >> 5) * WR + (q0 & 31);
-  const float2 *__restrict__ src = args.rope_cs + (size_t)(args.rope_pos0 + mseg + ro0) * PAIRS + p;
-  float2 *wr = tab + p * RS + q0;
-  float2 pre[KN];
-  int n[BJ], pcol[BJ];
-  float bias[BJ];
-  const bool odd = li & 1;  // column parity (nw is a multiple of 32)
-#pragma unroll
-  for (int j = 0; j < BJ; ++j) {
-    n[j] = nw + j * 32 + li;
-    pcol[j] = ((n[j] & (2 * PAIRS - 1)) >> 1) * RS;
-    bias[j] = (P.bias && n[j] < args.N) ? P.bias[n[j]] : 0.f;
-  }
-  const bool full_n = nw + 32 * BJ <= args.N;
-  const float2 *tl = tab + wm * 32 + 4 * hf;  // row 8 (r / 4) + r % 4 of this lane's half
-#pragma unroll
-  for (int i = 0; i < BI; ++i) {
-#pragma unroll
-    for (int k = 0; k < KN; ++k) {
-      const int qk = k * STEP;  // constant
-      const int c = (qk >> 5) * WR + (STEP <= 32 ? (qk & 31) : 0) + 32 * i;
-      pre[k] = src[(size_t)c * PAIRS];
-    }
-    if (i > 0) __syncthreads();  // phase i - 1's reads are done
-#pragma unroll
-    for (int k = 0; k < KN; ++k) wr[k * STEP] = pre[k];
-    __syncthreads();
-    const int mb = mw + i * 32;  // wave-uniform
-    if (full_n) {
-      float *__restrict__ cb = P.c + (size_t)(mb + 4 * hf) * args.ldc;
-      // groups of four rows: the scheduling barrier keeps later groups' LDS
-      // reads from being hoisted (their registers would cost the second
-      // workgroup per CU)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int dr = 8 * g + rr;
-          float *c = cb + (size_t)dr * args.ldc;
-#pragma unroll
-          for (int j = 0; j < BJ; ++j) {
-            const float2 cs = tl[pcol[j] + dr];
-            const float y = acc[i][j][4 * g + rr] + bias[j];
-            const float yp = swap_pair(y);
-            c[n[j]] = odd ? yp * cs.y + y * cs.x : y * cs.x - yp * cs.y;
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int dr = 8 * (r >> 2) + (r & 3);
-        const int m = mb + 4 * hf + dr;
-#pragma unroll
-        for (int j = 0; j < BJ; ++j) {
-          const float2 cs = tl[pcol[j] + dr];
-          const float y = acc[i][j][r] + bias[j];
-          const float yp = swap_pair(y);  // in every lane; only the store is predicated
-          const float out = odd ? yp * cs.y + y * cs.x : y * cs.x - yp * cs.y;
-          if (n[j] < args.N) P.c[(size_t)m * args.ldc + n[j]] = out;
-        }
-      }
-    }
-  }
-}
-
+// 1 / (1 + e^-x) for x >= 0, e^x / (1 + e^x) below, without a branch.
 __device__ __forceinline__ float stable_sigmoid(float x) {
-  if (x >= 0.f) return 1.f / (1.f + expf(-x));
-  const float z = expf(x);
-  return z / (1.f + z);
+  const float z = expf(-fabsf(x));
+  return (x >= 0.f ? 1.f : z) / (1.f + z);
 }
 
 // Activation and derivative codes of the derivative-from-output form
@@ -402,7 +307,10 @@ struct TileStage {
   }
 };
 
-// Guarded fallback of the forward layout (any K, any alignment).
+// Guarded fallback of the forward layout (any K, any alignment) on the fp32
+// MFMA: operand tiles in LDS as [rows][k] with row pitch BK + 4 floats, every
+// lane's operands 16-byte LDS reads that feed four v_mfma_f32_32x32x2_f32 each,
+// k in the permuted order kappa(s, h) = 8*(s/4) + 4*h + s%4 on both operands.
 template <bool VEC, bool EPI>
 __global__ void __launch_bounds__(NTHREADS) gemm_nt_kernel(const GemmArgs args) {
   __shared__ __attribute__((aligned(16))) float As[2][BM][LDSK];
@@ -504,99 +412,343 @@ __global__ void __launch_bounds__(NTHREADS) gemm_nt_kernel(const GemmArgs args) 
   }
 }
 
-// Global -> LDS staging of one ROWS x BKK operand tile of the tiled kernel;
-// the tile lands in LDS as [rows][k] (pitch BKK + 4) for either source layout.
-//   T = false: the source is [rows][K] (k contiguous, row stride ld): each
-//     thread moves 16-byte row pieces straight into LDS.  The F4R lanes of a
-//     row are consecutive; the rows of a wave's 16 are interleaved, so that
-//     consecutive lane quads write rows r, r + 4, r + 8, r + 12, whose 64-byte
-//     pieces fall in disjoint bank ranges at pitch BKK + 4 (rows r and r + 1
-//     share banks: c3's Q/K/V and output projections had 19.2 M and 6.4 M
-//     conflict cycles per dispatch, now 0.5 M and 0, with the matrix pipes
-//     busy 87.2% instead of 85.3% of the Q/K/V product's active cycles).
-//   T = true:  the source is [K][rows] (rows contiguous, k-row stride ld):
-//     each thread loads four consecutive rows of one k and stores them as four
-//     LDS words.  Consecutive lanes take consecutive k, so the four stores of
-//     a wave fall in distinct banks.
-// Each thread's offsets are fixed for the whole K loop; rows past the end are
-// clamped to the last row (T: the last four rows; rows % 4 == 0), so loads
-// need no predication and clamped rows only feed results that are never
+// Global -> LDS staging of one ROWS x 16 operand tile of the tiled kernel,
+// split on the way into its three bf16 pieces (split_bf16x3), one LDS plane
+// each; a row's 16 k-values are 32 contiguous bytes of a plane.
+// Row r of the tile sits in cluster r % NC at place r / NC; odd clusters hold
+// their rows negated (see common.h).
+//   T = false: the source is [rows][K] (k contiguous, row stride ld): a unit
+//     is four k of one row, one 16-byte load and an 8-byte store per plane; a
+//     thread's units come in pairs of neighbouring rows, one in each of NC = 2
+//     clusters, so the stores of a wave cover 512 contiguous bytes.
+//   T = true:  the source is [K][rows] (rows contiguous, k-row stride ld): a
+//     unit is four rows of two k, two 16-byte loads and per row (NC = 4) a
+//     4-byte store per plane, 256 contiguous bytes for eight units.
+// The clusters start 16, 128 and 144 bytes past a multiple of 256, so that
+// the 16-byte pieces of sixteen lanes of an operand read fall in different
+// banks.  Each thread's offsets are fixed for the whole K loop; rows past the
+// end are clamped to the last row (T: the last four rows; rows % 4 == 0), so
+// loads need no predication and clamped rows only feed results that are never
 // stored.
-template <int ROWS, int BKK, int NT, bool T>
+template <int ROWS, int NT, bool T>
 struct OpStage {
-  static constexpr int LD = BKK + 4;
-  static constexpr int F4R = BKK / 4;   // T = false: vectors per row
-  static constexpr int RPP = NT / F4R;  // T = false: rows per pass
-  static constexpr int G = NT / BKK;    // T = true: four-row groups per pass
-  static constexpr int NP = T ? ROWS / (4 * G) : ROWS / RPP;
-  static_assert(NP >= 1 && (T ? ROWS % (4 * G) == 0 : ROWS % RPP == 0), "staging shape");
+  static constexpr int NC = T ? 4 : 2;
+  static constexpr int ROWB = ROWS / NC * 32;              // bytes of one row cluster
+  // Byte offset of cluster c in a plane: 16, 128 and 144 past a multiple of 256.
+  static __device__ __forceinline__ constexpr int cluster(int c) {
+    return c * ROWB + (c & 1) * 16 + (c >> 1) * 128;
+  }
+  static constexpr int PLANE = NC * ROWB + (T ? 256 : 64);  // bytes of one piece
+  static constexpr int BYTES = 3 * PLANE;
+  static constexpr int BLOCK = 32 / NC * 32;               // bytes between 32-row blocks
+  static constexpr int NP = ROWS * (T ? 2 : 4) / NT;       // units per thread
+  static constexpr int NV = T ? 2 * NP : NP;               // their loads
+  static constexpr int SPLITS = 2 * NV;                    // split_bf16x3 calls
+  static constexpr int STORES = T ? 12 * NP : 3 * NP;
+  static_assert(NP >= 1 && ROWS * (T ? 2 : 4) % NT == 0 && (T || NP % 2 == 0), "staging shape");
   uint32_t off[NP];
-  vf4 v[NP];
-  int sa, sb;  // T = false: (row, column); T = true: (k, row group)
+  vf4 v[NV];
+  int sa, sb;  // T = false: (row pair, first k / 4); T = true: (row group, k / 2)
+  int ldk;     // T = true: row stride of the source
 
+  // First tile row of unit i.
+  __device__ __forceinline__ int unit_row(int i) const {
+    return T ? 4 * (sa + NT / 8 * i) : 2 * sa + (i & 1) + NT / 2 * (i >> 1);
+  }
   __device__ __forceinline__ void init(int row0, int rows, int ld) {
     const int t = threadIdx.x;
-    if constexpr (T) {
-      sa = t % BKK;
-      sb = t / BKK;
+    sa = T ? t / 8 : t / 4;
+    sb = T ? t % 8 : t % 4;
+    ldk = ld;
 #pragma unroll
-      for (int i = 0; i < NP; ++i)
-        off[i] = (uint32_t)sa * (uint32_t)ld + (uint32_t)min(row0 + 4 * (sb + G * i), rows - 4);
-    } else {
-      static_assert(F4R == 4 && RPP % 16 == 0, "row interleave");
-      const int q = t / F4R;  // q's 16-row group keeps its rows, taken in the order 0, 4, 8, 12, 1, 5, ...
-      sa = (q & ~15) | ((q & 3) << 2) | ((q >> 2) & 3);
-      sb = (t % F4R) * 4;
-#pragma unroll
-      for (int i = 0; i < NP; ++i) off[i] = (uint32_t)min(row0 + sa + RPP * i, rows - 1) * (uint32_t)ld + sb;
+    for (int i = 0; i < NP; ++i) {
+      if constexpr (T)
+        off[i] = (uint32_t)(2 * sb) * (uint32_t)ld + (uint32_t)min(row0 + unit_row(i), rows - 4);
+      else
+        off[i] = (uint32_t)min(row0 + unit_row(i), rows - 1) * (uint32_t)ld + 4 * sb;
     }
   }
   // First element of k-tile kt.
   static __device__ __forceinline__ const float *tile(const float *x, int kt, int ld) {
-    return T ? x + (size_t)kt * BKK * ld : x + (size_t)kt * BKK;
+    return T ? x + (size_t)kt * 16 * ld : x + (size_t)kt * 16;
   }
   __device__ __forceinline__ void load(const float *__restrict__ base) {
 #pragma unroll
-    for (int i = 0; i < NP; ++i) v[i] = *reinterpret_cast<const vf4 *>(base + off[i]);
-  }
-  __device__ __forceinline__ void store(float (*lds)[LD]) const {
-    if constexpr (T) {
-#pragma unroll
-      for (int i = 0; i < NP; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) lds[4 * (sb + G * i) + c][sa] = v[i][c];
-    } else {
-#pragma unroll
-      for (int i = 0; i < NP; ++i) *reinterpret_cast<vf4 *>(&lds[sa + RPP * i][sb]) = v[i];
+    for (int i = 0; i < NP; ++i) {
+      if constexpr (T) {
+        v[2 * i] = *reinterpret_cast<const vf4 *>(base + off[i]);
+        v[2 * i + 1] = *reinterpret_cast<const vf4 *>(base + off[i] + ldk);
+      } else {
+        v[i] = *reinterpret_cast<const vf4 *>(base + off[i]);
+      }
     }
+  }
+  // The last, ragged k-tile: k at or past kvalid read as zero (T = false:
+  // kvalid % 4 == 0).
+  __device__ __forceinline__ void load_tail(const float *__restrict__ base, int kvalid) {
+    const vf4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if constexpr (T) {
+        v[2 * i] = v[2 * i + 1] = zero;
+        if (2 * sb < kvalid) v[2 * i] = *reinterpret_cast<const vf4 *>(base + off[i]);
+        if (2 * sb + 1 < kvalid) v[2 * i + 1] = *reinterpret_cast<const vf4 *>(base + off[i] + ldk);
+      } else {
+        v[i] = zero;
+        if (4 * sb < kvalid) v[i] = *reinterpret_cast<const vf4 *>(base + off[i]);
+      }
+    }
+  }
+  // FLIP: the values also change their sign bit with `flip` (0 or 1 << 31).
+  template <bool FLIP>
+  __device__ __forceinline__ void store(char *lds, uint32_t flip) const {
+    auto signed_value = [&](float x, bool neg) {
+      if (FLIP) x = __uint_as_float(__float_as_uint(x) ^ flip);
+      return neg ? -x : x;
+    };
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if constexpr (T) {
+        char *d = lds + (sa + NT / 8 * i) * 32 + sb * 4;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          uint32_t h, m, l;
+          split_bf16x3(signed_value(v[2 * i][c], c & 1), signed_value(v[2 * i + 1][c], c & 1), h, m, l);
+          *reinterpret_cast<uint32_t *>(d + cluster(c)) = h;
+          *reinterpret_cast<uint32_t *>(d + cluster(c) + PLANE) = m;
+          *reinterpret_cast<uint32_t *>(d + cluster(c) + 2 * PLANE) = l;
+        }
+      } else {
+        char *d = lds + cluster(i & 1) + (sa + NT / 4 * (i >> 1)) * 32 + sb * 8;
+        uint32_t h0, m0, l0, h1, m1, l1;
+        split_bf16x3(signed_value(v[i][0], i & 1), signed_value(v[i][1], i & 1), h0, m0, l0);
+        split_bf16x3(signed_value(v[i][2], i & 1), signed_value(v[i][3], i & 1), h1, m1, l1);
+        *reinterpret_cast<vu2 *>(d) = vu2{h0, h1};
+        *reinterpret_cast<vu2 *>(d + PLANE) = vu2{m0, m1};
+        *reinterpret_cast<vu2 *>(d + 2 * PLANE) = vu2{l0, l1};
+      }
+    }
+  }
+  // Byte offset of a lane's operand (eight k of row row0 + li) in a plane.
+  static __device__ __forceinline__ int operand(int row0, int li, int hf) {
+    return cluster(li % NC) + (row0 / NC + li / NC) * 32 + hf * 16;
   }
 };
 
-// Tiled fast path (K % BKK == 0, 16-byte aligned rows, element offsets
-// below 2^32; a transposed operand also needs rows % 4 == 0).  A workgroup of
-// WM x WN waves computes a TM x TN tile of C, each wave a (TM/WM) x (TN/WN)
-// block of 32x32 MFMA tiles.  K advances by BKK through double-buffered LDS.
-// The LDS operands of group u + 1 are read while the MFMAs of group u run, and
-// the k-tile after next is fetched while the current one is consumed.
-// Measured on MI355X, high occupancy (four waves per SIMD with two 512-thread
-// workgroups per CU) hides latency better than deeper register blocking.
+// A wave's BI x BJ blocks recomputed on the fp32 MFMA straight from memory,
+// one block after the other: only for blocks whose split products came out
+// non-finite (an infinity, a NaN, a value above the largest bf16, or a sum that
+// overflows), so that they hold what the fp32 sum gives.  k runs over [k0, k1)
+// of each of nseg operand pairs.
+template <int BI, int BJ, bool TA, bool TB>
+__device__ __forceinline__ void recompute_blocks(const GemmArgs &args, int prob, int nseg, int k0, int k1, int mw,
+                                                 int nw, int li, int hf, floatx16 (&acc)[BI][BJ]) {
+#pragma unroll
+  for (int i = 0; i < BI; ++i) {
+    const size_t m = min(mw + i * 32 + li, args.M - 1);
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) {
+      const size_t n = min(nw + j * 32 + li, args.N - 1);
+      floatx16 c = {};
+#pragma unroll 1
+      for (int s = 0; s < nseg; ++s) {
+        const float *A = args.p[prob + s].a, *W = args.p[prob + s].w;
+#pragma unroll 1
+        for (int k = k0; k < k1; k += 2) {
+          const size_t kk = min(k + hf, k1 - 1);
+          const float av = A[TA ? kk * args.lda + m : m * args.lda + kk];
+          const float bv = W[TB ? kk * args.ldb + n : n * args.ldb + kk];
+          const bool in = k + hf < k1;
+          c = mfma32x32x2(in ? av : 0.f, in ? bv : 0.f, c);
+        }
+      }
+      acc[i][j] = c;
+    }
+  }
+}
+
+// Where a wave's blocks go: C (or a split-K partial, which takes neither bias
+// nor activation nor beta).
+struct TileOut {
+  float *c;
+  int ldc;
+  const float *bias;
+  int act, beta;
+  bool rope;
+};
+
+// Epilogue of a wave's BI x BJ blocks through `lds` (32 * (32 * BJ + 4) floats
+// of the wave's own; the k-loop has ended on a barrier, so the operand tiles
+// are free): one 32-row band at a time is laid down as the MFMA holds it and
+// read back as rows, so that a lane has four consecutive columns: bias,
+// activation, training options (EPI) and stores take 16-byte accesses where
+// the strides allow them, and both halves of a rotary pair are in one lane.
+// The operands of four rows are loaded before any of their stores (a load
+// issued after a store waits for it).  The loop over rows is rolled, so the
+// activations cost no code per register (unrolled over the accumulators they
+// took the kernels into scratch memory).
+template <int BI, int BJ, bool EPI, bool ROPE>
+__device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &out,
+                                           const floatx16 (&acc)[BI][BJ], int mw, int nw, int lane, float *lds) {
+#pragma clang fp contract(off)
+  constexpr int PITCH = 32 * BJ + 4;
+  constexpr int RPI = 8 / BJ;  // rows per step of the wave (8 BJ lanes hold a row)
+  constexpr int GROUP = 4;     // steps whose loads run ahead of their stores
+  static_assert(8 % BJ == 0 && 32 % (GROUP * RPI) == 0, "epilogue shape");
+  const int M = args.M, N = args.N;
+  const int li = lane & 31, hf = lane >> 5;
+  const int n = nw + 4 * (lane % (8 * BJ)), r0 = lane / (8 * BJ);
+  bool vec = N % 4 == 0 && out.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(out.c) & 15) == 0;
+  if (EPI) {
+    if (args.pre) vec = vec && args.ldpre % 4 == 0 && (reinterpret_cast<uintptr_t>(args.pre) & 15) == 0;
+    if (args.dz) vec = vec && args.lddz % 4 == 0 && (reinterpret_cast<uintptr_t>(args.dz) & 15) == 0;
+    if (args.add) vec = vec && args.ldadd % 4 == 0 && (reinterpret_cast<uintptr_t>(args.add) & 15) == 0;
+  }
+  auto get = [&](auto full, const float *p) {  // four columns from n, zero past N
+    vf4 x = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (decltype(full)::value) {
+      x = *reinterpret_cast<const vf4 *>(p);
+    } else if (vec) {
+      if (n < N) x = *reinterpret_cast<const vf4 *>(p);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) x[c] = p[c];
+    }
+    return x;
+  };
+  auto put = [&](auto full, float *p, vf4 x) {
+    if constexpr (decltype(full)::value) {
+      *reinterpret_cast<vf4 *>(p) = x;
+    } else if (vec) {
+      if (n < N) *reinterpret_cast<vf4 *>(p) = x;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) p[c] = x[c];
+    }
+  };
+  vf4 bias = {0.f, 0.f, 0.f, 0.f};
+  if (out.bias) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (n + c < N) bias[c] = out.bias[n + c];
+  }
+  // rotary pairs of columns n, n + 1 and n + 2, n + 3 in their heads
+  const bool rope = ROPE && out.rope;
+  int p0 = 0, p1 = 0, pairs = 0;
+  if (rope) {
+    pairs = args.rope_hd >> 1;
+    p0 = (n % args.rope_hd) >> 1;
+    p1 = ((n + 2) % args.rope_hd) >> 1;
+  }
+#pragma unroll 1
+  for (int i = 0; i < BI; ++i) {
+#pragma unroll
+    for (int ii = 0; ii < BI; ++ii)
+      if (ii == i) {  // the accumulators need constant indices, the loop's body only one copy
+#pragma unroll
+        for (int j = 0; j < BJ; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) lds[(8 * (r >> 2) + 4 * hf + (r & 3)) * PITCH + j * 32 + li] = acc[ii][j][r];
+      }
+    auto rows = [&](auto full) {
+      constexpr bool FULL = decltype(full)::value;  // every row and column exists, 16-byte accesses
+#pragma unroll 1
+    for (int g = 0; g < 32; g += GROUP * RPI) {
+      vf4 z[GROUP], zv[GROUP], av[GROUP], old[GROUP];
+      float2 t0[GROUP], t1[GROUP];
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) {
+        const int row = g + u * RPI + r0, m = mw + i * 32 + row;
+        z[u] = *reinterpret_cast<const vf4 *>(&lds[row * PITCH + (n - nw)]);
+        if (FULL || m < M) {
+          if (EPI && args.dz) zv[u] = get(full, args.dz + (size_t)m * args.lddz + n);
+          if (EPI && args.add) av[u] = get(full, args.add + (size_t)m * args.ldadd + n);
+          if (out.beta) old[u] = get(full, out.c + (size_t)m * out.ldc + n);
+          if (ROPE && rope && (FULL || n < N)) {
+            const int pos = args.rope_pos0 + (args.rope_seg > 0 ? m % args.rope_seg : m);
+            const float2 *cs = args.rope_cs + (size_t)pos * pairs;
+            t0[u] = cs[p0];
+            t1[u] = cs[p1];
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) {
+        const int row = g + u * RPI + r0, m = mw + i * 32 + row;
+        if (!FULL && m >= M) continue;
+        vf4 v;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = z[u][c] + bias[c];
+        if (EPI && args.pre) put(full, args.pre + (size_t)m * args.ldpre + n, v);
+        if (!ROPE && out.act != CDML_ACT_NONE) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = activate(v[c], out.act);
+        }
+        if (EPI && args.dz) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] *= act_deriv(zv[u][c], args.dact);
+        }
+        if (EPI && args.add) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] += av[u][c];
+        }
+        if (ROPE && rope) {
+          // each rotation product rounded before the sum, as the reference
+          // (AccelerationCPU.cs:4947-4975) and the in-place rope kernels
+          // evaluate it: no fused multiply-add
+          v = vf4{v[0] * t0[u].x - v[1] * t0[u].y, v[0] * t0[u].y + v[1] * t0[u].x,
+                  v[2] * t1[u].x - v[3] * t1[u].y, v[2] * t1[u].y + v[3] * t1[u].x};
+        }
+        if (out.beta) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = old[u][c] + v[c];
+        }
+        put(full, out.c + (size_t)m * out.ldc + n, v);
+      }
+    }
+    };
+    if (vec && mw + (i + 1) * 32 <= M && nw + 32 * BJ <= N) rows(std::true_type{});
+    else rows(std::false_type{});
+  }
+}
+
+// Tiled kernel (16-byte aligned rows, element offsets below 2^32; K % 4 == 0
+// where an operand is [rows][K], rows % 4 == 0 where it is [K][rows]).  A
+// workgroup of WM x WN waves computes a TM x TN tile of C, each wave a
+// (TM/WM) x (TN/WN) block of 32x32 tiles on the bf16 MFMA, both operands split
+// into three bf16 pieces on their way into LDS (common.h).  K advances by 16
+// through NB LDS buffers; the k-tile after the last staged one is fetched into
+// registers while the current one is multiplied.
+//
+// With NB = 3 the next k-tile is complete in LDS while the current one is
+// multiplied, so the operands of its first product are read before the
+// barrier, and the split (VALU) and LDS instructions are spread between the
+// MFMAs by scheduling groups; with NB = 2 (small tiles) several workgroups per
+// CU hide each other's staging.  Measured on MI355X, 128 x 128 tiles
+// (fp32-equivalent TFLOP/s, forward, dX and dW of 16384 x 4096 x 1024): 194, 182
+// and 183, where the fp32 MFMA form that this replaces had 138, 128 and 131.  The
+// library's own bf16 product reaches 1170-1340 TFLOP/s, a sixth of which is
+// 195-223: the power of the matrix cores bounds both (a loop of MFMAs alone on
+// random data runs at 1.8 of 2.4 GHz; on zeros this kernel takes 274).  256 x 256
+// tiles would take 208-229 with one accumulator (see common.h); the registers do
+// not hold two.
 //
 // With TA and a bias-gradient pointer, the workgroups of the first column
-// tile also sum each opA tile in LDS while it is current (every valid k-tile
-// exactly once) and add the row sums to bgrad: the bias gradient of a
-// weight-gradient GEMM costs no extra pass over dY.  Each thread keeps one
-// partial sum (row t % TM, a 1/(NT/TM) slice of the k-tile); the slices meet
-// in LDS at the end.
-template <int TM, int TN, int BKK, int WM, int WN, int MINB, int ACT, bool TA, bool TB, bool EPI>
+// tile also sum the opA values that they stage (every k once) and add the row
+// sums to bgrad: the bias gradient of a weight-gradient GEMM costs no extra
+// pass over dY.  Each thread sums its own k pair of its rows; the eight k pairs
+// of a row sit in neighbouring lanes.
+template <int TM, int TN, int WM, int WN, int MINB, int NB, bool ROPE, bool TA, bool TB, bool EPI>
 __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const GemmArgs args) {
   constexpr int NT = 64 * WM * WN;
-  constexpr int LD = BKK + 4;
   constexpr int BI = TM / WM / 32, BJ = TN / WN / 32;
-  static_assert(BI >= 1 && BJ >= 1, "tile shape");
-  typedef OpStage<TM, BKK, NT, TA> StageA;
-  typedef OpStage<TN, BKK, NT, TB> StageB;
-  __shared__ __attribute__((aligned(16))) float As[2][TM][LD];
-  __shared__ __attribute__((aligned(16))) float Bs[2][TN][LD];
+  static_assert(BI >= 1 && BJ >= 1 && (NB == 2 || NB == 3), "tile shape");
+  typedef OpStage<TM, NT, TA> StageA;
+  typedef OpStage<TN, NT, TB> StageB;
+  __shared__ __attribute__((aligned(16))) char smem[NB * (StageA::BYTES + StageB::BYTES)];
+  char *const As = smem, *const Bs = smem + NB * StageA::BYTES;
 
   int lid = xcd_remap(blockIdx.x, args.padded);
   if (lid >= args.total) return;
@@ -616,11 +768,7 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
   const int gsize = min(args.tiles_m - first_m, GROUP_M);
   const int tm = first_m + (lid % in_group) % gsize;
   const int tn_all = (lid % in_group) / gsize;
-  // The RoPE instance keeps the problem index in a scalar register (the
-  // divisions above run on the vector unit; left there, the values it keeps
-  // for the staged-table epilogue cost its k-loop the VGPRs of the second
-  // workgroup per CU).  Other instances allocate better without the hint.
-  const int prob = ACT == kActRope ? __builtin_amdgcn_readfirstlane(tn_all / args.tiles_n) : tn_all / args.tiles_n;
+  const int prob = __builtin_amdgcn_readfirstlane(tn_all / args.tiles_n);
   const int tn = tn_all % args.tiles_n;
 
   const GemmProblem P = args.p[prob];
@@ -632,11 +780,265 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int li = lane & 31, hf = lane >> 5;
+  const int mw = m0 + wm * (TM / WM), nw = n0 + wn * (TN / WN);
 
   StageA sa;
   StageB sb;
   sa.init(m0, M, args.lda);
   sb.init(n0, N, args.ldb);
+  floatx16 acc[BI][BJ], cor[BI][BJ];  // hh, and the five corrections
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = cor[i][j][r] = 0.f;
+  const int kt0 = chunk * args.kchunk;
+  const int nk = args.ksplit > 1 ? min(args.kchunk, K / 16 - kt0) : K / 16;
+  const int ktail = args.ksplit > 1 ? 0 : K % 16;  // split-K: the reduce adds the ragged rows
+  const float *__restrict__ A = StageA::tile(P.a, kt0, args.lda);
+  const float *__restrict__ W = StageB::tile(P.w, kt0, args.ldb);
+  // K segments exist only in the plain input-gradient instance; the segment of
+  // k-tile kt is wave-uniform, so choosing it takes scalar selects only.
+  constexpr bool SEG = TB && !TA && !EPI;
+  auto load = [&](int kt) {
+    if (SEG && args.kseg > 0) {
+      const int sg = (kt >= args.kseg) + (kt >= 2 * args.kseg);
+      const int kl = kt - sg * args.kseg;
+      sa.load(StageA::tile(sg == 0 ? args.p[0].a : sg == 1 ? args.p[1].a : args.p[2].a, kl, args.lda));
+      sb.load(StageB::tile(sg == 0 ? args.p[0].w : sg == 1 ? args.p[1].w : args.p[2].w, kl, args.ldb));
+    } else {
+      sa.load(StageA::tile(A, kt, args.lda));
+      sb.load(StageB::tile(W, kt, args.ldb));
+    }
+  };
+  const bool bsum = TA && P.bgrad && tn == 0;
+  float bpart[TA ? 4 * StageA::NP : 1];
+  if constexpr (TA) {
+#pragma unroll
+    for (int i = 0; i < 4 * StageA::NP; ++i) bpart[i] = 0.f;
+  }
+  auto add_bias = [&]() {
+    if constexpr (TA) {
+#pragma unroll
+      for (int i = 0; i < StageA::NP; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) bpart[4 * i + c] += sa.v[2 * i][c] + sa.v[2 * i + 1][c];
+    }
+  };
+  // Split-K chunks take turns in the sign of opA: the drift of the partial
+  // sums (common.h) would otherwise add up over the chunks.
+  constexpr bool FLIP = TA && TB;
+  const uint32_t flip = FLIP ? (uint32_t)(chunk & 1) << 31 : 0;
+  auto stage = [&](int buf) {
+    sa.template store<FLIP>(As + buf * StageA::BYTES, flip);
+    sb.template store<false>(Bs + buf * StageB::BYTES, 0);
+  };
+  const int ao = StageA::operand(wm * (TM / WM), li, hf), bo = StageB::operand(wn * (TN / WN), li, hf);
+  bf16x8 a[3][BI], b[3][BJ];
+  auto read_a = [&](int p, int buf) {
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+      a[p][i] = *reinterpret_cast<const bf16x8 *>(As + buf * StageA::BYTES + p * StageA::PLANE + ao +
+                                                  i * StageA::BLOCK);
+  };
+  auto read_b = [&](int p, int buf) {
+#pragma unroll
+    for (int j = 0; j < BJ; ++j)
+      b[p][j] = *reinterpret_cast<const bf16x8 *>(Bs + buf * StageB::BYTES + p * StageB::PLANE + bo +
+                                                  j * StageB::BLOCK);
+  };
+  auto product = [&](int q) {
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) {
+        floatx16 &c = q == kSplitMain ? acc[i][j] : cor[i][j];
+        c = mfma32x32x16(a[kSplitA[q]][i], b[kSplitB[q]][j], c);
+      }
+  };
+
+  if (nk > 0) {
+    // k-tiles 0 .. NB - 2 -> LDS, k-tile NB - 1 -> registers.  Past the end
+    // (here and in the loop) loads and stages repeat the last tile into a
+    // buffer that nothing reads again: unconditional, they keep the staging
+    // registers out of scratch memory.
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      load(min(i, nk - 1));
+      if (i < NB - 1) {
+        if (TA && bsum && i < nk) add_bias();
+        stage(i);
+      }
+    }
+    __syncthreads();
+    if constexpr (NB == 3) {
+      read_a(2, 0);
+      read_b(0, 0);
+    }
+    int cur = 0;
+#pragma unroll 1
+    for (int kt = 0; kt < nk; ++kt) {
+      const int nxt = cur + 1 < NB ? cur + 1 : 0;
+      const int st = NB == 2 ? nxt : (nxt + 1 < NB ? nxt + 1 : 0);  // the buffer k-tile kt - 1 has left
+      if (TA && bsum && kt + NB - 1 < nk) add_bias();
+      if constexpr (NB == 2) {
+        read_a(2, cur);
+        read_b(0, cur);
+      }
+      read_a(0, cur);
+      read_b(2, cur);
+      read_a(1, cur);
+      read_b(1, cur);
+      product(0);
+      product(1);
+      stage(st);
+      load(min(kt + NB, nk - 1));
+      product(2);
+      product(3);
+      product(4);
+      product(5);
+      if constexpr (NB == 3) {
+        read_a(2, nxt);
+        read_b(0, nxt);
+        constexpr int NM = kSplitProducts * BI * BJ;
+        constexpr int NR = 2 * (BI + BJ);  // reads between the first MFMAs, then the stores
+        constexpr int VALU = (11 * (StageA::SPLITS + StageB::SPLITS) + NM - 1) / NM + 1;
+        constexpr int STORES = StageA::STORES + StageB::STORES;
+        constexpr int AT_ONCE = (STORES + NM - NR - 1) / (NM - NR);
+        constexpr int EVERY = STORES > (NM - NR) / 2 ? 1 : 2;
+#pragma unroll
+        for (int q = 0; q < NM; ++q) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);  // VALU
+          if (q < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                             // LDS read
+          else if (q % EVERY == EVERY - 1) __builtin_amdgcn_sched_group_barrier(0x200, AT_ONCE, 0);  // LDS write
+        }
+      }
+      __syncthreads();
+      cur = nxt;
+    }
+  }
+  if (ktail) {  // uniform over the workgroup
+    sa.load_tail(StageA::tile(A, nk, args.lda), ktail);
+    sb.load_tail(StageB::tile(W, nk, args.ldb), ktail);
+    if (TA && bsum) add_bias();
+    stage(0);
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      read_a(p, 0);
+      read_b(p, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < kSplitProducts; ++q) product(q);
+    __syncthreads();
+  }
+  {
+    // rows and columns of odd index were negated (rows 8 (r / 4) + 4 hf + r % 4)
+    const uint32_t s0 = ((uint32_t)(li & 1) << 31) ^ flip, s1 = s0 ^ (1u << 31);
+    float bad = 0.f;
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[i][j][r] = __uint_as_float(__float_as_uint(acc[i][j][r] + cor[i][j][r]) ^ (r & 1 ? s1 : s0));
+        bad = nonfinite_sum(acc[i][j], bad);
+      }
+    if (any_nonfinite(bad)) {
+      const bool seg = SEG && args.kseg > 0;
+      recompute_blocks<BI, BJ, TA, TB>(args, seg ? 0 : prob, seg ? 3 : 1, seg ? 0 : kt0 * 16,
+                                       seg ? args.kseg * 16 : kt0 * 16 + nk * 16 + ktail, mw, nw, li, hf, acc);
+    }
+  }
+
+  if constexpr (TA) {
+    if (bsum) {
+      // the eight k pairs of four rows are lanes 8 g .. 8 g + 7
+#pragma unroll
+      for (int i = 0; i < StageA::NP; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          float s = bpart[4 * i + c];
+#pragma unroll
+          for (int off = 4; off > 0; off >>= 1) s += __shfl_xor(s, off);
+          const int m = m0 + sa.unit_row(i) + c;
+          if (sa.sb == 0 && m < M) {
+            if (args.ksplit > 1)
+              args.wsb[((size_t)chunk * args.nprob + prob) * M + m] = s;
+            else
+              P.bgrad[m] += s;
+          }
+        }
+    }
+  }
+  float *band = reinterpret_cast<float *>(smem) + wave * 32 * (32 * BJ + 4);
+  static_assert(sizeof(smem) >= sizeof(float) * WM * WN * 32 * (32 * BJ + 4), "epilogue bands");
+  TileOut out{P.c, args.ldc, P.bias, args.act, args.beta, ROPE && prob < 2};
+  if (TA && args.ksplit > 1)  // the partial product of this chunk, reduced later
+    out = TileOut{args.ws + ((size_t)chunk * args.nprob + prob) * (size_t)M * N, N, nullptr, CDML_ACT_NONE, 0, false};
+  store_tile<BI, BJ, EPI, ROPE>(args, out, acc, mw, nw, lane, band);
+}
+
+// Forward product on the fp32 MFMA (K % 16 == 0, 16-byte aligned rows, element
+// offsets below 2^32), for the pre-activations of ReLU and leaky ReLU layers
+// that train (GemmArgs::f32): the sign of z picks the derivative, so a z within
+// rounding of 0 moves a whole row of the layer below's gradient by up to a
+// tenth of its rms when its last bits change; these products keep the bits they
+// have always had.  fp32-equivalent 116-138 TFLOP/s against the split kernel's
+// 160-199.
+//
+// Both operand tiles sit in LDS as [rows][16] with pitch 20 floats, double
+// buffered; lanes read 16-byte operands that feed four v_mfma_f32_32x32x2_f32
+// each, so k is visited in the order 8 (s / 4) + 4 h + s % 4.  The rows of a
+// wave's 16 are stored in the order 0, 4, 8, 12, 1, 5, ..., whose 64-byte
+// pieces fall in disjoint banks.
+template <int TM, int TN, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArgs args) {
+  constexpr int NT = 64 * WM * WN, BKK = 16, LD = BKK + 4;
+  constexpr int BI = TM / WM / 32, BJ = TN / WN / 32;
+  constexpr int RPP = NT / 4, NA = TM / RPP, NB = TN / RPP;
+  constexpr int TILES = 2 * (TM + TN) * LD, BANDS = WM * WN * 32 * (32 * BJ + 4);
+  __shared__ __attribute__((aligned(16))) float smem[TILES > BANDS ? TILES : BANDS];
+  float(*const As)[LD] = reinterpret_cast<float(*)[LD]>(smem);  // buffer b: rows [b TM, (b + 1) TM)
+  float(*const Bs)[LD] = reinterpret_cast<float(*)[LD]>(smem + 2 * TM * LD);
+
+  const int lid = xcd_remap(blockIdx.x, args.padded);
+  if (lid >= args.total) return;
+  const int in_group = GROUP_M * args.tiles_n;
+  const int group = lid / in_group;
+  const int first_m = group * GROUP_M;
+  const int gsize = min(args.tiles_m - first_m, GROUP_M);
+  const int tm = first_m + (lid % in_group) % gsize;
+  const int tn = (lid % in_group) / gsize;
+  const GemmProblem P = args.p[0];
+  const int m0 = tm * TM, n0 = tn * TN;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int li = lane & 31, hf = lane >> 5;
+
+  const int q = t / 4, row = (q & ~15) | ((q & 3) << 2) | ((q >> 2) & 3), col = (t % 4) * 4;
+  uint32_t offa[NA], offb[NB];
+  vf4 va[NA], vb[NB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) offa[i] = (uint32_t)min(m0 + row + RPP * i, args.M - 1) * (uint32_t)args.lda + col;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) offb[i] = (uint32_t)min(n0 + row + RPP * i, args.N - 1) * (uint32_t)args.ldb + col;
+  auto load = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) va[i] = *reinterpret_cast<const vf4 *>(P.a + (size_t)kt * BKK + offa[i]);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) vb[i] = *reinterpret_cast<const vf4 *>(P.w + (size_t)kt * BKK + offb[i]);
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) *reinterpret_cast<vf4 *>(&As[buf * TM + row + RPP * i][col]) = va[i];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) *reinterpret_cast<vf4 *>(&Bs[buf * TN + row + RPP * i][col]) = vb[i];
+  };
   floatx16 acc[BI][BJ];
 #pragma unroll
   for (int i = 0; i < BI; ++i)
@@ -644,247 +1046,38 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
     for (int j = 0; j < BJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  const int kt0 = chunk * args.kchunk;
-  const int nk = args.ksplit > 1 ? min(args.kchunk, K / BKK - kt0) : K / BKK;
-  const float *__restrict__ A = StageA::tile(P.a, kt0, args.lda);
-  const float *__restrict__ W = StageB::tile(P.w, kt0, args.ldb);
-  // K segments exist only in the plain input-gradient instance (in the
-  // epilogue instances their selects would cost the registers of the second
-  // workgroup per CU); the segment of k-tile kt is wave-uniform, so choosing
-  // it takes scalar selects only.
-  constexpr bool SEG = TB && !TA && !EPI;
-  const bool seg = SEG && args.kseg > 0;
-  auto load_seg = [&](int kt) {
-    const int sg = (kt >= args.kseg) + (kt >= 2 * args.kseg);
-    const int kl = kt - sg * args.kseg;
-    sa.load(StageA::tile(sg == 0 ? args.p[0].a : sg == 1 ? args.p[1].a : args.p[2].a, kl, args.lda));
-    sb.load(StageB::tile(sg == 0 ? args.p[0].w : sg == 1 ? args.p[1].w : args.p[2].w, kl, args.ldb));
-  };
-  const bool bsum = TA && P.bgrad && tn == 0;
-  constexpr int KCH = NT / TM;  // k slices per row for the bias-gradient sums
-  static_assert(NT % TM == 0 && BKK % (4 * KCH) == 0, "bias-gradient slices");
-  float bpart = 0.f;
-
-  // k-tile 0 -> LDS, k-tile 1 -> registers
-  if (SEG && seg) {
-    load_seg(0);
-  } else {
-    sa.load(StageA::tile(A, 0, args.lda));
-    sb.load(StageB::tile(W, 0, args.ldb));
-  }
-  sa.store(As[0]);
-  sb.store(Bs[0]);
-  {
-    const int k1 = min(1, nk - 1);
-    if (SEG && seg) {
-      load_seg(k1);
-    } else {
-      sa.load(StageA::tile(A, k1, args.lda));
-      sb.load(StageB::tile(W, k1, args.ldb));
-    }
-  }
+  const int nk = args.K / BKK;
+  load(0);
+  stage(0);
+  load(min(1, nk - 1));
   __syncthreads();
-
+#pragma unroll 1
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
-    const float(*as)[LD] = &As[cur][wm * (TM / WM) + li];
-    const float(*bsh)[LD] = &Bs[cur][wn * (TN / WN) + li];
-    vf4 a4[BI], b4[BJ];
-#pragma unroll
-    for (int i = 0; i < BI; ++i) a4[i] = *reinterpret_cast<const vf4 *>(&as[i * 32][hf * 4]);
-#pragma unroll
-    for (int j = 0; j < BJ; ++j) b4[j] = *reinterpret_cast<const vf4 *>(&bsh[j * 32][hf * 4]);
+    const float(*as)[LD] = &As[cur * TM + wm * (TM / WM) + li];
+    const float(*bs)[LD] = &Bs[cur * TN + wn * (TN / WN) + li];
 #pragma unroll
     for (int u = 0; u < BKK / 8; ++u) {
-      vf4 an[BI], bn[BJ];
-      if (u + 1 < BKK / 8) {
+      vf4 a4[BI], b4[BJ];
 #pragma unroll
-        for (int i = 0; i < BI; ++i) an[i] = *reinterpret_cast<const vf4 *>(&as[i * 32][(u + 1) * 8 + hf * 4]);
+      for (int i = 0; i < BI; ++i) a4[i] = *reinterpret_cast<const vf4 *>(&as[i * 32][u * 8 + hf * 4]);
 #pragma unroll
-        for (int j = 0; j < BJ; ++j) bn[j] = *reinterpret_cast<const vf4 *>(&bsh[j * 32][(u + 1) * 8 + hf * 4]);
-      }
+      for (int j = 0; j < BJ; ++j) b4[j] = *reinterpret_cast<const vf4 *>(&bs[j * 32][u * 8 + hf * 4]);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int i = 0; i < BI; ++i)
 #pragma unroll
           for (int j = 0; j < BJ; ++j) acc[i][j] = mfma32x32x2(a4[i][r], b4[j][r], acc[i][j]);
-      if (u + 1 < BKK / 8) {
-#pragma unroll
-        for (int i = 0; i < BI; ++i) a4[i] = an[i];
-#pragma unroll
-        for (int j = 0; j < BJ; ++j) b4[j] = bn[j];
-      }
     }
-    // Stage k-tile kt + 1 (already in registers) and fetch k-tile kt + 2.
-    // Past the end both are unconditional re-stages of the last tile into
-    // the idle buffer, which nothing reads again: keeping them unconditional
-    // keeps the staging registers out of scratch memory.
-    sa.store(As[cur ^ 1]);
-    sb.store(Bs[cur ^ 1]);
-    if constexpr (TA) {
-      if (bsum) {  // k-tile kt, stable in As[cur] until the barrier below
-        const float *row = &As[cur][t % TM][(t / TM) * (BKK / KCH)];
-#pragma unroll
-        for (int e = 0; e < BKK / KCH; e += 4) {
-          const vf4 x = *reinterpret_cast<const vf4 *>(row + e);
-          bpart += (x[0] + x[1]) + (x[2] + x[3]);
-        }
-      }
-    }
-    const int k2 = min(kt + 2, nk - 1);
-    if (SEG && seg) {
-      load_seg(k2);
-    } else {
-      sa.load(StageA::tile(A, k2, args.lda));
-      sb.load(StageB::tile(W, k2, args.ldb));
-    }
+    // past the end both repeat the last tile into the idle buffer
+    stage(cur ^ 1);
+    load(min(kt + 2, nk - 1));
     __syncthreads();
   }
-
-  if constexpr (TA) {
-    if (bsum) {  // uniform over the workgroup; the loop ended on a barrier
-      float *red = &As[0][0][0];
-      red[t] = bpart;
-      __syncthreads();
-      if (t < TM && m0 + t < M) {
-        float s = 0.f;
-#pragma unroll
-        for (int c = 0; c < KCH; ++c) s += red[t + c * TM];
-        if (args.ksplit > 1)
-          args.wsb[((size_t)chunk * args.nprob + prob) * M + m0 + t] = s;
-        else
-          P.bgrad[m0 + t] += s;
-      }
-    }
-    if (args.ksplit > 1) {  // the partial product of this chunk, reduced later
-      float *out = args.ws + ((size_t)chunk * args.nprob + prob) * (size_t)M * N;
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) {
-        const int n = n0 + wn * (TN / WN) + j * 32 + li;
-        if (n >= N) continue;
-#pragma unroll
-        for (int i = 0; i < BI; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int m = m0 + wm * (TM / WM) + i * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
-            if (m < M) out[(size_t)m * N + n] = acc[i][j][r];
-          }
-      }
-      return;
-    }
-  }
-
-  if constexpr (ACT == kActRope) {
-    if (prob < 2) {
-      // uniform: the whole workgroup takes one form
-      const int pairs = args.rope_hd >> 1, seg = args.rope_seg;
-      const int mseg = seg > 0 ? m0 % seg : m0;
-      static_assert(sizeof(As) >= sizeof(float2) * 32 * (WM * 32 + 2), "RoPE table in LDS");
-      // (the 128 x 128 configuration keeps store_rope: with the LDS form its
-      // k-loop needs more than the 128 VGPRs of four waves per SIMD)
-      const bool lds = TM == 256 && m0 + TM <= M && (seg <= 0 || mseg + TM <= seg);
-      float2 *tab = reinterpret_cast<float2 *>(&As[0][0][0]);
-      const int mw = m0 + wm * (TM / WM), nw = n0 + wn * (TN / WN);
-      if (lds && pairs == 32)
-        store_rope_lds<TM, WM, NT, BI, BJ, 5>(args, P, acc, mseg, wm, mw, nw, li, hf, tab);
-      else if (lds && pairs == 16)
-        store_rope_lds<TM, WM, NT, BI, BJ, 4>(args, P, acc, mseg, wm, mw, nw, li, hf, tab);
-      else if (lds && pairs == 8)
-        store_rope_lds<TM, WM, NT, BI, BJ, 3>(args, P, acc, mseg, wm, mw, nw, li, hf, tab);
-      else if (lds && pairs == 4)
-        store_rope_lds<TM, WM, NT, BI, BJ, 2>(args, P, acc, mseg, wm, mw, nw, li, hf, tab);
-      else
-        store_rope<BI, BJ>(args, P, acc, m0 + wm * (TM / WM), n0 + wn * (TN / WN), li, hf);
-      return;
-    }
-  }
-  // Epilogue: D[i][j] of block (bi, bj) sits at row 8*(r/4) + 4*hf + r%4,
-  // column li; 32 lanes store 32 consecutive columns of one row.
-  if constexpr (!EPI) {
-    const int mw = m0 + wm * (TM / WM), nw = n0 + wn * (TN / WN);
-    if (!args.beta && mw + TM / WM <= M && nw + TN / WN <= N) {
-      // every row and column of this wave's blocks exists: no predicates, and
-      // per row only a wave-uniform offset from the lane's base
-      float bias[BJ];
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) bias[j] = P.bias ? P.bias[nw + j * 32 + li] : 0.f;
-      float *cb = P.c + (size_t)(mw + 4 * hf) * args.ldc + nw + li;
-#pragma unroll
-      for (int i = 0; i < BI; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float *c = cb + (size_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * args.ldc;
-#pragma unroll
-          for (int j = 0; j < BJ; ++j)
-            c[j * 32] = activate(acc[i][j][r] + bias[j], ACT == kActRope ? CDML_ACT_NONE : ACT);
-        }
-      return;
-    }
-  } else if constexpr (!TA) {
-    const int mw = m0 + wm * (TM / WM), nw = n0 + wn * (TN / WN);
-    if (!args.beta && mw + TM / WM <= M && nw + TN / WN <= N) {
-      // The training epilogue on a whole wave block: the dz and add operands
-      // of four rows are loaded before any of their stores (a load issued
-      // after a store waits for it), and every address is a lane base plus a
-      // wave-uniform row offset.
-      float bias[BJ];
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) bias[j] = P.bias ? P.bias[nw + j * 32 + li] : 0.f;
-      const size_t lane_c = (size_t)(mw + 4 * hf) * args.ldc + nw + li;
-      const size_t lane_pre = (size_t)(mw + 4 * hf) * args.ldpre + nw + li;
-      const size_t lane_dz = (size_t)(mw + 4 * hf) * args.lddz + nw + li;
-      const size_t lane_add = (size_t)(mw + 4 * hf) * args.ldadd + nw + li;
-#pragma unroll
-      for (int i = 0; i < BI; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float zv[4][BJ], av[4][BJ];
-          if (args.dz) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr)
-#pragma unroll
-              for (int j = 0; j < BJ; ++j)
-                zv[rr][j] = args.dz[lane_dz + (size_t)(i * 32 + 8 * g + rr) * args.lddz + j * 32];
-          }
-          if (args.add) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr)
-#pragma unroll
-              for (int j = 0; j < BJ; ++j)
-                av[rr][j] = args.add[lane_add + (size_t)(i * 32 + 8 * g + rr) * args.ldadd + j * 32];
-          }
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) {
-            const int r = 4 * g + rr, d = i * 32 + 8 * g + rr;
-#pragma unroll
-            for (int j = 0; j < BJ; ++j) {
-              const float z = acc[i][j][r] + bias[j];
-              if (args.pre) args.pre[lane_pre + (size_t)d * args.ldpre + j * 32] = z;
-              float v = activate(z, ACT == kActRope ? CDML_ACT_NONE : ACT);
-              if (args.dz) v *= act_deriv(zv[rr][j], args.dact);
-              if (args.add) v += av[rr][j];
-              P.c[lane_c + (size_t)d * args.ldc + j * 32] = v;
-            }
-          }
-        }
-      return;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < BJ; ++j) {
-    const int n = n0 + wn * (TN / WN) + j * 32 + li;
-    if (n >= N) continue;
-    const float bias = P.bias ? P.bias[n] : 0.f;
-#pragma unroll
-    for (int i = 0; i < BI; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * (TM / WM) + i * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
-        if (m < M) store_elem<EPI>(args, P, m, n, acc[i][j][r] + bias, ACT == kActRope ? CDML_ACT_NONE : ACT);
-      }
-    }
-  }
+  const TileOut out{P.c, args.ldc, P.bias, args.act, args.beta, false};
+  store_tile<BI, BJ, true, false>(args, out, acc, m0 + wm * (TM / WM), n0 + wn * (TN / WN), lane,
+                                  smem + wave * 32 * (32 * BJ + 4));
 }
 
 // Few rows (decode steps, short batches: M <= MR), non-transposed operands,
@@ -1316,11 +1509,6 @@ __global__ void __launch_bounds__(256) wgrad_small_reduce_kernel(const GemmArgs 
   }
 }
 
-// The 256 x 128 eight-wave tiles for M >= 1024, and for weight gradients
-// (both operands transposed, a long row reduction split over chunks) whose
-// M is a multiple of 256; 128 x 128 four-wave tiles otherwise.
-inline bool big_tiles(int M, bool wgrad) { return M >= 1024 || (wgrad && M % 256 == 0); }
-
 SplitPlan splitk_plan(int M, int N, int K, int nprob) {
   SplitPlan sp;
   const int nk = K / 16;  // whole k-tiles; the reduce or a tail launch adds a ragged tail
@@ -1340,10 +1528,8 @@ SplitPlan splitk_plan(int M, int N, int K, int nprob) {
     sp.bytes = (size_t)bound * nprob * ((size_t)M * N + M) * sizeof(float);
     return sp;
   }
-  const bool big = big_tiles(M, true);
-  const int TM = big ? 256 : 128, TN = 128;
-  const int tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN) * nprob;
-  const int slots = big ? 512 : 1024;
+  const int tiles = ((M + 127) / 128) * ((N + 127) / 128) * nprob;
+  const int slots = 512;  // two 128 x 128 workgroups per CU
   // at least eight k-tiles per chunk, or two for a small output (at most
   // 64 K elements, so a chunk's partial is at most 256 KB): a short
   // reduction into a few tiles is otherwise one workgroup's serial k-loop
@@ -1365,28 +1551,7 @@ SplitPlan splitk_plan(int M, int N, int K, int nprob) {
   return sp;
 }
 
-// The forward tile kernel for the launch's activation.
-template <int TM, int TN, int BKK, int WM, int WN, int MINB, bool EPI>
-void launch_tile_act(const GemmArgs &g, dim3 grid, dim3 block, hipStream_t stream) {
-  switch (g.act) {
-    case CDML_ACT_NONE: gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_NONE, false, false, EPI><<<grid, block, 0, stream>>>(g); break;
-    case CDML_ACT_SIGMOID: gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_SIGMOID, false, false, EPI><<<grid, block, 0, stream>>>(g); break;
-    case CDML_ACT_TANH: gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_TANH, false, false, EPI><<<grid, block, 0, stream>>>(g); break;
-    case CDML_ACT_RELU: gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_RELU, false, false, EPI><<<grid, block, 0, stream>>>(g); break;
-    case CDML_ACT_LEAKYRELU: gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_LEAKYRELU, false, false, EPI><<<grid, block, 0, stream>>>(g); break;
-    case kActReluMarked:
-      if constexpr (!EPI) {  // only launches without z use it
-        gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, kActReluMarked, false, false, false><<<grid, block, 0, stream>>>(g);
-        break;
-      }
-      [[fallthrough]];
-    default: gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_SWISH, false, false, EPI><<<grid, block, 0, stream>>>(g); break;
-  }
-}
-
-// Two tile configurations: 256 x 128 with eight waves for M >= 1024, and
-// 128 x 128 with four waves for smaller M (decode rows, short sequences).
-template <int TM, int TN, int BKK, int WM, int WN, int MINB, bool TA, bool TB>
+template <int TM, int TN, int WM, int WN, int MINB, int NB, bool TA, bool TB>
 int launch_tile(GemmArgs g, hipStream_t stream) {
   g.tiles_m = (g.M + TM - 1) / TM;
   g.tiles_n = (g.N + TN - 1) / TN;
@@ -1395,44 +1560,63 @@ int launch_tile(GemmArgs g, hipStream_t stream) {
   g.total = g.tiles * g.ksplit;
   g.padded = pad_to_xcd(g.total);
   const dim3 grid(g.padded), block(64 * WM * WN);
-  if constexpr (TA || TB) {
-    if (has_epi(g))
-      gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_NONE, TA, TB, true><<<grid, block, 0, stream>>>(g);
+  if (!TA && !TB && g.rope_cs)
+    gemm_tile_kernel<TM, TN, WM, WN, MINB, NB, !TA && !TB, TA, TB, false><<<grid, block, 0, stream>>>(g);
+  else if (!(TA && TB) && has_epi(g))
+    gemm_tile_kernel<TM, TN, WM, WN, MINB, NB, false, TA, TB, !(TA && TB)><<<grid, block, 0, stream>>>(g);
+  else
+    gemm_tile_kernel<TM, TN, WM, WN, MINB, NB, false, TA, TB, false><<<grid, block, 0, stream>>>(g);
+  if (TA && TB && g.ksplit > 1) {
+    const size_t outs = std::max((size_t)g.M * (g.N / 4), (size_t)g.M);
+    if (g.ksplit >= 32)
+      splitk_reduce_kernel<8><<<dim3((unsigned)((outs * 8 + 255) / 256), g.nprob), dim3(256), 0, stream>>>(g);
     else
-      gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, CDML_ACT_NONE, TA, TB, false><<<grid, block, 0, stream>>>(g);
-    if (g.ksplit > 1) {
-      const size_t outs = std::max((size_t)g.M * (g.N / 4), (size_t)g.M);
-      if (g.ksplit >= 32)
-        splitk_reduce_kernel<8><<<dim3((unsigned)((outs * 8 + 255) / 256), g.nprob), dim3(256), 0, stream>>>(g);
-      else
-        splitk_reduce_kernel<1><<<dim3((unsigned)((outs + 255) / 256), g.nprob), dim3(256), 0, stream>>>(g);
-    }
-  } else {
-    if (g.rope_cs) {
-      gemm_tile_kernel<TM, TN, BKK, WM, WN, MINB, kActRope, false, false, false><<<grid, block, 0, stream>>>(g);
-      return CDML_OK;
-    }
-    if (has_epi(g)) {
-      launch_tile_act<TM, TN, BKK, WM, WN, MINB, true>(g, grid, block, stream);
-    } else {
-      launch_tile_act<TM, TN, BKK, WM, WN, MINB, false>(g, grid, block, stream);
-    }
+      splitk_reduce_kernel<1><<<dim3((unsigned)((outs + 255) / 256), g.nprob), dim3(256), 0, stream>>>(g);
   }
   return CDML_OK;
 }
 
 // Whether a [rows, K] (T = false) or [K, rows] (T = true) operand with row
 // stride ld and base p suits the tiled kernel's staging.
-bool stage_ok(const float *p, int rows, int ld, bool T, int bkk) {
+bool stage_ok(const float *p, int rows, int K, int ld, bool T) {
   if (!aligned16(p) || ld % 4) return false;
-  if (T) return rows % 4 == 0 && (unsigned long long)bkk * ld + rows < (1ull << 32);
-  return (unsigned long long)rows * ld < (1ull << 32);
+  if (T) return rows % 4 == 0 && 16ull * (unsigned long long)ld + (unsigned long long)rows < (1ull << 32);
+  return K % 4 == 0 && (unsigned long long)rows * ld < (1ull << 32);
+}
+
+// 128 x 128 tiles (two workgroups per CU) where they give three quarters of
+// the CUs one, 64 x 64 otherwise, four times as many (fwd / dX, us): 4096 x 1024
+// x 1024, 256 tiles of 128 x 128: 56 / 64 against 67 / 69; 2048 x 1024 x 1024, 128
+// tiles: 50 / 62 against 49 / 54; 512 x 1024 x 1024: 44 / 54 against 36 / 44.
+// (256 x 128 with eight waves, one workgroup per CU, is 1-3% faster than 128 x
+// 128 forward and 2-8% slower in both gradients, whose short k-loops and long
+// epilogues another workgroup has to cover.)
+template <bool TA, bool TB>
+int launch_tiled(GemmArgs &g, hipStream_t stream) {
+  const long long tiles = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.nprob * std::max(g.ksplit, 1);
+  if (4 * tiles >= 3LL * num_cus()) return launch_tile<128, 128, 2, 2, 2, 3, TA, TB>(g, stream);
+  return launch_tile<64, 64, 2, 1, 3, 2, TA, TB>(g, stream);
+}
+
+// 256 x 128 tiles unless they would not fill one round of two workgroups per
+// CU: then 128 x 128 tiles spread the same work over twice as many workgroups
+// (16384 x 512 -> 512: 81 -> 78 us, same bits).
+template <int TM, int TN, int WM, int WN>
+void launch_f32_tile(GemmArgs &g, hipStream_t stream) {
+  g.tiles_m = (g.M + TM - 1) / TM;
+  g.tiles_n = (g.N + TN - 1) / TN;
+  g.total = g.tiles_m * g.tiles_n;
+  g.padded = pad_to_xcd(g.total);
+  gemm_f32_kernel<TM, TN, WM, WN><<<dim3(g.padded), dim3(64 * WM * WN), 0, stream>>>(g);
+}
+void launch_f32(GemmArgs &g, hipStream_t stream) {
+  const long long big = (long long)((g.M + 255) / 256) * ((g.N + 127) / 128);
+  if (g.M >= 1024 && big >= 2 * num_cus()) launch_f32_tile<256, 128, 4, 2>(g, stream);
+  else launch_f32_tile<128, 128, 2, 2>(g, stream);
 }
 
 template <bool TA, bool TB>
-int launch_layout(GemmArgs &g, bool fast, hipStream_t stream) {
-  if (fast) return big_tiles(g.M, TA && TB) ? launch_tile<256, 128, 16, 4, 2, 2, TA, TB>(g, stream)
-                                            : launch_tile<128, 128, 16, 2, 2, 2, TA, TB>(g, stream);
+int launch_any(GemmArgs &g, hipStream_t stream) {
   const dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, g.nprob);
   if (has_epi(g)) gemm_any_kernel<TA, TB, true><<<grid, dim3(256), 0, stream>>>(g);
   else gemm_any_kernel<TA, TB, false><<<grid, dim3(256), 0, stream>>>(g);
@@ -1447,26 +1631,17 @@ int launch_gemm(GemmArgs &g, bool ta, bool tb, hipStream_t stream, const char *w
   if (g.M == 0 || g.N == 0) return CDML_OK;
   if ((ta || tb) && (g.M > 65535 * 64 || g.N > 65535 * 64))
     return fail(CDML_E_INVALID, "%s: matrix too large", what);
-  bool fast = g.K % 16 == 0 && g.K > 0;
+  bool fast = g.K > 0;
   for (int i = 0; i < g.nprob; ++i)
-    fast = fast && stage_ok(g.p[i].a, g.M, g.lda, ta, 16) && stage_ok(g.p[i].w, g.N, g.ldb, tb, 16);
+    fast = fast && stage_ok(g.p[i].a, g.M, g.K, g.lda, ta) && stage_ok(g.p[i].w, g.N, g.K, g.ldb, tb);
   if (g.kseg) {  // only the tiled input-gradient kernel reads K segments
     bool ok = !ta && tb && !has_epi(g) && g.nprob == 1 && g.ksplit <= 1 && g.kseg * 16 * 3 == g.K;
     for (int i = 0; ok && i < 3; ++i)
-      ok = stage_ok(g.p[i].a, g.M, g.lda, false, 16) && stage_ok(g.p[i].w, g.N, g.ldb, true, 16);
+      ok = stage_ok(g.p[i].a, g.M, g.kseg * 16, g.lda, false) && stage_ok(g.p[i].w, g.N, g.kseg * 16, g.ldb, true);
     if (!ok) return fail(CDML_E_INVALID, "%s: K segments need the tiled input-gradient kernel", what);
     fast = true;
   }
   if (ta || tb) {
-    int rc;
-    // A ragged K: the tiled kernel covers the whole 16-row k-tiles (it never
-    // reads past them) and the last K % 16 rows are added by a second launch
-    // (C += tail, bgrad += tail row sums) -- unless an epilogue must see the
-    // complete sum.
-    const int ktail = g.K % 16;
-    bool split_tail = tb && ktail != 0 && g.K >= 16 && !g.dz && !g.add && !g.pre && g.act == CDML_ACT_NONE;
-    for (int i = 0; split_tail && i < g.nprob; ++i)
-      split_tail = stage_ok(g.p[i].a, g.M, g.lda, ta, 16) && stage_ok(g.p[i].w, g.N, g.ldb, tb, 16);
     if (!ta && tb && g.K <= 16 && g.K > 0 && g.M > 16 && g.N <= 1024) {  // few layer outputs
       const int rpp = 256 / ((g.N + 3) / 4);
       const dim3 grid((unsigned)std::min((g.M + rpp - 1) / rpp, 2048), (unsigned)g.nprob), block(256);
@@ -1485,27 +1660,16 @@ int launch_gemm(GemmArgs &g, bool ta, bool tb, hipStream_t stream, const char *w
       wgrad_small_reduce_kernel<<<dim3((n + 255) / 256, g.nprob), dim3(256), 0, stream>>>(g);
       return check_launch(what);
     }
-    if (ta && tb && split_tail && g.ksplit > 1 && !g.small && g.N % 4 == 0) {
-      // split-K: the reduce adds the last K % 16 rows, no tail launch
-      g.ktail0 = g.K - ktail;
-      split_tail = false;
-      rc = launch_layout<true, true>(g, true, stream);
-    } else if (ta && tb) rc = launch_layout<true, true>(g, fast || split_tail, stream);
-    else if (tb) rc = launch_layout<false, true>(g, fast || split_tail, stream);
-    else rc = launch_layout<true, false>(g, false, stream);
-    if (rc) return rc;
-    if (split_tail) {
-      const int kmain = g.K - ktail;
-      GemmArgs t = g;
-      t.K = ktail;
-      t.beta = 1;
-      t.ksplit = 1;
-      for (int i = 0; i < t.nprob; ++i) {
-        t.p[i].a += ta ? (size_t)kmain * g.lda : (size_t)kmain;
-        t.p[i].w += tb ? (size_t)kmain * g.ldb : (size_t)kmain;
-      }
-      rc = ta ? launch_layout<true, true>(t, false, stream) : launch_layout<false, true>(t, false, stream);
-      if (rc) return rc;
+    if (fast && ta && tb) {
+      if (g.ksplit > 1) g.ktail0 = g.K % 16 ? g.K - g.K % 16 : 0;  // the reduce adds the last K % 16 rows
+      launch_tiled<true, true>(g, stream);
+    } else if (fast && tb) {
+      launch_tiled<false, true>(g, stream);
+    } else {
+      g.ksplit = 1;
+      if (ta && tb) launch_any<true, true>(g, stream);
+      else if (tb) launch_any<false, true>(g, stream);
+      else launch_any<true, false>(g, stream);
     }
     return check_launch(what);
   }
@@ -1539,16 +1703,10 @@ int launch_gemm(GemmArgs &g, bool ta, bool tb, hipStream_t stream, const char *w
           : gemm_rows_kernel<16, false><<<grid, block, 0, stream>>>(g);
     return check_launch(what);
   }
-  // 256 x 128 tiles unless they would not fill one round of two workgroups
-  // per CU: then 128 x 128 tiles spread the same work over twice as many
-  // workgroups (16384 x 512 -> 512: 81 -> 78 us, same bits).
-  const long long big_tiles_fwd = (long long)((g.M + 255) / 256) * ((g.N + 127) / 128) * g.nprob;
-  if (fast && g.M >= 1024 && big_tiles_fwd >= 2 * num_cus()) {
-    int rc = launch_tile<256, 128, 16, 4, 2, 2, false, false>(g, stream);
-    if (rc) return rc;
-  } else if (fast) {
-    int rc = launch_tile<128, 128, 16, 2, 2, 2, false, false>(g, stream);
-    if (rc) return rc;
+  if (fast && g.f32 && g.K % 16 == 0) {
+    launch_f32(g, stream);
+  } else if (fast && !g.f32) {
+    launch_tiled<false, false>(g, stream);
   } else if (vec)
     has_epi(g) ? gemm_nt_kernel<true, true><<<dim3(g.padded), dim3(NTHREADS), 0, stream>>>(g)
                : gemm_nt_kernel<true, false><<<dim3(g.padded), dim3(NTHREADS), 0, stream>>>(g);
@@ -1832,6 +1990,7 @@ extern "C" int cdml_linear_preact(const float *x, int ldx, const float *w, const
   g.act = !z && activation == CDML_ACT_RELU ? kActReluMarked : activation;
   g.pre = z;
   g.ldpre = ldy;
+  g.f32 = activation == CDML_ACT_RELU || activation == CDML_ACT_LEAKYRELU;
   return launch_gemm(g, false, false, as_hip(stream), "cdml_linear_preact");
 }
 
@@ -1883,7 +2042,7 @@ extern "C" int cdml_backprop_qkv(const float *x, const float *dq, const float *d
     const float *w[3] = {wq, wk, wv};
     bool fused = out_dim > 0 && out_dim % 16 == 0 && (long long)3 * out_dim <= INT32_MAX;
     for (int s = 0; fused && s < 3; ++s)
-      fused = stage_ok(d[s], rows, out_dim, false, 16) && stage_ok(w[s], in_dim, in_dim, true, 16);
+      fused = stage_ok(d[s], rows, out_dim, out_dim, false) && stage_ok(w[s], in_dim, out_dim, in_dim, true);
     if (fused) {
       GemmArgs g{};
       g.lda = out_dim;
