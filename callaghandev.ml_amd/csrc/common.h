@@ -115,6 +115,16 @@ __device__ __forceinline__ void split_bf16x3(float a, float b, uint32_t &h, uint
   l = pack_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
 }
 
+// The three pieces of eight values as MFMA operands.
+__device__ __forceinline__ void split_operand(const float (&x)[8], bf16x8 (&p)[3]) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) split_bf16x3(x[2 * i], x[2 * i + 1], h[i], m[i], l[i]);
+  p[0] = __builtin_bit_cast(bf16x8, (vu4{h[0], h[1], h[2], h[3]}));
+  p[1] = __builtin_bit_cast(bf16x8, (vu4{m[0], m[1], m[2], m[3]}));
+  p[2] = __builtin_bit_cast(bf16x8, (vu4{l[0], l[1], l[2], l[3]}));
+}
+
 // bf16 MFMA 32x32x16: D = A(32x16) * B(16x32) + C.  Lane l holds eight
 // consecutive k, 8 * (l / 32) + 0..7, of row (A) or column (B) l % 32; D as
 // mfma32x32x2.

@@ -2,28 +2,36 @@
 // and MultiHeadAttentionForward of the reference, AccelerationCPU.cs:1647-1956).
 //
 // One 256-thread workgroup owns 128 queries of one (sequence, head); each of
-// its four waves owns 32 queries for the whole key loop.  Per key tile of BN
-// keys (K and V staged through double-buffered LDS, next tile prefetched into
-// registers while the current one is consumed):
+// its four waves owns 32 queries for the whole key loop.  All products run on
+// the bf16 matrix cores from three bf16 pieces per fp32 value (common.h): K and V
+// are split on their way into LDS, Q once into registers, the probabilities in
+// registers.  Per key tile of BN keys (double-buffered LDS, next tile prefetched
+// into registers while the current one is consumed):
 //
-//   S^T = K Q^T     v_mfma_f32_32x32x2_f32, A = K rows from LDS (16-byte
-//                   reads), B = the wave's Q held in registers for the whole
-//                   loop.  Computing S transposed puts one query per lane
-//                   (lane % 32) and 16 keys per lane in the accumulator, so the
-//                   softmax row reductions are in-lane plus one swap between
-//                   the two half-waves.
+//   S^T = K Q^T     A = K rows from LDS, B = the wave's Q pieces held in
+//                   registers for the whole loop.  Computing S transposed puts
+//                   one query per lane (lane % 32) and 16 keys per lane in the
+//                   accumulator, so the softmax row reductions are in-lane plus
+//                   one swap between the two half-waves.
 //   online softmax  running max / sum per query in the exp2 domain
 //                   (scale * log2 e folded into Q), masked keys -inf.
-//   O^T += V^T P^T  the probabilities stay in the S accumulator registers:
-//                   accumulator r of a lane holds key 8*(r/4) + 4*h + r%4,
-//                   exactly the key the B operand of MFMA step r needs, so
-//                   P is consumed in place; V is staged transposed in LDS,
-//                   so one 16-byte read feeds four MFMA steps.
+//   O^T += V^T P^T  accumulators 8 s .. 8 s + 7 of a lane hold the keys 16 s +
+//                   {4 h .. 4 h + 3, 8 + 4 h .. 8 + 4 h + 3} (h = lane / 32): V is
+//                   staged transposed with its keys in that order, so the
+//                   probabilities are consumed in place.
 //
 // Causal: tiles entirely above the diagonal are never loaded; a wave skips
 // MFMA work for its 32-key sub-blocks that lie wholly in its future; heavy
 // query tiles are dispatched first.  A row whose keys are all masked ends
 // with sum 0 and is written as 0 (AccelerationCPU.cs:1908-1911).
+//
+// What bounds it: at head dim 64 a 32 x 32 sub-block costs a wave 48 MFMAs
+// (1536 cycles of the matrix pipe) and about 250 VALU instructions (half of them
+// the two splits), at head dim 32 half the MFMAs and 210: the vector units there.
+// Measured on MI355X: the causal layer 4 x 4096, 16 heads of 64, of which this
+// kernel is half, 1750 -> 1560 us against the same kernel on the fp32 MFMA; the
+// matrix pipes are busy 61% of its cycles at head dim 64 and 45% at 32 (vector
+// units 55% and 73%).
 #include <cfloat>
 
 #include "common.h"
@@ -62,156 +70,118 @@ struct FlashArgs {
   float scale_log2;
   int n_qt, n_bh, n_items;  // query tiles per sequence, (sequence, head) pairs, n_bh * n_qt
   UDiv by_bh, by_heads;     // division by n_bh and by heads
-  int fast;                 // sub-blocks may skip their maximum (see try_fast)
 };
 
-// Stages one BN x HD tile of K or V (rows [k0, k0+BN) of head column block
-// `col0`) from global memory into registers and then into LDS.  Each
-// thread's element offsets inside a tile are fixed (set once); a tile load
-// adds them to the wave-uniform tile base.  Rows past lk (the sequence end)
-// are clamped to row lk - 1: their scores are masked to -inf and their
-// probabilities are exactly 0.
+// Stages one tile of BN keys: K rows [k0, k0 + BN) and V transposed, of head
+// column block `col0`, from global memory into registers and then, split into
+// three bf16 pieces, into LDS (one plane per piece, rows of 16 values = 32
+// bytes, as the GEMM's operand tiles).  The upper half of the workgroup's
+// waves stages K, the lower half V, eight values per unit pair and unit.
+//   K: slab s holds dims 16 s .. 16 s + 15 of every key: rows are keys, even
+//      and odd ones in two clusters.  A unit is four dims of one key.
+//   V: slab s holds keys 16 s .. 16 s + 15 of every dim: rows are dims, in four
+//      clusters by d % 4, odd dims negated (common.h; the output undoes it).  A
+//      unit is four dims of two keys; key k of a slab sits at place
+//      8 (k / 4 % 2) + 4 (k / 8) + k % 4, the order the P.V product reads.
+// Each thread's offsets inside a tile are fixed.  Rows past lk (the sequence
+// end) are clamped to row lk - 1: their scores are masked to -inf and their
+// probabilities are exactly 0.  Without VEC (head dims other than HD, unaligned
+// rows) columns at or past hd read as zero.
 template <int HD, int BN, bool VEC>
 struct KvStage {
-  static constexpr int F4_ROW = HD / 4;
-  static constexpr int ROWS_PER_PASS = FA_THREADS / F4_ROW;
-  static constexpr int NV = BN / ROWS_PER_PASS;
-  static constexpr int NS = BN * HD / FA_THREADS;
-  vf4 r[VEC ? NV : 1];  // a native vector, so the prefetch stays a register load issued at the loop top
-  float s[VEC ? 1 : NS];
-  uint32_t off[VEC ? NV : 1];  // byte offsets of this thread's rows in a tile
-  int col;
+  static constexpr int HALF = FA_THREADS / 2;
+  static constexpr int KROWB = BN / 2 * 32, VROWB = HD / 4 * 32;  // bytes of one row cluster
+  static constexpr int KSLAB = 2 * KROWB + 128, VSLAB = 4 * VROWB + 256;
+  static constexpr int KPLANE = HD / 16 * KSLAB, VPLANE = BN / 16 * VSLAB;
+  static constexpr int BYTES = 3 * (KPLANE + VPLANE);  // K planes, then V planes
+  static constexpr int VU = (HD / 4) * (BN / 2) / HALF;  // V units per thread; twice as many K units
+  static constexpr int NV = 2 * VU;                      // loads of either
+  static_assert(VU >= 1 && (HD / 4) * (BN / 2) % HALF == 0 && HALF / 8 % 16 == 0, "tile units");
+  static __device__ __forceinline__ constexpr int kcluster(int c) { return c * (KROWB + 16); }
+  static __device__ __forceinline__ constexpr int vcluster(int c) {
+    return c * VROWB + (c & 1) * 16 + (c >> 1) * 128;
+  }
+  // What a thread's further units add to its first: K unit i is KSTEP keys
+  // further down; V unit i is VG groups of four dims and whole slabs further.
+  static constexpr int CH = HD / 4, KSTEP = HALF / CH;
+  static __device__ __forceinline__ constexpr int vgroups(int i) { return HALF / 8 * i % CH; }
+  static __device__ __forceinline__ constexpr int vslabs(int i) { return HALF / 8 * i / CH; }
+  vf4 r[NV];
+  uint32_t off;  // byte offset of the first load in a tile
+  int col;       // its first column
+  int dst;       // LDS byte offset of the first unit
+  bool kside;
 
-  __device__ __forceinline__ void init(int ld) {
-    if constexpr (VEC) {
-      const int t = threadIdx.x;
-      col = (t % F4_ROW) * 4;
-#pragma unroll
-      for (int i = 0; i < NV; ++i) off[i] = 4u * (uint32_t)((t / F4_ROW + ROWS_PER_PASS * i) * ld + col);
-    }
+  __device__ __forceinline__ void init(int ldk, int ldv) {
+    kside = __builtin_amdgcn_readfirstlane(threadIdx.x) >= HALF;
+    const int t = threadIdx.x & (HALF - 1);
+    // K: the P keys of one load instruction share a cluster
+    constexpr int P = 64 / CH;
+    const int c = t % CH, j = t / CH, kkey = (j & ~(2 * P - 1)) | ((j & (P - 1)) << 1) | ((j / P) & 1);
+    const int sb = t & 7, g = (t >> 3) % CH, slab = (t >> 3) / CH;
+    const int place = ((sb >> 1) & 1) * 4 + (sb >> 2) * 2 + (sb & 1);  // of V's key pair
+    col = kside ? 4 * c : 4 * g;
+    off = 4u * (uint32_t)((kside ? kkey * ldk : (16 * slab + 2 * sb) * ldv) + col);
+    dst = kside ? (c >> 2) * KSLAB + kcluster(kkey & 1) + (kkey >> 1) * 32 + (c & 3) * 8
+                : 3 * KPLANE + slab * VSLAB + g * 32 + place * 4;
   }
 
-  __device__ __forceinline__ void load(const float *__restrict__ base, int ld, int k0, int lk,
-                                       int hd) {
-    if constexpr (VEC) {
-      // wave-uniform tile base plus a 32-bit per-lane byte offset (one
-      // scalar-base global load per row, no 64-bit address arithmetic)
-      const char *tile = reinterpret_cast<const char *>(base + (size_t)k0 * ld);
-      const uint32_t lim = 4u * ((uint32_t)(min(lk - 1 - k0, BN - 1) * ld) + col);
+  __device__ __forceinline__ void load(const float *__restrict__ kbase, const float *__restrict__ vbase, int ldk,
+                                       int ldv, int k0, int lk, int hd) {
+    // wave-uniform tile base plus a 32-bit per-lane byte offset (one
+    // scalar-base global load per row, no 64-bit address arithmetic)
+    const int ld = kside ? ldk : ldv;
+    const char *tile = reinterpret_cast<const char *>((kside ? kbase : vbase) + (size_t)k0 * ld);
+    const uint32_t last = 4u * (uint32_t)min(lk - 1 - k0, BN - 1) * (uint32_t)ld;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) r[i] = *reinterpret_cast<const vf4 *>(tile + min(off[i], lim));
-    } else {
-      const int t = threadIdx.x;
+    for (int i = 0; i < NV; ++i) {
+      const int dc = kside ? 0 : 4 * vgroups(i / 2);
+      const int rows = kside ? KSTEP * i : 16 * vslabs(i / 2) + (i & 1);
+      const char *p = tile + min(off + 4u * (uint32_t)(rows * ld + dc), last + 4u * (uint32_t)(col + dc));
+      if constexpr (VEC) {
+        r[i] = *reinterpret_cast<const vf4 *>(p);
+      } else {
 #pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        const int e = t + FA_THREADS * i;
-        const int row = e / HD, c = e % HD;
-        const int key = k0 + row;
-        s[i] = (key < lk && c < hd) ? base[(size_t)key * ld + c] : 0.f;
+        for (int c = 0; c < 4; ++c) r[i][c] = col + dc + c < hd ? reinterpret_cast<const float *>(p)[c] : 0.f;
       }
     }
   }
 
-  __device__ __forceinline__ void store(float (*lds)[HD + 4]) {
-    const int t = threadIdx.x;
-    if constexpr (VEC) {
+  __device__ __forceinline__ void store(char *lds) const {
+    if (kside) {
 #pragma unroll
-      for (int i = 0; i < NV; ++i)
-        *reinterpret_cast<vf4 *>(&lds[t / F4_ROW + ROWS_PER_PASS * i][col]) = r[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        const int e = t + FA_THREADS * i;
-        lds[e / HD][e % HD] = s[i];
-      }
-    }
-  }
-};
-
-// Stages one BN x HD tile of V transposed into LDS, Vt[d][key] with row pitch
-// BN + 4, so that the P.V step reads the four consecutive keys of one V^T
-// column it needs for four MFMA steps in a single 16-byte read.  A thread
-// takes two consecutive keys of a 4-wide column group (two 16-byte global
-// loads) and writes them as four 8-byte pairs Vt[c + j][2p .. 2p + 1].
-// Lanes 8m .. 8m + 7 of a wave take key pairs 0..7 (of an 8-pair block) of
-// column group m (of an 8-group block): the sixteen lanes of an 8-byte store
-// phase then cover two column groups, whose V^T rows (4 * pitch floats apart,
-// 16 banks apart) each receive eight contiguous pairs, so no two lanes share
-// a bank, and each 16-byte load instruction still reads 128 contiguous bytes
-// of each of 8 rows.  (With consecutive lanes on consecutive column groups
-// of one key pair, sixteen lanes' rows fell on two bank groups.)  Rows past
-// lk are clamped as in KvStage.
-template <int HD, int BN, bool VEC>
-struct VtStage {
-  static constexpr int NCG = HD / 4;               // 4-wide column groups
-  static constexpr int NKP = BN / 2;               // key pairs
-  static constexpr int NU = NKP * NCG / FA_THREADS;  // (key pair, column group) units per thread
-  static_assert(NKP % 8 == 0 && NCG % 8 == 0, "V tile blocks of 8 key pairs x 8 column groups");
-  // key pair and column group of unit u (64 units per 8 x 8 block)
-  __device__ __forceinline__ static int unit_kp(int u) { return (u & 7) + 8 * ((u >> 6) % (NKP / 8)); }
-  __device__ __forceinline__ static int unit_cg(int u) { return ((u >> 3) & 7) + 8 * ((u >> 6) / (NKP / 8)); }
-  static constexpr int NS = BN * HD / FA_THREADS;
-  static_assert(NKP * NCG % FA_THREADS == 0, "V tile units must divide the workgroup");
-  vf4 r[VEC ? 2 * NU : 1];
-  float s[VEC ? 1 : NS];
-  uint32_t off[VEC ? NU : 1];  // byte offset of each unit's first row in a tile
-  int col[VEC ? NU : 1];
-
-  __device__ __forceinline__ void init(int ld) {
-    if constexpr (VEC) {
-#pragma unroll
-      for (int i = 0; i < NU; ++i) {
-        const int u = threadIdx.x + FA_THREADS * i;
-        col[i] = unit_cg(u) * 4;
-        off[i] = 4u * (uint32_t)(2 * unit_kp(u) * ld + col[i]);
-      }
-    }
-  }
-
-  __device__ __forceinline__ void load(const float *__restrict__ base, int ld, int k0, int lk,
-                                       int hd) {
-    if constexpr (VEC) {
-      const char *tile = reinterpret_cast<const char *>(base + (size_t)k0 * ld);
-      const uint32_t last = (uint32_t)min(lk - 1 - k0, BN - 1) * (uint32_t)ld;
-      const uint32_t row = 4u * (uint32_t)ld;
-#pragma unroll
-      for (int i = 0; i < NU; ++i) {
-        const uint32_t lim = 4u * (last + col[i]);
-        r[2 * i] = *reinterpret_cast<const vf4 *>(tile + min(off[i], lim));
-        r[2 * i + 1] = *reinterpret_cast<const vf4 *>(tile + min(off[i] + row, lim));
+      for (int i = 0; i < NV; ++i) {
+        uint32_t h0, m0, l0, h1, m1, l1;
+        split_bf16x3(r[i][0], r[i][1], h0, m0, l0);
+        split_bf16x3(r[i][2], r[i][3], h1, m1, l1);
+        char *d = lds + dst + KSTEP / 2 * 32 * i;
+        *reinterpret_cast<vu2 *>(d) = vu2{h0, h1};
+        *reinterpret_cast<vu2 *>(d + KPLANE) = vu2{m0, m1};
+        *reinterpret_cast<vu2 *>(d + 2 * KPLANE) = vu2{l0, l1};
       }
     } else {
-      const int t = threadIdx.x;
 #pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        const int e = t + FA_THREADS * i;
-        const int rw = e / HD, c = e % HD;
-        const int key = k0 + rw;
-        s[i] = (key < lk && c < hd) ? base[(size_t)key * ld + c] : 0.f;
-      }
-    }
-  }
-
-  __device__ __forceinline__ void store(float (*lds)[BN + 4]) {
-    if constexpr (VEC) {
+      for (int i = 0; i < VU; ++i)
 #pragma unroll
-      for (int i = 0; i < NU; ++i) {
-        const int u = threadIdx.x + FA_THREADS * i;
-        const int kp = 2 * unit_kp(u);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          typedef float vf2 __attribute__((ext_vector_type(2)));
-          *reinterpret_cast<vf2 *>(&lds[col[i] + j][kp]) = vf2{r[2 * i][j], r[2 * i + 1][j]};
+        for (int c = 0; c < 4; ++c) {
+          uint32_t h, m, l;
+          const float x = r[2 * i][c], y = r[2 * i + 1][c];
+          split_bf16x3(c & 1 ? -x : x, c & 1 ? -y : y, h, m, l);
+          char *d = lds + dst + vslabs(i) * VSLAB + vgroups(i) * 32 + vcluster(c);
+          *reinterpret_cast<uint32_t *>(d) = h;
+          *reinterpret_cast<uint32_t *>(d + VPLANE) = m;
+          *reinterpret_cast<uint32_t *>(d + 2 * VPLANE) = l;
         }
-      }
-    } else {
-      const int t = threadIdx.x;
-#pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        const int e = t + FA_THREADS * i;
-        lds[e % HD][e / HD] = s[i];
-      }
     }
+  }
+
+  // Byte offsets of a lane's operands in a plane: dims 16 s + 8 hf + 0..7 of key
+  // row0 + li (row0 a multiple of 32), and eight keys of slab s for dim 32 db + li.
+  static __device__ __forceinline__ int koperand(int li, int hf) {
+    return kcluster(li & 1) + (li >> 1) * 32 + hf * 16;
+  }
+  static __device__ __forceinline__ int voperand(int li, int hf) {
+    return 3 * KPLANE + vcluster(li & 3) + (li >> 2) * 32 + hf * 16;
   }
 };
 
@@ -249,76 +219,38 @@ __device__ __forceinline__ constexpr int acc_key(int r) { return 8 * (r >> 2) + 
 // nothing overflows (the running sums stay below 2^32 times the key count).
 constexpr float kFastSumLimit = 4294967296.0f;  // 2^32
 
-// Which query tiles a workgroup runs, one after the other.  Item i of a
-// launch is (sequence, head) i % n_bh and, under the causal rule, query tile
-// n_qt - 1 - i / n_bh (heaviest rows first), else tile i / n_bh.
-//  * kOne: workgroup i runs item i.  With workgroup i on XCD i % 8, all tiles
-//    of one (sequence, head) share an XCD and its L2 whenever n_bh is a
-//    multiple of 8, and every XCD receives the heaviest tiles first (a
-//    near-optimal greedy schedule for a launch of several rounds).
-//  * kPair (causal launches that fit in one round): workgroup i runs tiles
-//    n_qt - 1 - p and p of its (sequence, head), p = i / n_bh, so every
-//    workgroup has the same work (n_qt + 1 key tiles; the middle tile of an
-//    odd count runs alone) and the round finishes together.
-// The last key tile of a workgroup's first item prefetches the first key tile
-// and the Q rows of the second.
-enum { kOne = 0, kPair = 1 };
-
-struct Item {
-  int bh, qt;
-};
-
-template <bool CAUSAL, int SCHED>
-__device__ __forceinline__ bool item_at(const FlashArgs &a, int k, Item &it) {
-  const int i = blockIdx.x;
-  if (SCHED == kPair) {
-    const int slot = a.by_bh.div(i);
-    it.bh = i - slot * a.n_bh;
-    if (k == 0) it.qt = a.n_qt - 1 - slot;
-    else if (k == 1 && 2 * slot + 1 != a.n_qt) it.qt = slot;
-    else return false;
-    return true;
-  } else if (k > 0) {
-    return false;
-  }
-  const int slot = a.by_bh.div(i);
-  it.bh = i - slot * a.n_bh;
-  it.qt = CAUSAL ? a.n_qt - 1 - slot : slot;
-  return true;
-}
-
-// Q^T operand of a wave: register 4u + r holds q[qi][8u + 4*hf + r], not yet
-// scaled.  Rows past lq read row lq - 1: they are computed but never stored.
+// Q^T operand of a wave: the three bf16 pieces of q[qi][16 s + 8 hf + 0..7] times
+// scale_log2.  Rows past lq read row lq - 1: they are computed but never stored.
 template <int HD, bool VEC>
-__device__ __forceinline__ void load_q(float (&qreg)[HD / 2], const FlashArgs &a, int b, int col0, int qi,
-                                       int hf) {
+__device__ __forceinline__ void load_q(bf16x8 (&q)[HD / 16][3], const FlashArgs &a, int b, int col0, int qi, int hf) {
   const float *qrow = a.q + ((size_t)b * a.lq + min(qi, a.lq - 1)) * a.ldq + col0;
 #pragma unroll
-  for (int u = 0; u < HD / 8; ++u) {
-    const int d = 8 * u + 4 * hf;
-    if constexpr (VEC) {
-      const vf4 t4 = *reinterpret_cast<const vf4 *>(qrow + d);
+  for (int s = 0; s < HD / 16; ++s) {
+    float x[8];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) qreg[4 * u + r] = t4[r];
-    } else {
+    for (int g = 0; g < 2; ++g) {
+      const int d = 16 * s + 8 * hf + 4 * g;
+      if constexpr (VEC) {
+        const vf4 t4 = *reinterpret_cast<const vf4 *>(qrow + d);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) qreg[4 * u + r] = d + r < a.hd ? qrow[d + r] : 0.f;
+        for (int r = 0; r < 4; ++r) x[4 * g + r] = t4[r] * a.scale_log2;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[4 * g + r] = d + r < a.hd ? qrow[d + r] * a.scale_log2 : 0.f;
+      }
     }
+    split_operand(x, q[s]);
   }
 }
 
 // The online softmax of one wave's 32 query rows (one per lane % 32) over
 // 32-key sub-blocks.
-template <int HD, bool HAS_MASK>
+template <int HD, int BN, bool HAS_MASK, bool VEC>
 struct OnlineRows {
+  typedef KvStage<HD, BN, VEC> Tile;
   static constexpr int NDB = HD / 32;     // 32-wide head-dim blocks of O^T
-  static constexpr int NQ = HD / 2;       // MFMA k-steps of Q.K
-  static constexpr int NKG = HD / 8;      // float4 groups of a K row slice
-  // P.V steps whose V operands are read at once (8: at head dim 32 every
-  // variant but the masked ones keeps four waves per SIMD)
-  static constexpr int VCH = 8;
-  static constexpr int NVG = VCH / 4;            // 16-byte V^T reads per chunk and head-dim block
-  floatx16 oacc[NDB];
+  static constexpr int NS = HD / 16;      // MFMA k-steps of Q.K
+  floatx16 oacc[NDB], ocor[NDB];          // hh, and its corrections (common.h)
   // The reference max of this lane's query (exp2 domain) is subtracted by
   // the MFMA itself: the first step of every S^T block starts from negm,
   // -m_run in all 16 entries (0 until the first visible key sets m_run), so
@@ -332,7 +264,7 @@ struct OnlineRows {
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
+      for (int r = 0; r < 16; ++r) oacc[db][r] = ocor[db][r] = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) negm[r] = 0.f;
     m_run = -INFINITY;
@@ -358,26 +290,28 @@ struct OnlineRows {
     }
   }
 
-  // O^T += V^T P^T: accumulator r of the lane holds the probability of key
-  // acc_key(r) + 4*hf, the key B-operand slot of MFMA step r needs.  vr holds
-  // the first chunk's V^T operands.
-  template <int VP>
-  __device__ __forceinline__ void accumulate_pv(const floatx16 &p, vf4 (&vr)[NVG][NDB], const float (*vt)[VP],
-                                                int key0, int li, int hf) {
+  // O^T += V^T P^T for the sub-block whose first V slab is at vt (this lane's
+  // operand of plane 0, dim block 0).
+  __device__ __forceinline__ void accumulate_pv(const floatx16 &p, const char *vt) {
 #pragma unroll
-    for (int ch = 0; ch < 16 / VCH; ++ch) {
-      if (ch > 0) {
+    for (int s = 0; s < 2; ++s) {
+      float x[8];
 #pragma unroll
-        for (int g = 0; g < NVG; ++g)
+      for (int e = 0; e < 8; ++e) x[e] = p[8 * s + e];
+      bf16x8 pp[3];
+      split_operand(x, pp);
 #pragma unroll
-          for (int db = 0; db < NDB; ++db)
-            vr[g][db] = *reinterpret_cast<const vf4 *>(&vt[db * 32 + li][key0 + 8 * (ch * NVG + g) + 4 * hf]);
+      for (int db = 0; db < NDB; ++db) {
+        bf16x8 v[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          v[q] = *reinterpret_cast<const bf16x8 *>(vt + q * Tile::VPLANE + s * Tile::VSLAB + db * 256);
+#pragma unroll
+        for (int q = 0; q < kSplitProducts; ++q) {
+          floatx16 &c = q == kSplitMain ? oacc[db] : ocor[db];
+          c = mfma32x32x16(v[kSplitA[q]], pp[kSplitB[q]], c);
+        }
       }
-#pragma unroll
-      for (int st = 0; st < VCH; ++st)
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-          oacc[db] = mfma32x32x2(vr[st / 4][db][st % 4], p[ch * VCH + st], oacc[db]);
     }
   }
 
@@ -386,16 +320,8 @@ struct OnlineRows {
   // score far above the reference) or NaN does the caller take the full path
   // (consume) on recomputed scores.  sacc is turned into probabilities in
   // place; on false the running state is unchanged and sacc is garbage.
-  template <int VP>
-  __device__ __forceinline__ bool try_fast(floatx16 &sacc, const float (*vt)[VP], int key0, int li, int hf,
-                                           bool masked, int last_vis, const uint8_t *mrow, int kb0, int key_cap,
-                                           bool row_ok) {
-    vf4 vr[NVG][NDB];
-#pragma unroll
-    for (int g = 0; g < NVG; ++g)
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-        vr[g][db] = *reinterpret_cast<const vf4 *>(&vt[db * 32 + li][key0 + 8 * g + 4 * hf]);
+  __device__ __forceinline__ bool try_fast(floatx16 &sacc, const char *vt, int hf, bool masked, int last_vis,
+                                           const uint8_t *mrow, int kb0, int key_cap, bool row_ok) {
     if (HAS_MASK || masked) apply_mask(sacc, hf, last_vis, mrow, kb0, key_cap, row_ok);
 #pragma unroll
     for (int r = 0; r < 16; ++r) sacc[r] = fast_exp2(sacc[r]);
@@ -406,47 +332,40 @@ struct OnlineRows {
     const float ps = ((s8[0] + s8[1]) + (s8[2] + s8[3])) + ((s8[4] + s8[5]) + (s8[6] + s8[7]));
     if (__builtin_amdgcn_ballot_w64(!(ps <= kFastSumLimit))) return false;
     l_a += ps;
-    accumulate_pv(sacc, vr, vt, key0, li, hf);
+    accumulate_pv(sacc, vt);
     return true;
   }
 
-  // S^T = K Q^T for the 32 keys whose rows start at krow; the K operand group
-  // u + 1 is read while group u multiplies.
-  template <int KP>
-  __device__ __forceinline__ floatx16 scores(const float (*krow)[KP], const float (&qreg)[NQ], int li,
-                                             int hf) const {
-    floatx16 sacc;
-    float4 kcur = *reinterpret_cast<const float4 *>(&krow[li][4 * hf]);
+  // S^T = K Q^T for the 32 keys whose operands start at kt (this lane's operand
+  // of plane 0, slab 0), relative to the reference.
+  __device__ __forceinline__ floatx16 scores(const char *kt, const bf16x8 (&q)[NS][3]) const {
+    floatx16 sacc = negm, cor = {};
 #pragma unroll
-    for (int u = 0; u < NKG; ++u) {
-      float4 knext;
-      if (u + 1 < NKG) knext = *reinterpret_cast<const float4 *>(&krow[li][8 * (u + 1) + 4 * hf]);
-      sacc = mfma32x32x2(kcur.x, qreg[4 * u + 0], u == 0 ? negm : sacc);
-      sacc = mfma32x32x2(kcur.y, qreg[4 * u + 1], sacc);
-      sacc = mfma32x32x2(kcur.z, qreg[4 * u + 2], sacc);
-      sacc = mfma32x32x2(kcur.w, qreg[4 * u + 3], sacc);
-      if (u + 1 < NKG) kcur = knext;
+    for (int s = 0; s < NS; ++s) {
+      bf16x8 k[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) k[p] = *reinterpret_cast<const bf16x8 *>(kt + p * Tile::KPLANE + s * Tile::KSLAB);
+#pragma unroll
+      for (int i = 0; i < kSplitProducts; ++i) {
+        floatx16 &c = i == kSplitMain ? sacc : cor;
+        c = mfma32x32x16(k[kSplitA[i]], q[s][kSplitB[i]], c);
+      }
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sacc[r] += cor[r];
     return sacc;
   }
 
-  // Softmax of one sub-block's scores and O^T += V^T P^T.  vt: V^T rows
-  // (pitch VP) whose columns key0 .. key0 + 31 are this sub-block's keys.
-  // masked (wave-uniform): some key of the sub-block may be invisible (see
-  // apply_mask).
-  template <int VP>
-  __device__ __forceinline__ void consume(floatx16 sacc, const float (*vt)[VP], int key0, int li, int hf,
-                                          bool masked, int last_vis, const uint8_t *mrow, int kb0,
-                                          int key_cap, bool row_ok) {
-    // V^T operands of the first P.V chunk, in flight during the softmax: steps
-    // 4g .. 4g + 3 take keys 8g + 4h .. 8g + 4h + 3 of column db * 32 + li.
-    vf4 vr[NVG][NDB];
-#pragma unroll
-    for (int g = 0; g < NVG; ++g)
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-        vr[g][db] = *reinterpret_cast<const vf4 *>(&vt[db * 32 + li][key0 + 8 * g + 4 * hf]);
+  // Softmax of one sub-block's scores and O^T += V^T P^T.  masked
+  // (wave-uniform): some key of the sub-block may be invisible (see apply_mask).
+  __device__ __forceinline__ void consume(floatx16 sacc, const char *vt, int hf, bool masked, int last_vis,
+                                          const uint8_t *mrow, int kb0, int key_cap, bool row_ok) {
+    softmax(sacc, hf, masked, last_vis, mrow, kb0, key_cap, row_ok);
+    accumulate_pv(sacc, vt);
+  }
 
+  __device__ __forceinline__ void softmax(floatx16 &sacc, int hf, bool masked, int last_vis, const uint8_t *mrow,
+                                          int kb0, int key_cap, bool row_ok) {
     if (HAS_MASK || masked) apply_mask(sacc, hf, last_vis, mrow, kb0, key_cap, row_ok);
     // tile max relative to the reference (-inf: no visible key)
     // (a tree of depth 3: eight v_max3 whose inputs do not wait on each other)
@@ -479,7 +398,10 @@ struct OnlineRows {
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+          for (int r = 0; r < 16; ++r) {
+            oacc[db][r] *= alpha;
+            ocor[db][r] *= alpha;
+          }
       }
     }
 #pragma unroll
@@ -490,14 +412,56 @@ struct OnlineRows {
       else l_a += p;
     }
     warm = !__builtin_amdgcn_ballot_w64(m_run == -INFINITY);
-    accumulate_pv(sacc, vr, vt, key0, li, hf);
+  }
+
+  // Joins the two accumulators and undoes the sign of the odd dims; whether
+  // some row came out non-finite (wave-uniform).
+  __device__ __forceinline__ bool finish() {
+    float bad = (l_a + l_b) * 0.f;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float o = oacc[db][r] + ocor[db][r];
+        oacc[db][r] = r & 1 ? -o : o;
+      }
+      bad = nonfinite_sum(oacc[db], bad);
+    }
+    return any_nonfinite(bad);
+  }
+
+  // The wave's rows on the fp32 MFMA straight from memory: only for rows that
+  // came out non-finite (an infinity or NaN in Q, K or V, or a product that
+  // overflows), so that they hold what the fp32 products give.
+  __device__ __forceinline__ void recompute(const FlashArgs &a, int b, int col0, int qi, int li, int hf, int kend,
+                                            int key_last, const uint8_t *mrow) {
+    init();
+    const float *qrow = a.q + ((size_t)b * a.lq + min(qi, a.lq - 1)) * a.ldq + col0;
+    const float *kb = a.k + (size_t)b * a.lk * a.ldk + col0, *vb = a.v + (size_t)b * a.lk * a.ldv + col0;
+#pragma unroll 1
+    for (int kb0 = 0; kb0 < kend; kb0 += 32) {
+      const float *krow = kb + (size_t)min(kb0 + li, a.lk - 1) * a.ldk;
+      floatx16 sacc = negm;
+#pragma unroll 1
+      for (int d = 0; d < HD; d += 2) {
+        const bool in = d + hf < a.hd;
+        sacc = mfma32x32x2(in ? krow[d + hf] : 0.f, in ? qrow[d + hf] * a.scale_log2 : 0.f, sacc);
+      }
+      softmax(sacc, hf, true, key_last - kb0 - 4 * hf, mrow, kb0, a.lk - 1, qi < a.lq);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float *vrow = vb + (size_t)min(kb0 + acc_key(r) + 4 * hf, a.lk - 1) * a.ldv;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+          oacc[db] = mfma32x32x2(db * 32 + li < a.hd ? vrow[db * 32 + li] : 0.f, sacc[r], oacc[db]);
+      }
+    }
   }
 
   // Normalise and store row qi of (sequence b, head bh): the lane holds dims
   // db*32 + 8*(r/4) + 4*hf + r%4.  For the backward pass the row statistic
   // lse = m + log2(l) recovers every probability as exp2(s * scale * log2 e
   // - lse) (+inf for a row with no visible key, whose p are all 0).
-  template <bool VEC>
   __device__ __forceinline__ void store(const FlashArgs &a, int bh, int b, int qi, int col0, int hf) const {
     const float l_tot = halves_sum(l_a + l_b);
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
@@ -525,130 +489,88 @@ struct OnlineRows {
   }
 };
 
-template <int HD, int BN, bool CAUSAL, bool HAS_MASK, bool VEC, int SCHED>
-__global__ void __launch_bounds__(FA_THREADS, 2) flash_fwd_kernel(const FlashArgs a) {
+// Workgroup i runs (sequence, head) i % n_bh and, under the causal rule, query
+// tile n_qt - 1 - i / n_bh (heaviest rows first), else tile i / n_bh.  With
+// workgroup i on XCD i % 8, all tiles of one (sequence, head) share an XCD and
+// its L2 whenever n_bh is a multiple of 8, and every XCD receives the heaviest
+// tiles first (a near-optimal greedy schedule for a launch of several rounds).
+template <int HD, int BN, bool CAUSAL, bool HAS_MASK, bool VEC>
+__global__ void __launch_bounds__(FA_THREADS, HD <= 32 ? 3 : (HD <= 64 ? 2 : 1)) flash_fwd_kernel(const FlashArgs a) {
   constexpr int NKB = BN / 32;   // 32-key sub-blocks per tile
-  constexpr int NQ = HD / 2;     // MFMA k-steps of Q.K
-  __shared__ __attribute__((aligned(16))) float Ks[2][BN][HD + 4];
-  __shared__ __attribute__((aligned(16))) float Vt[2][HD][BN + 4];  // V transposed
+  typedef KvStage<HD, BN, VEC> Stage;
+  __shared__ __attribute__((aligned(16))) char lds[2][Stage::BYTES];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 31, hf = lane >> 5;
+  const int slot = a.by_bh.div(blockIdx.x), bh = blockIdx.x - slot * a.n_bh;
+  const int qt = CAUSAL ? a.n_qt - 1 - slot : slot;
+  const int b = a.by_heads.div(bh), col0 = (bh - b * a.heads) * a.hd;
+  const int q0 = qt * FA_BM;
+  const int qw0 = q0 + wave * 32;   // first query of this wave (wave-uniform)
+  const int qi = qw0 + li;          // this lane's query
+  const float *__restrict__ kbase = a.k + (size_t)b * a.lk * a.ldk + col0;
+  const float *__restrict__ vbase = a.v + (size_t)b * a.lk * a.ldv + col0;
 
-  KvStage<HD, BN, VEC> sk;
-  VtStage<HD, BN, VEC> sv;
-  sk.init(a.ldk);
-  sv.init(a.ldv);
-
-  // The first item: its Q rows and first key tile.
-  Item it;
-  item_at<CAUSAL, SCHED>(a, 0, it);
-  float qreg[NQ];
-  {
-    const int b = a.by_heads.div(it.bh), col0 = (it.bh - b * a.heads) * a.hd;
-    load_q<HD, VEC>(qreg, a, b, col0, it.qt * FA_BM + wave * 32 + li, hf);
-    sk.load(a.k + (size_t)b * a.lk * a.ldk + col0, a.ldk, 0, a.lk, a.hd);
-    sv.load(a.v + (size_t)b * a.lk * a.ldv + col0, a.ldv, 0, a.lk, a.hd);
-  }
-  sk.store(Ks[0]);
-  sv.store(Vt[0]);
+  Stage st;
+  st.init(a.ldk, a.ldv);
+  st.load(kbase, vbase, a.ldk, a.ldv, 0, a.lk, a.hd);
+  bf16x8 q[HD / 16][3];
+  load_q<HD, VEC>(q, a, b, col0, qi, hf);
+  st.store(lds[0]);
   __syncthreads();
-  int buf = 0;  // LDS buffer holding the current key tile
 
-  for (int k = 0;; ++k) {
-    const int b = a.by_heads.div(it.bh), h = it.bh - b * a.heads;
-    const int q0 = it.qt * FA_BM;
-    const int qw0 = q0 + wave * 32;   // first query of this wave (wave-uniform)
-    const int qi = qw0 + li;          // this lane's query
-    const int col0 = h * a.hd;
-    const float *__restrict__ kbase = a.k + (size_t)b * a.lk * a.ldk + col0;
-    const float *__restrict__ vbase = a.v + (size_t)b * a.lk * a.ldv + col0;
+  const int kend = CAUSAL ? min(q0 + FA_BM, a.lk) : a.lk;
+  const int n_kt = (kend + BN - 1) / BN;
+  OnlineRows<HD, BN, HAS_MASK, VEC> rows;
+  rows.init();
+  // Last key this lane may attend (the causal diagonal and the sequence end).
+  const int key_last = CAUSAL ? min(qi, a.lk - 1) : a.lk - 1;
+  const uint8_t *mrow = HAS_MASK ? a.mask + (size_t)min(qi, a.lq - 1) * a.lk : nullptr;
+  const int ko = Stage::koperand(li, hf), vo = Stage::voperand(li, hf);
 
-    // Q in the exp2 domain: the scores leave the MFMA as s * scale * log2(e)
+  for (int kt = 0; kt < n_kt; ++kt) {
+    const int cur = kt & 1;
+    const int k0 = kt * BN;
+    // Next tile into registers; the last iteration re-stages its own tile into
+    // the idle buffer (nobody reads it again): an unconditional stage keeps the
+    // staging registers out of scratch memory.
+    st.load(kbase, vbase, a.ldk, a.ldv, kt + 1 < n_kt ? k0 + BN : k0, a.lk, a.hd);
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) qreg[i] *= a.scale_log2;
-
-    Item nx = it;
-    const bool has_next = item_at<CAUSAL, SCHED>(a, k + 1, nx);
-    const int nb = a.by_heads.div(nx.bh), ncol0 = (nx.bh - nb * a.heads) * a.hd;  // used only with has_next
-
-    const int kend = CAUSAL ? min(q0 + FA_BM, a.lk) : a.lk;
-    const int n_kt = (kend + BN - 1) / BN;
-
-    OnlineRows<HD, HAS_MASK> rows;
-    rows.init();
-    // Last key this lane may attend (the causal diagonal and the sequence end).
-    const int key_last = CAUSAL ? min(qi, a.lk - 1) : a.lk - 1;
-    const uint8_t *mrow = HAS_MASK ? a.mask + (size_t)min(qi, a.lq - 1) * a.lk : nullptr;
-
-    for (int kt = 0; kt < n_kt; ++kt) {
-      const int cur = buf;
-      const int k0 = kt * BN;
-      const bool last = kt + 1 == n_kt;
-      // Next tile into registers: this item's next tile, else the next
-      // item's first tile.  Without a next item the last iteration re-stages
-      // its own tile into the idle buffer (nobody reads it again): an
-      // unconditional stage keeps the staging registers out of scratch memory.
-      {
-        const bool to_next = last && has_next;
-        const int ks = !last ? k0 + BN : (has_next ? 0 : k0);
-        sk.load(to_next ? a.k + (size_t)nb * a.lk * a.ldk + ncol0 : kbase, a.ldk, ks, a.lk, a.hd);
-        sv.load(to_next ? a.v + (size_t)nb * a.lk * a.ldv + ncol0 : vbase, a.ldv, ks, a.lk, a.hd);
-      }
-      bool q_next = false;  // the next item's Q rows are loading
-
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        const int kb0 = k0 + kb * 32;
-        // A sub-block wholly past the sequence end or in this wave's future
-        // contributes nothing (every probability would be 0), and a wave
-        // whose rows all lie past lq (the last tile of a ragged length) has
-        // nothing to compute: skip.
-        if (kb0 >= a.lk || qw0 >= a.lq || (CAUSAL && kb0 > qw0 + 31)) continue;
-        floatx16 sacc = rows.scores(&Ks[cur][kb * 32], qreg, li, hf);
-        // Q is last read by the final sub-block of the last tile: the next
-        // item's Q rows load while this sub-block's softmax and P.V run.
-        if (kb == NKB - 1 && last && has_next) {
-          load_q<HD, VEC>(qreg, a, nb, ncol0, nx.qt * FA_BM + wave * 32 + li, hf);
-          q_next = true;
+    for (int kb = 0; kb < NKB; ++kb) {
+      const int kb0 = k0 + kb * 32;
+      // A sub-block wholly past the sequence end or in this wave's future
+      // contributes nothing (every probability would be 0), and a wave
+      // whose rows all lie past lq (the last tile of a ragged length) has
+      // nothing to compute: skip.
+      if (kb0 >= a.lk || qw0 >= a.lq || (CAUSAL && kb0 > qw0 + 31)) continue;
+      const char *kop = lds[cur] + ko + kb * 512, *vop = lds[cur] + vo + 2 * kb * Stage::VSLAB;
+      floatx16 sacc = rows.scores(kop, q);
+      // masking is needed on the diagonal and at the sequence end (wave-uniform)
+      const bool masked = kb0 + 31 > (CAUSAL ? min(qw0, a.lk - 1) : a.lk - 1);
+      const int last_vis = key_last - kb0 - 4 * hf;
+      // Once every row has its reference, a sub-block is accumulated without
+      // its maximum unless its probabilities come out unbounded; then its
+      // scores are recomputed (K is still in LDS) for the full path.  Explicit
+      // masks keep the full path.
+      bool done = false;
+      if (!HAS_MASK && rows.warm) {
+        done = rows.try_fast(sacc, vop, hf, masked, last_vis, mrow, kb0, a.lk - 1, qi < a.lq);
+        if (!done) {
+          // K is read from LDS again (the compiler may not keep the first
+          // scores, which would hold them live through the fast path)
+          asm volatile("" ::: "memory");
+          sacc = rows.scores(kop, q);
         }
-        // masking is needed on the diagonal and at the sequence end (wave-uniform)
-        const bool masked = kb0 + 31 > (CAUSAL ? min(qw0, a.lk - 1) : a.lk - 1);
-        const int last_vis = key_last - kb0 - 4 * hf;
-        // Once every row has its reference, a sub-block is accumulated without
-        // its maximum unless its probabilities come out unbounded; then its
-        // scores are recomputed (K is still in LDS and Q in registers: a kOne
-        // workgroup loads no further Q rows) for the full path.  Explicit
-        // masks keep the full path (the mask reads in both paths would cost
-        // the registers of a fourth wave per SIMD), and so do launches of
-        // fewer than three workgroups per CU, whose waves cannot hide the wait
-        // of the check before the P.V step (every paired launch is one).
-        bool done = false;
-        if (!HAS_MASK && SCHED == kOne && a.fast && rows.warm) {
-          done = rows.try_fast(sacc, Vt[cur], kb * 32, li, hf, masked, last_vis, mrow, kb0, a.lk - 1, qi < a.lq);
-          if (!done) {
-            // K is read from LDS again (the compiler may not keep the first
-            // scores, which would hold them live through the fast path)
-            asm volatile("" ::: "memory");
-            sacc = rows.scores(&Ks[cur][kb * 32], qreg, li, hf);
-          }
-        }
-        if (!done)
-          rows.consume(sacc, Vt[cur], kb * 32, li, hf, masked, last_vis, mrow, kb0, a.lk - 1, qi < a.lq);
       }
-      // a wave that skipped the final sub-block loads the next Q rows here
-      if (last && has_next && !q_next) load_q<HD, VEC>(qreg, a, nb, ncol0, nx.qt * FA_BM + wave * 32 + li, hf);
-
-      sk.store(Ks[cur ^ 1]);
-      sv.store(Vt[cur ^ 1]);
-      __syncthreads();
-      buf = cur ^ 1;
+      if (!done) rows.consume(sacc, vop, hf, masked, last_vis, mrow, kb0, a.lk - 1, qi < a.lq);
     }
-    rows.template store<VEC>(a, it.bh, b, qi, col0, hf);
-    if (!has_next) break;
-    it = nx;
+    st.store(lds[cur ^ 1]);
+    __syncthreads();
   }
+  if (rows.finish() && qw0 < a.lq)
+    rows.recompute(a, b, col0, qi, li, hf, CAUSAL ? min(qw0 + 32, a.lk) : a.lk, key_last, mrow);
+  rows.store(a, bh, b, qi, col0, hf);
 }
 
 // Head dims above 128: one workgroup per (sequence, head, query), keys in
@@ -712,35 +634,11 @@ __global__ void __launch_bounds__(256) flash_generic_kernel(const FlashArgs a, i
   for (int d = t; d < a.hd; d += 256) orow[d] = ov[d] * inv;
 }
 
-template <int HD, int BN, bool CAUSAL, bool HAS_MASK, bool VEC>
-void launch_sched(const FlashArgs &a, hipStream_t st) {
-  // Pairs of causal tiles when one tile per workgroup would fit in a single
-  // round of resident workgroups (four per CU), so that the round lasts as
-  // long as its longest tile, and the pairs still give every CU two
-  // workgroups (fewer would leave SIMDs with a single wave).  Only for
-  // sequences of at most four query tiles: with more, one workgroup per tile
-  // (which keeps the no-maximum sub-block path) measured 3-6% faster
-  // (c2, 16 x 1024 with 8 heads of 64: 161-167 against 172-175 us; 8 x 2048
-  // heads of 64: 294-296 against 310 us), while 32 x 512 heads of 64 still
-  // gain 4-6% from pairs.
-  const long long cus = num_cus();
-  FlashArgs b = a;
-  if constexpr (CAUSAL) {
-    const long long pairs = (long long)a.n_bh * ((a.n_qt + 1) / 2);
-    if (a.n_qt > 1 && a.n_qt <= 4 && (long long)a.n_items <= 4 * cus && pairs >= 2 * cus) {
-      b.fast = 0;
-      flash_fwd_kernel<HD, BN, CAUSAL, HAS_MASK, VEC, kPair><<<dim3((unsigned)pairs), dim3(FA_THREADS), 0, st>>>(b);
-      return;
-    }
-  }
-  b.fast = (long long)a.n_items >= 3 * cus;
-  flash_fwd_kernel<HD, BN, CAUSAL, HAS_MASK, VEC, kOne><<<dim3(a.n_items), dim3(FA_THREADS), 0, st>>>(b);
-}
-
 template <int HD, int BN, bool CAUSAL, bool HAS_MASK>
 void launch_tpl(const FlashArgs &a, bool vec, hipStream_t st) {
-  if (vec) launch_sched<HD, BN, CAUSAL, HAS_MASK, true>(a, st);
-  else launch_sched<HD, BN, CAUSAL, HAS_MASK, false>(a, st);
+  const dim3 grid(a.n_items), block(FA_THREADS);
+  if (vec) flash_fwd_kernel<HD, BN, CAUSAL, HAS_MASK, true><<<grid, block, 0, st>>>(a);
+  else flash_fwd_kernel<HD, BN, CAUSAL, HAS_MASK, false><<<grid, block, 0, st>>>(a);
 }
 
 template <int HD, int BN>
@@ -803,7 +701,7 @@ int flash_forward(const float *q, int ldq, const float *k, int ldk, const float 
   long long total = (long long)batch * num_heads * a.n_qt;
   if (total > (1LL << 30)) return fail(CDML_E_INVALID, "cdml_sdpa_fwd: problem too large");
   a.n_items = (int)total;
-  if (hd_pad == 32) launch_hd<32, 64>(a, causal, vec, st);
+  if (hd_pad == 32) launch_hd<32, 32>(a, causal, vec, st);
   else if (hd_pad == 64) launch_hd<64, 32>(a, causal, vec, st);
   else launch_hd<128, 32>(a, causal, vec, st);
   return check_launch("flash_fwd_kernel");

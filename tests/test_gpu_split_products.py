@@ -65,3 +65,68 @@ def test_values_outside_the_split(rows, ind, out):
     wg, bg, dx = G.linear_backward(x, dy, w, np.zeros((out, ind), np.float32), np.zeros(out, np.float32))
     check(dx, dy, w, "input gradient")
     check(wg, dy.T, x, "weight gradient")
+
+
+def attention64(q, k, v, heads, scale, causal):
+    """float64 softmax attention of one sequence; (o, sum p |v|, largest sum |q| |k| of a row's scores)."""
+    L, D = q.shape
+    hd = D // heads
+    o, w, m = (np.zeros((L, D)) for _ in range(3))
+    for h in range(heads):
+        c = slice(h * hd, (h + 1) * hd)
+        Q, K, V = (t[:, c].astype(np.float64) for t in (q, k, v))
+        with np.errstate(all="ignore"):
+            s, a = Q @ K.T * scale, np.abs(Q) @ np.abs(K).T * abs(scale)
+            if causal:
+                s = np.where(np.tril(np.ones(s.shape, bool)), s, -np.inf)
+                a = np.where(np.tril(np.ones(s.shape, bool)), a, 0)
+            p = np.exp(s - s.max(1, keepdims=True))
+            p /= p.sum(1, keepdims=True)
+            o[:, c], w[:, c], m[:, c] = p @ V, p @ np.abs(V), a.max(1, keepdims=True)
+    return o, w, m
+
+
+def check_attention(got, q, k, v, heads, scale, causal, what):
+    """A score's error is (hd / 8 + 8) 2^-24 sum |q| |k| scale, which moves a probability by as much
+    relatively; the sums over keys add (L / 8 + 8) 2^-24, exp2 and the scaling a few 2^-23."""
+    L, D = q.shape
+    want, w, m = attention64(q, k, v, heads, scale, causal)
+    assert np.array_equal(np.isnan(got), np.isnan(want)), f"{what}: NaNs elsewhere"
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf]), f"{what}: infinities"
+    fine = np.isfinite(want)
+    bound = (2 * (D // heads / 8 + 8) * m + L / 8 + 32) * 2.0 ** -24 * w
+    with np.errstate(invalid="ignore"):
+        err = np.abs(got.astype(np.float64) - want)
+    assert np.all(err[fine] <= bound[fine]), f"{what}: {np.nanmax(err[fine] / bound[fine]):.3g} of the bound"
+
+
+# head dims on both sides of the padded sizes 32, 64 and 128 (40 and 20 take the scalar loads), lengths around a
+# 32-key tile, a wave's 32 and a workgroup's 128 queries
+@pytest.mark.parametrize("L", [1, 31, 33, 127, 129, 300])
+@pytest.mark.parametrize("hd", [20, 32, 40, 64, 128])
+def test_attention_forward(hd, L):
+    heads = 2
+    q, k, v = (synth.normal(i, (L, heads * hd)) for i in (1, 2, 3))
+    q = q * np.float32(3.0)  # probabilities over many binades
+    for causal in (False, True):
+        got = G.sdpa(q, k, v, heads, causal=causal, scale=1.0 / np.sqrt(hd))
+        check_attention(got, q, k, v, heads, 1.0 / np.sqrt(hd), causal, f"hd {hd} L {L} causal {causal}")
+
+
+@pytest.mark.parametrize("hd", [32, 40, 64, 128])
+def test_attention_values_outside_the_split(hd):
+    """Rows that an infinity, a NaN or a value above the largest bf16 reaches come out as the fp32 products give
+    them; the others are untouched."""
+    L, heads = 130, 2
+    q, k, v = (synth.normal(i, (L, heads * hd)) for i in (4, 5, 6))
+    q[7, 3], v[0, hd + 1] = np.nan, 3.4e38
+    k[40, :] = 0.0
+    k[40, 2] = -np.inf  # score -inf or +inf by the sign of q: weight 0, or a row of NaNs
+    for causal in (False, True):
+        got = G.sdpa(q, k, v, heads, causal=causal, scale=1.0 / np.sqrt(hd))
+        check_attention(got, q, k, v, heads, 1.0 / np.sqrt(hd), causal, f"hd {hd} causal {causal}")
+    q, k = (synth.normal(i, (L, heads * hd)) for i in (4, 5))
+    v[5, 1] = np.inf  # every row sees it without the causal rule
+    got = G.sdpa(q, k, v, heads, scale=1.0 / np.sqrt(hd))
+    check_attention(got, q, k, v, heads, 1.0 / np.sqrt(hd), False, f"hd {hd} infinite value")
