@@ -1,5 +1,5 @@
 // Attention backward for gfx950: MultiHeadAttentionBackward of the reference
-// (AccelerationCPU.cs:1011-1280) on fp32 MFMA.
+// (AccelerationCPU.cs:1011-1280).
 //
 // With P = softmax(S), S = scale * Q K^T per (sequence, head) under the
 // causal rule (key j visible to query i iff j <= i) and/or a mask:
@@ -9,16 +9,18 @@
 //   1. the forward kernel with row statistics: O and lse_i (log2 of the
 //      softmax normaliser), so that P_ij = exp2(s_ij * scale * log2 e - lse_i);
 //   2. bwd_delta_kernel: D = rowsum(dO * O) per head;
-//   3. flash_bwd_dkdv_kernel, key-block major: a workgroup owns 128 keys of
-//      one (sequence, head), each wave 32 keys whose K and V rows stay in
+//   3. dK and dV, key-block major: a workgroup owns 128 keys of one (sequence,
+//      head), 32 to a wave or a pair of waves, whose K and V rows stay in
 //      registers; Q, dO, lse and D tiles stream through double-buffered LDS.
 //      Per 32-query sub-block: S = Q K^T and dP = dO V^T land with one key
 //      per lane and 16 queries per lane in registers, exactly the B operand
 //      layout that dV^T += dO^T P and dK^T += Q^T dS need, so P and dS are
-//      consumed in place;
-//   4. flash_bwd_dq_kernel, query-block major like the forward: S^T = K Q^T
-//      and dP^T = V dO^T put one query per lane, dS^T is consumed in place by
-//      dQ^T += K^T dS^T.
+//      consumed in place (flash_bwd_dkdv_split_kernel on bf16 pieces for head
+//      dims up to 64, flash_bwd_dkdv_kernel on fp32 MFMA above);
+//   4. dQ, query-block major like the forward: from dS blocks that step 3 stored
+//      (flash_bwd_dq_ds_kernel, on bf16 pieces), or recomputed on fp32 MFMA
+//      (flash_bwd_dq_kernel): S^T = K Q^T and dP^T = V dO^T put one query per
+//      lane, dS^T is consumed in place by dQ^T += K^T dS^T.
 // Every output element is written by one lane of one workgroup: no atomics,
 // and the result is the same on every run.  Head dims below 128 other than
 // 32 and 64, or rows that are not 16-byte aligned, run the same kernels at the
@@ -153,18 +155,60 @@ __global__ void __launch_bounds__(256) bwd_delta_scalar_kernel(const BwdArgs a) 
   a.delta[((size_t)b * a.heads + h) * a.lq + i] = s;
 }
 
-// dK and dV.  Workgroup i takes (sequence, head) i % n_bh and key tile
-// i / n_bh: under the causal rule the first key tiles are seen by the most
-// queries, so the heaviest tiles go out first on every XCD.
-//
-// With STORE_DS (causal, lq == lk) the kernel also writes every dS sub-block
-// it forms, for flash_bwd_dq_ds_kernel: block (query block i, key block j),
-// j <= i, holds 32 x 32 floats at ds + bh * ds_bh + (i (i + 1) / 2 + j) * 1024,
-// query row r of the block at [32 r, 32 r + 32) with key 2s + c at 16 c + s,
-// which is the A operand order of the dQ product (16 contiguous floats per
-// lane).
-template <int HD, int BQ, bool CAUSAL, bool HAS_MASK, bool VEC, bool STORE_DS>
-__global__ void __launch_bounds__(BW_THREADS, (HD <= 32 && !HAS_MASK) ? 3 : (HD <= 64 ? 2 : 1)) flash_bwd_dkdv_kernel(const BwdArgs a) {
+// Stores one row of a gradient: this lane's x (register 4g + c of block db is
+// dimension db*32 + 8g + 4*hf + c) times scale, rotated back by the pairs of
+// rope_cs when non-NULL (the table row of its position).
+template <int HD, bool VEC>
+__device__ __forceinline__ void store_column(const BwdArgs &a, const floatx16 (&x)[HD / 32], float *row, float scale,
+                                             const float2 *rope_cs, int hf) {
+  constexpr int NDB = HD / 32;
+  // (cos, sin) of the row's pairs, loaded before any store (a load issued after
+  // a store waits for it)
+  float2 cs[NDB][4][2];
+  if (rope_cs) {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int d = db * 32 + 8 * g + 4 * hf + 2 * j;
+          cs[db][g][j] = d < a.hd ? rope_cs[d >> 1] : make_float2(1.f, 0.f);
+        }
+  }
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = db * 32 + 8 * g + 4 * hf;
+      vf4 y;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) y[c] = x[db][4 * g + c] * scale;
+      if (rope_cs) {  // dims d + c and d + c + 1 are one pair, in this lane
+#pragma unroll
+        for (int c = 0; c < 4; c += 2) {
+          const float2 r = rope_inverse_pair(y[c], y[c + 1], cs[db][g][c >> 1]);
+          y[c] = r.x;
+          y[c + 1] = r.y;
+        }
+      }
+      if constexpr (VEC) {
+        *reinterpret_cast<vf4 *>(row + d) = y;
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (d + c < a.hd) row[d + c] = y[c];
+      }
+    }
+  }
+}
+
+// dK and dV on fp32 MFMA, for head dims above 64: two tensors' pieces of a
+// wave's keys need 384 registers there.  Workgroup i takes (sequence, head)
+// i % n_bh and key tile i / n_bh: under the causal rule the first key tiles are
+// seen by the most queries, so the heaviest tiles go out first on every XCD.
+template <int HD, int BQ, bool CAUSAL, bool HAS_MASK, bool VEC>
+__global__ void __launch_bounds__(BW_THREADS, HD <= 64 ? 2 : 1) flash_bwd_dkdv_kernel(const BwdArgs a) {
   constexpr int NQB = BQ / 32;  // 32-query sub-blocks per tile
   constexpr int NDB = HD / 32;  // 32-wide head-dim blocks of dK^T / dV^T
   constexpr int NKG = HD / 8;   // 8-dim groups of the Q.K and dO.V products
@@ -231,12 +275,6 @@ __global__ void __launch_bounds__(BW_THREADS, (HD <= 32 && !HAS_MASK) ? 3 : (HD 
   sq.init(a.ldq);
   sg.init(a.lddo);
   float lreg = 0.f, dreg = 0.f;
-  // The stored dS blocks of this (sequence, head) as a buffer resource (the
-  // launch keeps ds_bh * 4 bytes within 2^31), and the byte offset of this
-  // lane's entries in a block (row 4 hf + acc_row(r), key li).
-  const __amdgpu_buffer_rsrc_t ds_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      STORE_DS ? a.ds + (size_t)bh * a.ds_bh : nullptr, (short)0, STORE_DS ? (int)(a.ds_bh * 4) : 0, kBufferWord3);
-  const int ds_lane = 4 * (4 * hf * 32 + (li & 1) * 16 + (li >> 1));
   if (n_it > 0) {
     sq.load(qbase, a.ldq, q_begin, a.lq, a.hd);
     sg.load(gbase, a.lddo, q_begin, a.lq, a.hd);
@@ -336,22 +374,6 @@ __global__ void __launch_bounds__(BW_THREADS, (HD <= 32 && !HAS_MASK) ? 3 : (HD 
           }
         }
       }
-      if constexpr (STORE_DS) {
-        // buffer stores: the block's byte offset in a scalar register, this
-        // lane's fixed offset plus the row's immediate (one VGPR of address).
-        // Non-temporal (the nt bit): the blocks stream to HBM rather than
-        // sitting dirty in the caches, where the dQ pass's reads would evict
-        // and write them back under its own traffic (c5 attention backward
-        // 1170 -> 1146 us, c3 2902 -> 2841 us; non-temporal loads in the dQ
-        // pass were slower).
-        const int qi = qb0 >> 5, kj = kw0 >> 5;
-        const int boff = (qi * (qi + 1) / 2 + kj) * 4096;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dp[r]), ds_rsrc, ds_lane + 128 * acc_row(r), boff,
-                                                kCachePolicyNT);
-      }
-
       // dV^T += dO^T P and dK^T += Q^T dS: MFMA step st pairs query rows
       // acc_row(st) (half 0) and acc_row(st) + 4 (half 1), the rows held by
       // register st of P and dS.
@@ -375,57 +397,443 @@ __global__ void __launch_bounds__(BW_THREADS, (HD <= 32 && !HAS_MASK) ? 3 : (HD 
     __syncthreads();
   }
 
-  // Lane li holds key `key`: register 4g + c of block db is dimension
-  // db*32 + 8g + 4*hf + c.
   if (key < a.lk) {
-    float *dkrow = a.dk + ((size_t)b * a.lk + key) * a.lddk + col0;
-    float *dvrow = a.dv + ((size_t)b * a.lk + key) * a.lddv + col0;
-    // (cos, sin) of this key's pairs, loaded before any store (a load issued
-    // after a store waits for it)
-    float2 cs[NDB][4][2];
-    if (a.rope_cs) {
-      const float2 *t = a.rope_cs + (size_t)key * (a.hd >> 1);
+    const size_t krow = (size_t)b * a.lk + key;
+    store_column<HD, VEC>(a, dk, a.dk + krow * a.lddk + col0, a.scale,
+                          a.rope_cs ? a.rope_cs + (size_t)key * (a.hd >> 1) : nullptr, hf);
+    store_column<HD, VEC>(a, dv, a.dv + krow * a.lddv + col0, 1.f, nullptr, hf);
+  }
+}
+
+// One tile of 32 query rows of Q and of dO for the split dK/dV kernel, split
+// into three bf16 pieces on its way into LDS, each tensor in two layouts (rows of
+// 16 values = 32 bytes, one plane per piece, as the GEMM's operand tiles):
+//   rows:       slab s holds dims 16 s .. 16 s + 15 of every query (S and dP);
+//               even and odd queries in two clusters;
+//   transposed: slab s holds queries 16 s .. 16 s + 15 of every dim (dV and dK),
+//               query k of a slab at place 8 (k / 4 % 2) + 4 (k / 8) + k % 4, the
+//               order in which the score accumulators hold them; four clusters by
+//               d % 4.
+// Odd dims are negated in both (common.h); K and V carry the same sign in the
+// wave's registers, and the stores undo it.  A unit is four dims of two queries:
+// its pieces are packed along the queries as they are split and repacked along
+// the dims by byte permutes.
+template <int HD, bool VEC>
+struct QgStage {
+  static constexpr int CH = HD / 4;
+  static constexpr int UNITS = CH * 16;                        // of one tensor
+  static constexpr int NU = 2 * UNITS / BW_THREADS;            // per thread: 2 (Q and dO) or 1 (either)
+  static constexpr int RSLAB = 2 * 512 + 128, TSLAB = 4 * (CH * 32) + 256;
+  static constexpr int RPLANE = HD / 16 * RSLAB, TPLANE = 2 * TSLAB;
+  static constexpr int TENSOR = 3 * (RPLANE + TPLANE);         // rows planes, then transposed planes
+  static constexpr int BYTES = 2 * TENSOR;
+  static_assert(NU == 1 || NU == 2, "tile units");
+  static __device__ __forceinline__ constexpr int rcluster(int c) { return c * (512 + 16); }
+  static __device__ __forceinline__ constexpr int tcluster(int c) { return c * CH * 32 + (c & 1) * 16 + (c >> 1) * 128; }
+  vf4 r[NU][2];
+  int row, col, rdst, tdst;  // first query and dim of the unit, its places in the two layouts
+  bool gside;                // NU == 1: this thread stages dO
+
+  __device__ __forceinline__ void init() {
+    const int t = threadIdx.x;  // the staging waves are the first four
+    gside = NU == 1 && __builtin_amdgcn_readfirstlane(t) >= UNITS;
+    const int u = t % UNITS, sb = u & 7, g = (u >> 3) % CH, slab = (u >> 3) / CH;
+    row = 16 * slab + 2 * sb;
+    col = 4 * g;
+    const int place = ((sb >> 1) & 1) * 4 + (sb >> 2) * 2 + (sb & 1);  // of the query pair
+    rdst = (g >> 2) * RSLAB + (row >> 1) * 32 + (g & 3) * 8;
+    tdst = 3 * RPLANE + slab * TSLAB + g * 32 + place * 4;
+  }
+  __device__ __forceinline__ void load(const float *__restrict__ qbase, const float *__restrict__ gbase, int ldq,
+                                       int ldg, int row0, int nrows, int hd) {
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
+    for (int i = 0; i < NU; ++i) {
+      const bool g = NU == 1 ? gside : i == 1;
+      const int ld = g ? ldg : ldq;
+      const float *tile = (g ? gbase : qbase) + (size_t)row0 * ld;  // wave-uniform
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+      for (int x = 0; x < 2; ++x) {
+        const float *p = tile + (uint32_t)(min(row + x, nrows - 1 - row0) * ld + col);
+        if constexpr (VEC) {
+          r[i][x] = *reinterpret_cast<const vf4 *>(p);
+        } else {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const int d = db * 32 + 8 * g + 4 * hf + 2 * j;
-            cs[db][g][j] = d < a.hd ? t[d >> 1] : make_float2(1.f, 0.f);
-          }
+          for (int c = 0; c < 4; ++c) r[i][x][c] = col + c < hd ? p[c] : 0.f;
+        }
+      }
     }
+  }
+  __device__ __forceinline__ void store(char *lds) const {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      char *base = lds + (NU == 1 ? (gside ? TENSOR : 0) : i * TENSOR);
+      uint32_t w[3][4];  // [piece][dim]: query `row` in the low half, `row + 1` in the high half
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float x = r[i][0][c], y = r[i][1][c];
+        split_bf16x3(c & 1 ? -x : x, c & 1 ? -y : y, w[0][c], w[1][c], w[2][c]);
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          *reinterpret_cast<uint32_t *>(base + tdst + q * TPLANE + tcluster(c)) = w[q][c];
+        // low halves of two words, high halves of two words
+        const vu2 even = {__builtin_amdgcn_perm(w[q][1], w[q][0], 0x05040100), __builtin_amdgcn_perm(w[q][3], w[q][2], 0x05040100)};
+        const vu2 odd = {__builtin_amdgcn_perm(w[q][1], w[q][0], 0x07060302), __builtin_amdgcn_perm(w[q][3], w[q][2], 0x07060302)};
+        *reinterpret_cast<vu2 *>(base + rdst + q * RPLANE) = even;
+        *reinterpret_cast<vu2 *>(base + rdst + q * RPLANE + rcluster(1)) = odd;
+      }
+    }
+  }
+  // Byte offsets of a lane's operands in plane 0 of a tensor.
+  static __device__ __forceinline__ int roperand(int li, int hf) {
+    return rcluster(li & 1) + (li >> 1) * 32 + hf * 16;
+  }
+  static __device__ __forceinline__ int toperand(int li, int hf) {
+    return 3 * RPLANE + tcluster(li & 3) + (li >> 2) * 32 + hf * 16;
+  }
+};
+
+// dK and dV on three bf16 pieces per fp32 operand (common.h), head dims up to 64;
+// workgroups over keys as flash_bwd_dkdv_kernel's.
+//
+// Head dim 64: a pair of waves owns 32 keys.  Wave w (0..3) holds K's pieces,
+// forms S and P and sums dV; wave w + 4 holds V's, forms dP, takes P through LDS,
+// forms and stores dS and sums dK.  A pair shares a SIMD, so one wave's
+// exponentials and splits run under the other's products, and each needs 221
+// registers (one wave for both needs 470 and is alone on its SIMD: 35% of the
+// cycles in the matrix pipes, paired 47%).  Per 32-query tile, two barriers: P is
+// written before the first, read after it.  Head dim 32: one wave does both in
+// 246 registers, two workgroups to a CU; pairs took 31% longer there, half the
+// products per barrier.
+// 4 x 4096 x 16 heads x 64, whole backward: 5.13 -> 3.92 ms; 511 x 256 x 8 x 32:
+// 2.33 -> 1.93 ms (this kernel 1.40 -> 1.05 ms), bound by the exponentials and splits
+// between the products: vector ALU 48% of the cycles, matrix pipes 34%.
+//
+// S and dP of odd keys are computed negated, so that the drift of the bf16 MFMA
+// (common.h) cancels in a query's sum of dS over its keys, which has to be zero.
+//
+// With STORE_DS (causal, lq == lk) the kernel also writes every dS sub-block
+// it forms, for flash_bwd_dq_ds_kernel: block (query block i, key block j),
+// j <= i, holds 32 x 32 floats at ds + bh * ds_bh + (i (i + 1) / 2 + j) * 1024,
+// query row r of the block at [32 r, 32 r + 32) with key 2s + c at 16 c + s,
+// which is the operand order of the dQ product (16 contiguous floats per lane).
+__host__ __device__ constexpr bool paired_keys(int hd) { return hd > 32; }
+template <int HD, bool CAUSAL, bool HAS_MASK, bool VEC, bool STORE_DS>
+__global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS, 2) flash_bwd_dkdv_split_kernel(const BwdArgs a) {
+  constexpr int BQ = 32;
+  constexpr int NDB = HD / 32;  // 32-wide head-dim blocks of dK^T / dV^T
+  constexpr int NS = HD / 16;   // MFMA k-steps of Q.K and dO.V
+  constexpr bool PAIRED = paired_keys(HD);
+  constexpr int NT = PAIRED ? 1 : 2;  // gradients of a wave: dV or dK, or dV (0) and dK (1)
+  typedef QgStage<HD, VEC> Stage;
+  __shared__ __attribute__((aligned(16))) char lds[2][Stage::BYTES];
+  __shared__ __attribute__((aligned(16))) vf4 Ps[PAIRED ? 4 : 1][4][64];  // P of a pair, as its lanes hold it
+  __shared__ __attribute__((aligned(16))) float Ls[2][BQ];   // lse
+  __shared__ __attribute__((aligned(16))) float Ds[2][BQ];   // D
+
+  const int n_bh = a.batch * a.heads;
+  const int bh = blockIdx.x % n_bh, kt = blockIdx.x / n_bh;
+  const int b = bh / a.heads, h = bh % a.heads;
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int pair = wave & 3;
+  const bool role_p = wave < 4;  // P and dV; else dS and dK
+  const int li = lane & 31, hf = lane >> 5;
+  const int k0 = kt * BW_TILE;
+  const int kw0 = k0 + pair * 32;  // first key of this pair
+  const int key = kw0 + li;        // this lane's key
+  const int col0 = h * (VEC ? HD : a.hd);
+
+  // B operands of S = Q K^T and / or dP = dO V^T: the pieces of K[key][16 s + 8 hf
+  // + 0..7] and of V, odd dims negated as in the staged tiles, and odd keys.
+  bf16x8 kv[NT][NS][3];
+#pragma unroll
+  for (int x = 0; x < NT; ++x) {
+    const size_t kr = (size_t)b * a.lk + min(key, a.lk - 1);
+    const float *row = (PAIRED ? role_p : x == 0) ? a.k + kr * a.ldk + col0 : a.v + kr * a.ldv + col0;
+    const uint32_t odd_key = (uint32_t)(li & 1) << 31;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int d = 16 * s + 8 * hf + e;
+        const float v = VEC || d < a.hd ? row[d] : 0.f;
+        f[e] = __uint_as_float(__float_as_uint(e & 1 ? -v : v) ^ odd_key);
+      }
+      split_operand(f, kv[x][s]);
+    }
+  }
+
+  const int q_begin = CAUSAL ? k0 : 0;  // queries before k0 see none of these keys
+  const int n_it = q_begin < a.lq ? (a.lq - q_begin + BQ - 1) / BQ : 0;
+  const float *__restrict__ qbase = a.q + (size_t)b * a.lq * a.ldq + col0;
+  const float *__restrict__ gbase = a.dout + (size_t)b * a.lq * a.lddo + col0;
+  const float *__restrict__ lse = a.lse + (size_t)bh * a.lq;
+  const float *__restrict__ dlt = a.delta + (size_t)bh * a.lq;
+
+  floatx16 acc[NT][NDB], cor[NT][NDB];  // hh, and its corrections
+#pragma unroll
+  for (int x = 0; x < NT; ++x)
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[x][db][r] = cor[x][db][r] = 0.f;
+
+  // P = exp2(S scale log2 e - lse) in place; scale_log2 carries the sign of an
+  // odd key.  l4(g): lse of query rows 8 g + 4 hf + 0..3 of the sub-block.
+  auto probabilities = [&](floatx16 &s, float scale_log2, int qb0, auto l4) {
+    // (the masked and the unmasked forms are separate branches: a select
+    // per element would run the mask arithmetic on every sub-block)
+    const bool need = HAS_MASK || (CAUSAL && qb0 < kw0 + 31) || qb0 + 31 >= a.lq;
+    if (need) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const vf4 l = l4(g);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int r = 4 * g + c;
+          const int qq = qb0 + 8 * g + 4 * hf + c;
+          bool ok = qq < a.lq;
+          if (CAUSAL) ok = ok && key <= qq;
+          if (HAS_MASK) ok = ok && key < a.lk && a.mask[(size_t)min(qq, a.lq - 1) * a.lk + min(key, a.lk - 1)];
+          s[r] = ok ? fast_exp2(fmaf(s[r], scale_log2, -l[c])) : 0.f;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const vf4 l = l4(g);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[4 * g + c] = fast_exp2(fmaf(s[4 * g + c], scale_log2, -l[c]));
+      }
+    }
+  };
+  // dS = P (sgn dP - D) in place of dP, and the dS store.
+  auto score_gradients = [&](const floatx16 &p, floatx16 &dp, float sgn, int qb0, auto d4) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const vf4 d = d4(g);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) dp[4 * g + c] = p[4 * g + c] * fmaf(sgn, dp[4 * g + c], -d[c]);
+    }
+    if constexpr (STORE_DS) {
+      // The stored dS blocks of this (sequence, head) as a buffer resource (the
+      // launch keeps ds_bh * 4 bytes within 2^31): the block's byte offset in a
+      // scalar register, this lane's fixed offset plus the row's immediate (one
+      // VGPR of address).  Non-temporal (the nt bit): the blocks stream to HBM
+      // rather than sitting dirty in the caches, where the dQ pass's reads would
+      // evict and write them back under its own traffic.
+      const __amdgpu_buffer_rsrc_t ds_rsrc = __builtin_amdgcn_make_buffer_rsrc(a.ds + (size_t)bh * a.ds_bh, (short)0,
+                                                                               (int)(a.ds_bh * 4), kBufferWord3);
+      const int ds_lane = 4 * (4 * hf * 32 + (li & 1) * 16 + (li >> 1));
+      const int qi = qb0 >> 5, kj = kw0 >> 5;
+      const int boff = (qi * (qi + 1) / 2 + kj) * 4096;
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dp[r]), ds_rsrc, ds_lane + 128 * acc_row(r), boff,
+                                              kCachePolicyNT);
+    }
+  };
+  // The 32 x 32 product of the staged rows of one tensor with K's or V's pieces.
+  const int ro = Stage::roperand(li, hf), to = Stage::toperand(li, hf);
+  auto row_product = [&](const char *rows, const bf16x8 (&w)[NS][3]) {
+    floatx16 m = {}, c = {};
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      bf16x8 x[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        x[p] = *reinterpret_cast<const bf16x8 *>(rows + ro + p * Stage::RPLANE + u * Stage::RSLAB);
+#pragma unroll
+      for (int i = 0; i < kSplitProducts; ++i) {
+        floatx16 &z = i == kSplitMain ? m : c;
+        z = mfma32x32x16(x[kSplitA[i]], w[u][kSplitB[i]], z);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) m[r] += c[r];
+    return m;
+  };
+  // acc[n] += (the staged transposed rows of one tensor) x w, w the 32 x 32 P or dS.
+  auto column_product = [&](const char *cols, const floatx16 &w, int n) {
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = w[8 * st + e];
+      bf16x8 wp[3];
+      split_operand(x, wp);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) {
+        bf16x8 g[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          g[p] = *reinterpret_cast<const bf16x8 *>(cols + to + p * Stage::TPLANE + st * Stage::TSLAB + db * 256);
+#pragma unroll
+        for (int i = 0; i < kSplitProducts; ++i) {
+          floatx16 &z = i == kSplitMain ? acc[n][db] : cor[n][db];
+          z = mfma32x32x16(g[kSplitA[i]], wp[kSplitB[i]], z);
+        }
+      }
+    }
+  };
+  // Sub-blocks wholly before these keys contribute nothing, and keys that all
+  // lie past lk take nothing.
+  auto active = [&](int qb0) { return kw0 < a.lk && !(CAUSAL && qb0 + 31 < kw0); };
+  const float sgn = li & 1 ? -1.f : 1.f;
+
+  auto lse4 = [&](int buf) {
+    return [&, buf](int g) { return *reinterpret_cast<const vf4 *>(&Ls[buf][8 * g + 4 * hf]); };
+  };
+  auto delta4 = [&](int buf) {
+    return [&, buf](int g) { return *reinterpret_cast<const vf4 *>(&Ds[buf][8 * g + 4 * hf]); };
+  };
+
+  if (!PAIRED || role_p) {
+    // Where waves are paired, the staging ones store nothing to memory, so that
+    // waiting for a tile's loads never waits for the dS stores.
+    Stage sg;
+    sg.init();
+    float lreg = 0.f, dreg = 0.f;
+    auto fetch = [&](int it) {  // past the end: the last tile again, into a buffer that nothing reads
+      const int row0 = q_begin + min(it, n_it - 1) * BQ;
+      sg.load(qbase, gbase, a.ldq, a.lddo, row0, a.lq, a.hd);
+      if (t < BQ) {
+        const int qq = min(row0 + t, a.lq - 1);
+        lreg = lse[qq];
+        dreg = dlt[qq];
+      }
+    };
+    auto stage = [&](int buf) {
+      sg.store(lds[buf]);
+      if (t < BQ) {
+        Ls[buf][t] = lreg;
+        Ds[buf][t] = dreg;
+      }
+    };
+    if (n_it > 0) {
+      fetch(0);
+      stage(0);
+    }
+    __syncthreads();
+    for (int it = 0; it < n_it; ++it) {
+      const int cur = it & 1, qb0 = q_begin + it * BQ;
+      fetch(it + 1);
+      floatx16 p;
+      if (active(qb0)) {
+        p = row_product(lds[cur], kv[0]);
+        if constexpr (PAIRED) {
+          probabilities(p, sgn * a.scale_log2, qb0, lse4(cur));
+#pragma unroll
+          for (int g = 0; g < 4; ++g) Ps[pair][g][lane] = vf4{p[4 * g], p[4 * g + 1], p[4 * g + 2], p[4 * g + 3]};
+        } else {
+          floatx16 dp = row_product(lds[cur] + Stage::TENSOR, kv[NT - 1]);
+          probabilities(p, sgn * a.scale_log2, qb0, lse4(cur));
+          column_product(lds[cur] + Stage::TENSOR, p, 0);
+          score_gradients(p, dp, sgn, qb0, delta4(cur));
+          column_product(lds[cur], dp, NT - 1);
+        }
+      }
+      if constexpr (PAIRED) {
+        __syncthreads();
+        if (active(qb0)) column_product(lds[cur] + Stage::TENSOR, p, 0);  // dV^T += dO^T P
+      }
+      stage(cur ^ 1);
+      __syncthreads();
+    }
+  } else {
+    __syncthreads();
+    for (int it = 0; it < n_it; ++it) {
+      const int cur = it & 1, qb0 = q_begin + it * BQ;
+      floatx16 dp;
+      if (active(qb0)) dp = row_product(lds[cur] + Stage::TENSOR, kv[0]);
+      __syncthreads();
+      if (active(qb0)) {
+        floatx16 p;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const vf4 x = Ps[pair][g][lane];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) p[4 * g + c] = x[c];
+        }
+        score_gradients(p, dp, sgn, qb0, delta4(cur));
+        column_product(lds[cur], dp, 0);  // dK^T += Q^T dS
+      }
+      __syncthreads();
+    }
+  }
+
+  // odd dims (registers of odd index) were negated
+  float bad = 0.f;
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = db * 32 + 8 * g + 4 * hf;
-        vf4 x, y;
+      for (int r = 0; r < 16; ++r) {
+        const float x = acc[n][db][r] + cor[n][db][r];
+        acc[n][db][r] = r & 1 ? -x : x;
+      }
+      bad = nonfinite_sum(acc[n][db], bad);
+    }
+  }
+  if (any_nonfinite(bad) && kw0 < a.lk) {
+    // An infinity or a NaN reached these keys, or a product overflowed: the
+    // whole column on the fp32 MFMA straight from memory, dS blocks included.
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          x[c] = dk[db][4 * g + c] * a.scale;
-          y[c] = dv[db][4 * g + c];
-        }
-        if (a.rope_cs) {  // dims d + c and d + c + 1 are one pair, in this lane
+    for (int n = 0; n < NT; ++n)
 #pragma unroll
-          for (int c = 0; c < 4; c += 2) {
-            const float2 r = rope_inverse_pair(x[c], x[c + 1], cs[db][g][c >> 1]);
-            x[c] = r.x;
-            x[c + 1] = r.y;
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][db][r] = 0.f;
+    const size_t krow = (size_t)b * a.lk + min(key, a.lk - 1);
+#pragma unroll 1
+    for (int qb0 = CAUSAL ? kw0 : 0; qb0 < a.lq; qb0 += 32) {
+      floatx16 s = {}, dp = {};
+      const size_t qrow = min(qb0 + li, a.lq - 1);
+#pragma unroll 1
+      for (int d = hf; d < a.hd + hf; d += 2) {
+        const bool in = d < a.hd;
+        const int dc = in ? d : 0;
+        s = mfma32x32x2(in ? qbase[qrow * a.ldq + dc] : 0.f, in ? a.k[krow * a.ldk + col0 + dc] : 0.f, s);
+        dp = mfma32x32x2(in ? gbase[qrow * a.lddo + dc] : 0.f, in ? a.v[krow * a.ldv + col0 + dc] : 0.f, dp);
+      }
+      auto four = [&](const float *x, int g) {
+        vf4 v;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = x[min(qb0 + 8 * g + 4 * hf + c, a.lq - 1)];
+        return v;
+      };
+      probabilities(s, a.scale_log2, qb0, [&](int g) { return four(lse, g); });
+      if (!PAIRED || !role_p) score_gradients(s, dp, 1.f, qb0, [&](int g) { return four(dlt, g); });
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const bool of_v = PAIRED ? role_p : n == 0;
+        const float *base = of_v ? gbase : qbase;
+        const int ld = of_v ? a.lddo : a.ldq;
+#pragma unroll
+        for (int st = 0; st < 16; ++st) {
+          const size_t qr = min(qb0 + acc_row(st) + 4 * hf, a.lq - 1);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            const int d = db * 32 + li;
+            acc[n][db] = mfma32x32x2(d < a.hd ? base[qr * ld + d] : 0.f, of_v ? s[st] : dp[st], acc[n][db]);
           }
         }
-        if constexpr (VEC) {
-          *reinterpret_cast<vf4 *>(dkrow + d) = x;
-          *reinterpret_cast<vf4 *>(dvrow + d) = y;
-        } else {
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (d + c < a.hd) {
-              dkrow[d + c] = x[c];
-              dvrow[d + c] = y[c];
-            }
-        }
       }
+    }
+  }
+  if (key < a.lk) {
+    const size_t krow = (size_t)b * a.lk + key;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      if (PAIRED ? role_p : n == 0) store_column<HD, VEC>(a, acc[n], a.dv + krow * a.lddv + col0, 1.f, nullptr, hf);
+      else store_column<HD, VEC>(a, acc[n], a.dk + krow * a.lddk + col0, a.scale,
+                                 a.rope_cs ? a.rope_cs + (size_t)key * (a.hd >> 1) : nullptr, hf);
     }
   }
 }
@@ -575,62 +983,70 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_kernel(const BwdAr
     __syncthreads();
   }
 
-  if (qi < a.lq) {
-    float *dqrow = a.dq + ((size_t)b * a.lq + qi) * a.lddq + col0;
-    float2 cs[NDB][4][2];  // (cos, sin) of this row's pairs, loaded before any store
-    if (a.rope_cs) {
-      const float2 *t = a.rope_cs + (size_t)qi * (a.hd >> 1);
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const int d = db * 32 + 8 * g + 4 * hf + 2 * j;
-            cs[db][g][j] = d < a.hd ? t[d >> 1] : make_float2(1.f, 0.f);
-          }
-    }
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = db * 32 + 8 * g + 4 * hf;
-        vf4 x;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) x[c] = dq[db][4 * g + c] * a.scale;
-        if (a.rope_cs) {
-#pragma unroll
-          for (int c = 0; c < 4; c += 2) {
-            const float2 r = rope_inverse_pair(x[c], x[c + 1], cs[db][g][c >> 1]);
-            x[c] = r.x;
-            x[c + 1] = r.y;
-          }
-        }
-        if constexpr (VEC) {
-          *reinterpret_cast<vf4 *>(dqrow + d) = x;
-        } else {
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (d + c < a.hd) dqrow[d + c] = x[c];
-        }
-      }
-    }
-  }
+  if (qi < a.lq)
+    store_column<HD, VEC>(a, dq, a.dq + ((size_t)b * a.lq + qi) * a.lddq + col0, a.scale,
+                          a.rope_cs ? a.rope_cs + (size_t)qi * (a.hd >> 1) : nullptr, hf);
 }
 
-// dQ from the dS blocks that flash_bwd_dkdv_kernel stored (causal, lq == lk,
-// 16-byte aligned rows): dQ = scale dS K, one product instead of recomputing
-// S and dP.  Query-tile major with the heaviest tiles first, as the forward.
-// Wave w owns query block i = q0 / 32 + w; for its key blocks j <= i the A
-// operand (dS[q][2s + c] in lane (q, c) for step s) is 16 contiguous floats
-// per lane, loaded two blocks ahead, and K streams through double-buffered LDS
-// as the B operand.  Lane d of the accumulator holds dQ[q][d] for the 16
-// query rows acc_row(r) + 4 c.
+// K^T tile of the stored-dS dQ kernel: BN keys of one head as 16-value rows of
+// dims (slab s holds keys 16 s .. 16 s + 15, key k of a slab at place
+// 8 (k % 2) + k / 2, the order of the stored dS operands), split into three bf16
+// planes.  A unit is four dims of two keys of equal parity; clusters by d % 4.
+template <int HD, int BN>
+struct KtStage {
+  static constexpr int CH = HD / 4;
+  static constexpr int NU = CH * (BN / 2) / BW_THREADS;
+  static constexpr int SLAB = 4 * (CH * 32) + 256, PLANE = BN / 16 * SLAB, BYTES = 3 * PLANE;
+  static_assert(NU >= 1 && CH * (BN / 2) % BW_THREADS == 0 && (BW_THREADS / 8) % CH == 0, "tile units");
+  static __device__ __forceinline__ constexpr int cluster(int c) { return c * CH * 32 + (c & 1) * 16 + (c >> 1) * 128; }
+  vf4 r[NU][2];
+  int row, col, dst;
+  __device__ __forceinline__ void init() {
+    const int t = threadIdx.x, sb = t & 7, g = (t >> 3) % CH, slab = (t >> 3) / CH;
+    row = 16 * slab + 4 * (sb >> 1) + (sb & 1);  // and row + 2
+    col = 4 * g;
+    dst = slab * SLAB + g * 32 + ((sb & 1) * 4 + (sb >> 1)) * 4;
+  }
+  __device__ __forceinline__ void load(const float *__restrict__ base, int ld, int row0, int nrows) {
+    const float *tile = base + (size_t)row0 * ld;
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+        r[i][x] = *reinterpret_cast<const vf4 *>(
+            tile + (uint32_t)(min(row + 16 * (BW_THREADS / 8 / CH) * i + 2 * x, nrows - 1 - row0) * ld + col));
+  }
+  __device__ __forceinline__ void store(char *lds) const {
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        uint32_t h, m, l;
+        split_bf16x3(r[i][0][c], r[i][1][c], h, m, l);
+        char *d = lds + dst + BW_THREADS / 8 / CH * SLAB * i + cluster(c);
+        *reinterpret_cast<uint32_t *>(d) = h;
+        *reinterpret_cast<uint32_t *>(d + PLANE) = m;
+        *reinterpret_cast<uint32_t *>(d + 2 * PLANE) = l;
+      }
+  }
+  static __device__ __forceinline__ int operand(int li, int hf) { return cluster(li & 3) + (li >> 2) * 32 + hf * 16; }
+};
+
+// dQ from the dS blocks that the dK/dV kernel stored (causal, lq == lk, 16-byte
+// aligned rows): dQ^T = scale K^T dS^T, one product instead of recomputing S and
+// dP, on three bf16 pieces per fp32 operand (common.h).  Query-tile major with
+// the heaviest tiles first, as the forward.  Wave w owns query block i = q0 / 32 +
+// w; for its key blocks j <= i the dS operand (dS[q][2s + c], s = 0..15, in lane
+// (q, c)) is 16 contiguous floats per lane, loaded two blocks ahead, and K^T
+// streams through double-buffered LDS.  A lane ends with one query's dims in
+// registers, so both halves of a rotary pair are in one lane and the stores are
+// 16 bytes wide.  The blocks' bytes bound it: 2.1 GB at 4 x 4096 x 16 heads.
 template <int HD, int BN>
 __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const BwdArgs a) {
   constexpr int NKB = BN / 32;
   constexpr int NDB = HD / 32;
-  __shared__ __attribute__((aligned(16))) float Ks[2][BN][HD + 4];
+  typedef KtStage<HD, BN> Stage;
+  __shared__ __attribute__((aligned(16))) char lds[2][Stage::BYTES];
 
   const int n_bh = a.batch * a.heads;
   const int bh = blockIdx.x % n_bh;
@@ -648,18 +1064,18 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
   const float *__restrict__ kbase = a.k + (size_t)b * a.lk * a.ldk + col0;
   const float *__restrict__ dsw = a.ds + (size_t)bh * a.ds_bh + (size_t)qi * (qi + 1) / 2 * 1024 + li * 32 + hf * 16;
 
-  floatx16 dq[NDB];
+  floatx16 dq[NDB], dqc[NDB];  // hh, and its corrections
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
+    for (int r = 0; r < 16; ++r) dq[db][r] = dqc[db][r] = 0.f;
 
   const int kend = min(q0 + BW_TILE, a.lk);
   const int n_kt = (kend + BN - 1) / BN;
-  RowStage<HD, BN, true> sk;
-  sk.init(a.ldk);
-  sk.load(kbase, a.ldk, 0, a.lk, HD);
-  sk.store(Ks[0]);
+  Stage sk;
+  sk.init();
+  sk.load(kbase, a.ldk, 0, a.lk);
+  sk.store(lds[0]);
   // dS operands two blocks ahead: cur (block j), n1 (j + 1), n2 (j + 2)
   vf4 cur[4], n1[4], n2[4];
   if (last >= 0) {
@@ -672,10 +1088,11 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
   }
   __syncthreads();
 
+  const int ko = Stage::operand(li, hf);
   for (int kt = 0; kt < n_kt; ++kt) {
     const int lbuf = kt & 1;
     const int k0 = kt * BN;
-    sk.load(kbase, a.ldk, kt + 1 < n_kt ? k0 + BN : k0, a.lk, HD);
+    sk.load(kbase, a.ldk, kt + 1 < n_kt ? k0 + BN : k0, a.lk);
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
       const int j = kt * NKB + kb;  // key block
@@ -684,12 +1101,26 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
 #pragma unroll
         for (int i = 0; i < 4; ++i) n2[i] = *reinterpret_cast<const vf4 *>(dsw + (size_t)(j + 2) * 1024 + 4 * i);
       }
-      const float(*krow)[HD + 4] = &Ks[lbuf][kb * 32];
 #pragma unroll
-      for (int st = 0; st < 16; ++st) {
-        const float av = cur[st >> 2][st & 3];
+      for (int st = 0; st < 2; ++st) {
+        float x[8];
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) dq[db] = mfma32x32x2(av, krow[2 * st + hf][db * 32 + li], dq[db]);
+        for (int e = 0; e < 8; ++e) x[e] = cur[2 * st + (e >> 2)][e & 3];
+        bf16x8 ds[3];
+        split_operand(x, ds);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+          bf16x8 k[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            k[p] = *reinterpret_cast<const bf16x8 *>(lds[lbuf] + ko + p * Stage::PLANE + (2 * kb + st) * Stage::SLAB +
+                                                     db * 256);
+#pragma unroll
+          for (int i = 0; i < kSplitProducts; ++i) {
+            floatx16 &c = i == kSplitMain ? dq[db] : dqc[db];
+            c = mfma32x32x16(k[kSplitA[i]], ds[kSplitB[i]], c);
+          }
+        }
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -697,102 +1128,36 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
         n1[i] = n2[i];
       }
     }
-    sk.store(Ks[lbuf ^ 1]);
+    sk.store(lds[lbuf ^ 1]);
     __syncthreads();
   }
 
+  float bad = 0.f;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int q = qw0 + acc_row(r) + 4 * hf;
-    if (q < a.lq) {
-      float *dqrow = a.dq + ((size_t)b * a.lq + q) * a.lddq + col0;
+  for (int db = 0; db < NDB; ++db) {
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) dqrow[db * 32 + li] = dq[db][r] * a.scale;
-    }
+    for (int r = 0; r < 16; ++r) dq[db][r] += dqc[db][r];
+    bad = nonfinite_sum(dq[db], bad);
   }
-}
-
-// dQ from the stored dS blocks for short sequences (lq <= 32 * MAXQB): one
-// workgroup per (sequence, head) stages the head's whole K in LDS once; wave
-// w owns query blocks w and nqb - 1 - w, so every wave has nqb + 1 key
-// blocks of work (the middle block of an odd count alone) and no barrier
-// follows the staging.  Operand order and the per-block product are those
-// of flash_bwd_dq_ds_kernel, with the dS operands four blocks ahead (a block
-// is about a thousand MFMA cycles at head dim 32, short of the load latency).
-template <int HD, int MAXQB>
-__global__ void __launch_bounds__(64 * (MAXQB / 2)) flash_bwd_dq_ds_short_kernel(const BwdArgs a) {
-  constexpr int NDB = HD / 32;
-  __shared__ __attribute__((aligned(16))) float Ks[32 * MAXQB][HD + 4];
-  const int bh = blockIdx.x;
-  const int b = bh / a.heads, h = bh % a.heads;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int li = lane & 31, hf = lane >> 5;
-  const int nqb = (a.lq + 31) >> 5;
-  const int col0 = h * HD;
-  // K rows [0, 32 nqb) of the head, rows past lk clamped (their dS is 0)
-  {
-    const float *kbase = a.k + (size_t)b * a.lk * a.ldk + col0;
-    constexpr int F4 = HD / 4;
-    for (int e = t; e < 32 * nqb * F4; e += blockDim.x) {
-      const int r = e / F4, c = (e % F4) * 4;
-      *reinterpret_cast<vf4 *>(&Ks[r][c]) =
-          *reinterpret_cast<const vf4 *>(kbase + (size_t)min(r, a.lk - 1) * a.ldk + c);
-    }
-  }
-  __syncthreads();
-  const float *__restrict__ dsbh = a.ds + (size_t)bh * a.ds_bh + li * 32 + hf * 16;
-  for (int pass = 0; pass < 2; ++pass) {
-    const int qi = pass == 0 ? nqb - 1 - wave : wave;
-    if (pass == 1 && qi >= nqb - 1 - wave) break;  // the middle block ran in pass 0
-    const float *dsw = dsbh + (size_t)qi * (qi + 1) / 2 * 1024;
-    floatx16 dq[NDB];
+  if (any_nonfinite(bad)) {  // on the fp32 MFMA straight from memory (see the dK/dV kernel)
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
-    // dS operands PF blocks ahead in a ring: block j lives in buf[j % PF]
-    // (the loop is unrolled by PF, so every index is a constant and no
-    // in-flight load is ever copied), and the load of block j + PF goes into
-    // the buffer block j has just left.
-    constexpr int PF = 4;
-    vf4 buf[PF][4];
+#pragma unroll 1
+    for (int j = 0; j <= last; ++j)
+#pragma unroll 1
+      for (int s = 0; s < 16; ++s) {
+        const float x = dsw[(size_t)j * 1024 + s];
+        const float *krow = kbase + (size_t)min(32 * j + 2 * s + hf, a.lk - 1) * a.ldk;
 #pragma unroll
-    for (int p = 0; p < PF; ++p)
-      if (p <= qi) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) buf[p][i] = *reinterpret_cast<const vf4 *>(dsw + (size_t)p * 1024 + 4 * i);
+        for (int db = 0; db < NDB; ++db) dq[db] = mfma32x32x2(krow[db * 32 + li], x, dq[db]);
       }
-    for (int j0 = 0; j0 <= qi; j0 += PF) {
-#pragma unroll
-      for (int u = 0; u < PF; ++u) {
-        const int j = j0 + u;
-        if (j > qi) break;
-        const float(*krow)[HD + 4] = &Ks[j * 32];
-#pragma unroll
-        for (int st = 0; st < 16; ++st) {
-          const float av = buf[u][st >> 2][st & 3];
-#pragma unroll
-          for (int db = 0; db < NDB; ++db) dq[db] = mfma32x32x2(av, krow[2 * st + hf][db * 32 + li], dq[db]);
-        }
-        if (j + PF <= qi) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            buf[u][i] = *reinterpret_cast<const vf4 *>(dsw + (size_t)(j + PF) * 1024 + 4 * i);
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int q = qi * 32 + acc_row(r) + 4 * hf;
-      if (q < a.lq) {
-        float *dqrow = a.dq + ((size_t)b * a.lq + q) * a.lddq + col0;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) dqrow[db * 32 + li] = dq[db][r] * a.scale;
-      }
-    }
   }
+  const int qrow = qw0 + li;
+  if (qrow < a.lq)
+    store_column<HD, true>(a, dq, a.dq + ((size_t)b * a.lq + qrow) * a.lddq + col0, a.scale,
+                          a.rope_cs ? a.rope_cs + (size_t)qrow * (a.hd >> 1) : nullptr, hf);
 }
 
 // Any head dim, any strides: one workgroup per (sequence, head) walks the
@@ -911,44 +1276,44 @@ int zero_rows(float *p, long long rows, int cols, int ld, hipStream_t st) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-// Returns whether dQ left rotated (a.rope_cs set and a dQ kernel that
-// applies it: the stored-dS dQ kernels do not, their 16 rows per lane would
-// cost the table registers they need for their occupancy).
 template <int HD, int BQ, int BN, bool CAUSAL, bool HAS_MASK, bool VEC>
-bool launch_bwd(BwdArgs &a, hipStream_t st) {
+void launch_bwd(BwdArgs &a, hipStream_t st) {
   const int n_bh = a.batch * a.heads;
   const int kt = (a.lk + BW_TILE - 1) / BW_TILE;
   a.n_tiles = (a.lq + BW_TILE - 1) / BW_TILE;
-  if constexpr (CAUSAL && !HAS_MASK && VEC && HD <= 64) {
-    if (a.ds) {  // dQ from the stored dS blocks
-      flash_bwd_dkdv_kernel<HD, BQ, true, false, true, true><<<dim3(n_bh * kt), dim3(BW_THREADS), 0, st>>>(a);
-      constexpr int kShortQB = HD <= 32 ? 16 : 8;  // the whole K of a head in LDS: 72 KB at most
-      const int nqb = (a.lq + 31) / 32;
-      if (nqb <= kShortQB)
-        flash_bwd_dq_ds_short_kernel<HD, kShortQB><<<dim3(n_bh), dim3(64 * ((nqb + 1) / 2)), 0, st>>>(a);
-      else
-        flash_bwd_dq_ds_kernel<HD, 64><<<dim3(n_bh * a.n_tiles), dim3(BW_THREADS), 0, st>>>(a);
-      return false;
+  const dim3 kgrid(n_bh * kt), qgrid(n_bh * a.n_tiles), block(BW_THREADS);
+  if constexpr (HD <= 64) {
+    const dim3 kblock(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS);
+    if constexpr (CAUSAL && !HAS_MASK && VEC) {
+      if (a.ds) {  // dQ from the stored dS blocks
+        flash_bwd_dkdv_split_kernel<HD, true, false, true, true><<<kgrid, kblock, 0, st>>>(a);
+        flash_bwd_dq_ds_kernel<HD, 64><<<qgrid, block, 0, st>>>(a);
+        return;
+      }
     }
+    flash_bwd_dkdv_split_kernel<HD, CAUSAL, HAS_MASK, VEC, false><<<kgrid, kblock, 0, st>>>(a);
+  } else {
+    flash_bwd_dkdv_kernel<HD, BQ, CAUSAL, HAS_MASK, VEC><<<kgrid, block, 0, st>>>(a);
   }
-  flash_bwd_dkdv_kernel<HD, BQ, CAUSAL, HAS_MASK, VEC, false><<<dim3(n_bh * kt), dim3(BW_THREADS), 0, st>>>(a);
-  flash_bwd_dq_kernel<HD, BN, CAUSAL, HAS_MASK, VEC><<<dim3(n_bh * a.n_tiles), dim3(BW_THREADS), 0, st>>>(a);
-  return a.rope_cs != nullptr;
+  flash_bwd_dq_kernel<HD, BN, CAUSAL, HAS_MASK, VEC><<<qgrid, block, 0, st>>>(a);
 }
 
 template <int HD, int BQ, int BN, bool VEC>
-bool launch_bwd_mode(BwdArgs &a, bool causal, hipStream_t st) {
+void launch_bwd_mode(BwdArgs &a, bool causal, hipStream_t st) {
   if (causal) {
-    if (a.mask) return launch_bwd<HD, BQ, BN, true, true, VEC>(a, st);
-    return launch_bwd<HD, BQ, BN, true, false, VEC>(a, st);
+    if (a.mask) launch_bwd<HD, BQ, BN, true, true, VEC>(a, st);
+    else launch_bwd<HD, BQ, BN, true, false, VEC>(a, st);
+  } else if (a.mask) {
+    launch_bwd<HD, BQ, BN, false, true, VEC>(a, st);
+  } else {
+    launch_bwd<HD, BQ, BN, false, false, VEC>(a, st);
   }
-  if (a.mask) return launch_bwd<HD, BQ, BN, false, true, VEC>(a, st);
-  return launch_bwd<HD, BQ, BN, false, false, VEC>(a, st);
 }
 
 template <int HD, int BQ, int BN>
-bool launch_bwd_hd(BwdArgs &a, bool causal, bool vec, hipStream_t st) {
-  return vec ? launch_bwd_mode<HD, BQ, BN, true>(a, causal, st) : launch_bwd_mode<HD, BQ, BN, false>(a, causal, st);
+void launch_bwd_hd(BwdArgs &a, bool causal, bool vec, hipStream_t st) {
+  if (vec) launch_bwd_mode<HD, BQ, BN, true>(a, causal, st);
+  else launch_bwd_mode<HD, BQ, BN, false>(a, causal, st);
 }
 
 }  // namespace
@@ -1011,7 +1376,7 @@ int sdpa_bwd_impl(const float *q, int ldq, const float *k, int ldk, const float 
                   int lddo, float *dq, int lddq, float *dk, int lddk, float *dv, int lddv, int batch,
                   int lq, int lk, int dim, int num_heads, float scale, int causal,
                   const uint8_t *mask, void *workspace, size_t workspace_bytes, cdml_stream stream,
-                  const char *what, const float *rope_cs = nullptr, int rope_npos = 0) {
+                  const char *what, const float *rope_cs = nullptr) {
   const bool saved = o_saved != nullptr;
   size_t need = 0;
   int rc = cdml_sdpa_bwd_workspace_size(batch, lq, lk, dim, num_heads, &need);
@@ -1130,14 +1495,10 @@ int sdpa_bwd_impl(const float *q, int ldq, const float *k, int ldk, const float 
       a.ds_bh = (long long)(extra / sizeof(float) / bh);
     }
   }
-  bool dq_rotated;
-  if (hd_pad == 32) dq_rotated = launch_bwd_hd<32, 64, 64>(a, causal != 0, vec, st);
-  else if (hd_pad == 64) dq_rotated = launch_bwd_hd<64, 64, 32>(a, causal != 0, vec, st);
-  else dq_rotated = launch_bwd_hd<128, 32, 32>(a, causal != 0, vec, st);
-  rc = check_launch("flash_bwd_dkdv_kernel / flash_bwd_dq_kernel");
-  if (rc || !rope_cs || dq_rotated) return rc;
-  // dK left rotated; dQ from the stored dS blocks takes the table RoPE
-  return cdml_rope_qk_table(dq, nullptr, batch * lq, lddq, hd, num_heads, rope_cs, rope_npos, 0, lq, 1, stream);
+  if (hd_pad == 32) launch_bwd_hd<32, 64, 64>(a, causal != 0, vec, st);
+  else if (hd_pad == 64) launch_bwd_hd<64, 64, 32>(a, causal != 0, vec, st);
+  else launch_bwd_hd<128, 32, 32>(a, causal != 0, vec, st);
+  return check_launch("flash_bwd_dkdv_kernel / flash_bwd_dq_kernel");
 }
 
 }  // namespace
@@ -1183,5 +1544,5 @@ extern "C" int cdml_sdpa_bwd_saved_rope(const float *q, int ldq, const float *k,
     return fail(CDML_E_INVALID, "%s: a %d-row table does not cover %d positions", what, n_pos, std::max(lq, lk));
   return sdpa_bwd_impl(q, ldq, k, ldk, v, ldv, o, ldo, lse, dout, lddo, dq, lddq, dk, lddk, dv, lddv,
                        batch, lq, lk, dim, num_heads, scale, causal, mask, workspace, workspace_bytes,
-                       stream, what, rope_cs, n_pos);
+                       stream, what, rope_cs);
 }

@@ -144,7 +144,7 @@ int cdml_memcpy2d_d2d_async(void *dst, size_t dpitch, const void *src,
  * GPU/TransformerCore.cs:1386-1464,1629-1665:
  *   q = x wq^T + bq,  k = x wk^T + bk,  v = x wv^T + bv
  * x [rows, in_dim]; w* [out_dim, in_dim]; b* [out_dim] (NULL = zero bias);
- * q, k, v [rows, out_dim], contiguous.  One launch, fp32 MFMA. */
+ * q, k, v [rows, out_dim], contiguous.  One launch. */
 int cdml_project_qkv(const float *x, const float *wq, const float *bq,
                      const float *wk, const float *bk, const float *wv,
                      const float *bv, float *q, float *k, float *v, int rows,
@@ -156,7 +156,10 @@ int cdml_project_qkv(const float *x, const float *wq, const float *bq,
  * AccelerationCPU.cs:2694-2715 and :342-404:
  *   y = act(x w^T + b)
  * x [rows, in_dim] with row stride ldx; w [out_dim, in_dim]; b [out_dim] or
- * NULL; y [rows, out_dim] with row stride ldy; activation CDML_ACT_*. */
+ * NULL; y [rows, out_dim] with row stride ldy; activation CDML_ACT_*.
+ * Matrix products here and below take fp32 operands as three bf16 pieces each
+ * (24 bits, exact) and sum six products in fp32, at no larger error than fp32
+ * sums; infinities, NaNs and overflows come out as in fp32. */
 int cdml_linear(const float *x, int ldx, const float *w, const float *b,
                 float *y, int ldy, int rows, int in_dim, int out_dim,
                 int activation, cdml_stream stream);
@@ -164,7 +167,8 @@ int cdml_linear(const float *x, int ldx, const float *w, const float *b,
 /* IAccelerationManager.MatrixMultiply (:20), replacing AccelerationCPU.cs:
  * 159-214 (the FFN backward's hidden deltas and input gradient,
  * NeuralNetwork.cs:861-881): c = a b with a [m, k] (row stride lda), b
- * [k, n] (row stride ldb), c [m, n] (row stride ldc); fp32 MFMA.
+ * [k, n] (row stride ldb), c [m, n] (row stride ldc); fp32
+ * results from bf16 pieces of the fp32 operands (see cdml_linear).
  * MatrixMultiplyTranspose (:26, a b^T) is cdml_linear with b as the weight
  * and no bias. */
 int cdml_matmul(const float *a, int lda, const float *b, int ldb, float *c,
@@ -178,7 +182,7 @@ int cdml_matmul(const float *a, int lda, const float *b, int ldb, float *c,
  * accumulate; dx [rows, in_dim] (row stride lddx) is overwritten
  * (accumulate_dx = 0, BackpropOutputProjection) or added to (1,
  * BackpropLinearProjection).  dx = NULL skips the input gradient; wgrad and
- * bgrad may be NULL to skip theirs.  fp32 MFMA; the bias gradient is summed
+ * bgrad may be NULL to skip theirs.  The bias gradient is summed
  * inside the weight-gradient GEMM.  When the weight gradient has too few
  * output tiles to fill the device (rows >> in_dim * out_dim / 2^15), its
  * reduction over rows is split into chunks whose partial sums go to
@@ -322,7 +326,7 @@ int cdml_mha_layer_fwd(const float *x, const float *wq, const float *bq,
  * (the bool[,] overload).  scale is used as passed (the attention scores are
  * q.k * scale).  A query with no visible key contributes nothing.
  * `workspace`: device memory of cdml_sdpa_bwd_workspace_size() bytes.  Head
- * dims up to 128 run on fp32 MFMA (a forward pass with row statistics, then
+ * dims up to 128 run on the matrix cores (a forward pass with row statistics, then
  * dK/dV and dQ kernels, no atomics; head dims other than 32, 64 and 128, and
  * rows that are not 16-byte aligned, take zero-padded scalar loads); larger
  * head dims run a per-row kernel. */
@@ -371,9 +375,8 @@ int cdml_sdpa_bwd_saved(const float *q, int ldq, const float *k, int ldk,
  * input gradients (TransformerTrainer.cs:978-985, the inverse of the rotation
  * at :811-848): every head of a row at the row's index within its sequence
  * (dQ rows modulo lq, dK rows modulo lk), with rope_cs a cdml_rope_table of
- * n_pos >= max(lq, lk) positions for the head dim (8-byte aligned).  dK, and
- * dQ where it is recomputed, are rotated as the kernels store them; dQ from
- * stored dS blocks takes one table-RoPE launch on dQ alone.  With lq == lk
+ * n_pos >= max(lq, lk) positions for the head dim (8-byte aligned).  dQ
+ * and dK are rotated as the kernels store them.  With lq == lk
  * (the trainer's causal self-attention) the bits are those of
  * cdml_sdpa_bwd_saved then cdml_rope_qk_table(dq, dk, ..., pos_offset 0,
  * seg_len lq, inverse 1) on the same rows.  Same workspace as
@@ -404,7 +407,7 @@ int cdml_linear_preact(const float *x, int ldx, const float *w, const float *b,
                        int out_dim, int activation, cdml_stream stream);
 
 /* One layer of NeuralNetwork.ComputeInputGradientBatch (NeuralNetwork.cs:
- * 841-881) on fp32 MFMA, with cdml_linear_backward's gradients:
+ * 841-881), with cdml_linear_backward's gradients:
  *   wgrad += dy^T x,  bgrad += column sums of dy,
  *   dx = (dy w) * act'(dz) + add
  * dz (the layer below's pre-activation, for its hidden deltas) and add (a

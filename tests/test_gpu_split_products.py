@@ -130,3 +130,109 @@ def test_attention_values_outside_the_split(hd):
     v[5, 1] = np.inf  # every row sees it without the causal rule
     got = G.sdpa(q, k, v, heads, scale=1.0 / np.sqrt(hd))
     check_attention(got, q, k, v, heads, 1.0 / np.sqrt(hd), False, f"hd {hd} infinite value")
+
+
+def backward(q, k, v, dout, heads, scale, causal, mask=None, stored=False):
+    """cdml_sdpa_bwd; stored: with the workspace that lets the dK/dV pass store dS."""
+    L, D = q.shape
+    bufs = [G.up(t) for t in (q, k, v, dout)]
+    grads = [G.N.DeviceBuffer(L * D * 4) for _ in range(3)]
+    bm = G.up(mask, np.uint8) if mask is not None else None
+    n = G.C.c_size_t(0)
+    if stored:
+        G.N.check(G.N.lib().cdml_sdpa_bwd_stored_ds_workspace_size(1, L, L, D, heads, int(causal), G.C.byref(n)))
+    else:
+        G.N.check(G.N.lib().cdml_sdpa_bwd_workspace_size(1, L, L, D, heads, G.C.byref(n)))
+    ws = G.N.DeviceBuffer(max(256, n.value))
+    ins = [x for b in bufs for x in (b.ptr, D)]
+    outs = [x for g in grads for x in (g.ptr, D)]
+    G.N.check(G.N.lib().cdml_sdpa_bwd(*ins, *outs, 1, L, L, D, heads, scale, int(causal), bm.ptr if bm else None,
+                                      ws.ptr, n.value, G.stream().handle))
+    return [G.down(g, (L, D)) for g in grads]
+
+
+def weighted(p, x):
+    """p @ x in which a weight of 0 leaves a term out, an infinite one too."""
+    out = p @ np.where(np.isfinite(x), x, 0.0)
+    for i, c in np.argwhere(~np.isfinite(x)):
+        out[p[:, i] != 0, c] += p[p[:, i] != 0, i] * x[i, c]
+    return out
+
+
+def backward64(q, k, v, dout, heads, scale, allowed, per=8):
+    """(gradient, its error bound) of dQ, dK and dV in float64, u = 2^-24.  A probability is off by (2 (hd / 8 + 8) m +
+    L / 8 + 32) u relatively (check_attention), dP by (hd / 8 + 8) u sum |dO| |V|, D by the output's error and
+    its own sum's, (hd / 8 + 8) u sum |dO| |O|; products of these with the last operand add (L / 8 + 8) u.
+    per: products that one rounding adds, 8 above; the fp32 MFMA adds 2."""
+    L, D = q.shape
+    hd, u = D // heads, 2.0 ** -24
+    out = [(np.empty((L, D)), np.empty((L, D))) for _ in range(3)]
+    for h in range(heads):
+        c = slice(h * hd, (h + 1) * hd)
+        Q, K, V, G_ = (t[:, c].astype(np.float64) for t in (q, k, v, dout))
+        with np.errstate(all="ignore"):
+            s = np.where(allowed, Q @ K.T * scale, -np.inf)
+            m = np.max(np.where(allowed, np.abs(Q) @ np.abs(K).T * scale, 0.0), 1, keepdims=True)
+            p = np.exp(s - s.max(1, keepdims=True))
+            p /= p.sum(1, keepdims=True)
+            o, dp = p @ V, G_ @ V.T
+            d = (G_ * o).sum(1, keepdims=True)
+            ds = np.where(p > 0, p * (dp - d), 0.0)
+            ep = (2 * (hd / per + 8) * m + L / per + 32) * u
+            edp = (hd / per + 8) * u * (np.abs(G_) @ np.abs(V).T)
+            ed = (np.abs(G_) * (ep * (p @ np.abs(V)) + (hd / per + 8) * u * np.abs(o))).sum(1, keepdims=True)
+            eds = np.where(p > 0, p * (ep * np.abs(dp - d) + edp + ed + 4 * u * (np.abs(dp) + np.abs(d))), 0.0)
+            sum_u = (L / per + 8) * u
+            out[0][0][:, c], out[0][1][:, c] = ds @ K * scale, (eds + sum_u * np.abs(ds)) @ np.abs(K) * scale
+            out[1][0][:, c], out[1][1][:, c] = ds.T @ Q * scale, (eds + sum_u * np.abs(ds)).T @ np.abs(Q) * scale
+            out[2][0][:, c], out[2][1][:, c] = weighted(p.T, G_), weighted((p * (ep + sum_u)).T, np.abs(G_))
+    return out
+
+
+def check_backward(got, want, what):
+    for g, (w, bound), name in zip(got, want, ("dQ", "dK", "dV")):
+        assert np.array_equal(np.isnan(g), np.isnan(w)), f"{what} {name}: NaNs elsewhere"
+        inf = np.isinf(w)
+        assert np.array_equal(g[inf], w[inf]), f"{what} {name}: infinities"
+        fine = np.isfinite(w)
+        # values under the smallest normal float may be flushed
+        with np.errstate(invalid="ignore"):
+            over = np.abs(g.astype(np.float64) - np.where(fine, w, 0.0)) - bound - 2.0 ** -126
+        assert np.all(over[fine] <= 0), f"{what} {name}: {np.max(over[fine]):.3g} over the bound"
+
+
+# lengths around the 32-query tiles, a wave's 32 and a workgroup's 128 keys; head dim 32 runs one wave per key block,
+# 64 two, 20 and 40 their scalar loads
+@pytest.mark.parametrize("L", [1, 31, 33, 97, 129, 300])
+@pytest.mark.parametrize("hd", [20, 32, 40, 64])
+def test_attention_backward(hd, L):
+    heads, scale = 2, 1.0 / np.sqrt(hd)
+    q, k, v, dout = (synth.normal(i, (L, heads * hd)) for i in (1, 2, 3, 4))
+    q = q * np.float32(2.0)
+    tril, full = np.tril(np.ones((L, L), bool)), np.ones((L, L), bool)
+    drop = synth.uniform(9, L * L).reshape(L, L) < 0.7
+    drop[:, 0] = True  # every query sees a key
+    for causal, mask in ((False, None), (True, None), (False, drop), (True, drop)):
+        allowed = (tril if causal else full) & (drop if mask is not None else full)
+        want = backward64(q, k, v, dout, heads, scale, allowed)
+        what = f"hd {hd} L {L} causal {causal} mask {mask is not None}"
+        check_backward(backward(q, k, v, dout, heads, scale, causal, mask), want, what)
+        if causal and mask is None:
+            check_backward(backward(q, k, v, dout, heads, scale, causal, stored=True), want, what + " stored dS")
+
+
+@pytest.mark.parametrize("hd", [32, 64])
+def test_attention_backward_values_outside_the_split(hd):
+    """An infinite and a huge output gradient: the keys they reach get what the fp32 products give, the others
+    their values."""
+    L, heads, scale = 130, 2, 1.0 / np.sqrt(hd)
+    q, k, v, dout = (synth.normal(i, (L, heads * hd)) for i in (1, 2, 3, 4))
+    # Query 31 sees all of the first 32 keys, in the first head.  (A masked pair of the same 32 x 32 block has weight
+    # 0, and 0 * inf is a NaN in fp32 too.)
+    dout[31, 3] = np.inf
+    dout[70, hd + 5] = 3.4e38  # above the largest bf16
+    v[:, hd + 5] *= np.float32(1e-30)
+    tril = np.tril(np.ones((L, L), bool))
+    want = backward64(q, k, v, dout, heads, scale, tril, per=2)  # what they reach is summed on the fp32 MFMA
+    for stored in (False, True):
+        check_backward(backward(q, k, v, dout, heads, scale, True, stored=stored), want, f"hd {hd} stored {stored}")
