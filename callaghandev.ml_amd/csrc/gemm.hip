@@ -1097,11 +1097,16 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArg
 // with the tree's additions.
 // Measured on MI355X: a decoder layer's step for 8 sequences (D 1024, FF 4096,
 // 2048 keys, 12.6 M weights) took 133.7 us with one float4 of each column in
-// flight, a branch per row and one pair per wave throughout, and takes 87.1 us.
+// flight, a branch per row and one pair per wave throughout, and takes 82.1 us.
 template <int MR, int KS, bool EPI>
 __global__ void __launch_bounds__(256) gemm_rows_kernel(const GemmArgs args) {
   static_assert(KS == 1 || KS == 4, "waves per column pair");
   constexpr int U = 4;  // steps whose W loads are in flight together
+  // x of the next step is loaded before this one's products: us without / with
+  // at KS = 1, 8 rows, 1024 -> 4096 9.3 / 7.5, 1024 -> 16384 24.1 / 21.1; one row
+  // gains nothing (4096 -> 2040 8.0 / 9.2), and at KS = 4 the registers cost more
+  // where K is short (1024 -> 1536 5.2 / 6.5).
+  constexpr bool AHEAD = KS == 1 && (MR == 4 || MR == 8);
   const int prob = blockIdx.y;
   const GemmProblem P = args.p[prob];
   const int M = args.M, N = args.N, K = args.K;
@@ -1118,12 +1123,15 @@ __global__ void __launch_bounds__(256) gemm_rows_kernel(const GemmArgs args) {
   float s[2 * MR];  // (row m, column n0 + c) at 2 m + c
 #pragma unroll
   for (int i = 0; i < 2 * MR; ++i) s[i] = 0.f;
-  auto step = [&](int k, const float4 &a, const float4 &b) {
+  auto load_x = [&](int k, float4 (&v)[MR]) {
+#pragma unroll
+    for (int m = 0; m < MR; ++m) v[m] = *reinterpret_cast<const float4 *>(x[m] + k);
+  };
+  auto step = [&](const float4 (&v)[MR], const float4 &a, const float4 &b) {
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
-      const float4 v = *reinterpret_cast<const float4 *>(x[m] + k);
-      s[2 * m] += (v.x * a.x + v.y * a.y) + (v.z * a.z + v.w * a.w);
-      s[2 * m + 1] += (v.x * b.x + v.y * b.y) + (v.z * b.z + v.w * b.w);
+      s[2 * m] += (v[m].x * a.x + v[m].y * a.y) + (v[m].z * a.z + v[m].w * a.w);
+      s[2 * m + 1] += (v[m].x * b.x + v[m].y * b.y) + (v[m].z * b.z + v[m].w * b.w);
     }
   };
   constexpr int KSTEP = 256 * KS;
@@ -1135,11 +1143,24 @@ __global__ void __launch_bounds__(256) gemm_rows_kernel(const GemmArgs args) {
       a[u] = *reinterpret_cast<const float4 *>(w0 + kb + u * KSTEP + 4 * lane);
       b[u] = *reinterpret_cast<const float4 *>(w1 + kb + u * KSTEP + 4 * lane);
     }
+    float4 v[AHEAD ? 2 : 1][MR];
+    if (AHEAD) load_x(kb + 4 * lane, v[0]);
 #pragma unroll
-    for (int u = 0; u < U; ++u) step(kb + u * KSTEP + 4 * lane, a[u], b[u]);
+    for (int u = 0; u < U; ++u) {
+      if (!AHEAD) {
+        load_x(kb + u * KSTEP + 4 * lane, v[0]);
+      } else {
+        if (u + 1 < U) load_x(kb + (u + 1) * KSTEP + 4 * lane, v[(u + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);  // keeps them ahead of this step's products
+      }
+      step(v[AHEAD ? u & 1 : 0], a[u], b[u]);
+    }
   }
-  for (int k = kb + 4 * lane; k < K; k += KSTEP)
-    step(k, *reinterpret_cast<const float4 *>(w0 + k), *reinterpret_cast<const float4 *>(w1 + k));
+  for (int k = kb + 4 * lane; k < K; k += KSTEP) {
+    float4 v[MR];
+    load_x(k, v);
+    step(v, *reinterpret_cast<const float4 *>(w0 + k), *reinterpret_cast<const float4 *>(w1 + k));
+  }
   // After the halving steps, lane l holds value l / (32 / MR).
 #pragma unroll
   for (int half = MR, off = 32; off > 0; off >>= 1, half >>= 1) {
@@ -1666,11 +1687,14 @@ int launch_any(GemmArgs &g, hipStream_t stream) {
 }
 
 // The four waves of a workgroup share a column pair (KS = 4) where one pair per
-// wave would give fewer workgroups than CUs and K has more than one step.
+// wave would give workgroups to fewer than three CUs in four and K has more than
+// one step.  us with KS = 1 / 4, 8 rows: 1024 -> 1024 5.3 / 4.9, 4096 -> 1024
+// 11.8 / 9.6, 512 -> 512 4.6 / 4.2; from 1536 outputs on (192 workgroups of 256
+// CUs) 1024 -> 1536 5.2 / 5.2, 1024 -> 2040 5.3 / 5.8, 4096 -> 2040 13.2 / 14.7.
 template <int MR>
 void launch_rows(const GemmArgs &g, hipStream_t stream) {
   const int pairs = (g.N + 1) / 2, wgs = (pairs + 3) / 4;
-  const bool epi = has_epi(g), split = (long long)wgs * g.nprob < num_cus() && g.K > 256;
+  const bool epi = has_epi(g), split = 4LL * wgs * g.nprob < 3 * num_cus() && g.K > 256;
   const dim3 grid((unsigned)(split ? pairs : wgs), (unsigned)g.nprob), block(256);
   if (split)
     epi ? gemm_rows_kernel<MR, 4, true><<<grid, block, 0, stream>>>(g)
