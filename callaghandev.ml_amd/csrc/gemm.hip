@@ -986,24 +986,27 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
 // offsets below 2^32), for the pre-activations of ReLU and leaky ReLU layers
 // that train (GemmArgs::f32): the sign of z picks the derivative, so a z within
 // rounding of 0 moves a whole row of the layer below's gradient by up to a
-// tenth of its rms when its last bits change; these products keep the bits they
-// have always had.  fp32-equivalent 116-138 TFLOP/s against the split kernel's
-// 160-199.
+// tenth of its rms when its last bits change; above 16 rows these products keep
+// the bits they have always had.  fp32-equivalent TFLOP/s with z / without:
+// 130816 x 256 -> 1024 112 / 124, 16380 x 1024 -> 4096 136 / 137 (the split
+// kernel has 160-199).
 //
 // Both operand tiles sit in LDS as [rows][16] with pitch 20 floats, double
 // buffered; lanes read 16-byte operands that feed four v_mfma_f32_32x32x2_f32
-// each, so k is visited in the order 8 (s / 4) + 4 h + s % 4.  The rows of a
-// wave's 16 are stored in the order 0, 4, 8, 12, 1, 5, ..., whose 64-byte
-// pieces fall in disjoint banks.
-template <int TM, int TN, int WM, int WN>
+// each, so k is visited in the order 8 (s / 4) + 4 h + s % 4.  The operands of
+// the second half of a k-tile are read while the MFMAs of the first run.  The
+// rows of a wave's 16 are stored in the order 0, 4, 8, 12, 1, 5, ..., whose
+// 64-byte pieces fall in disjoint banks.  The activation is a template argument
+// and the epilogue stores from the accumulators: with a run-time activation
+// behind store_tile, and without the read-ahead, the kernel took 696 instead of
+// 552 us for 130816 x 256 -> 1024 and 92 instead of 79 us for 16384 x 512 -> 512.
+template <int TM, int TN, int WM, int WN, int ACT, bool EPI>
 __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArgs args) {
   constexpr int NT = 64 * WM * WN, BKK = 16, LD = BKK + 4;
   constexpr int BI = TM / WM / 32, BJ = TN / WN / 32;
   constexpr int RPP = NT / 4, NA = TM / RPP, NB = TN / RPP;
-  constexpr int TILES = 2 * (TM + TN) * LD, BANDS = WM * WN * 32 * (32 * BJ + 4);
-  __shared__ __attribute__((aligned(16))) float smem[TILES > BANDS ? TILES : BANDS];
-  float(*const As)[LD] = reinterpret_cast<float(*)[LD]>(smem);  // buffer b: rows [b TM, (b + 1) TM)
-  float(*const Bs)[LD] = reinterpret_cast<float(*)[LD]>(smem + 2 * TM * LD);
+  __shared__ __attribute__((aligned(16))) float As[2][TM][LD];
+  __shared__ __attribute__((aligned(16))) float Bs[2][TN][LD];
 
   const int lid = xcd_remap(blockIdx.x, args.padded);
   if (lid >= args.total) return;
@@ -1014,6 +1017,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArg
   const int tm = first_m + (lid % in_group) % gsize;
   const int tn = (lid % in_group) / gsize;
   const GemmProblem P = args.p[0];
+  const int M = args.M, N = args.N;
   const int m0 = tm * TM, n0 = tn * TN;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1024,9 +1028,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArg
   uint32_t offa[NA], offb[NB];
   vf4 va[NA], vb[NB];
 #pragma unroll
-  for (int i = 0; i < NA; ++i) offa[i] = (uint32_t)min(m0 + row + RPP * i, args.M - 1) * (uint32_t)args.lda + col;
+  for (int i = 0; i < NA; ++i) offa[i] = (uint32_t)min(m0 + row + RPP * i, M - 1) * (uint32_t)args.lda + col;
 #pragma unroll
-  for (int i = 0; i < NB; ++i) offb[i] = (uint32_t)min(n0 + row + RPP * i, args.N - 1) * (uint32_t)args.ldb + col;
+  for (int i = 0; i < NB; ++i) offb[i] = (uint32_t)min(n0 + row + RPP * i, N - 1) * (uint32_t)args.ldb + col;
   auto load = [&](int kt) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) va[i] = *reinterpret_cast<const vf4 *>(P.a + (size_t)kt * BKK + offa[i]);
@@ -1035,9 +1039,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArg
   };
   auto stage = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) *reinterpret_cast<vf4 *>(&As[buf * TM + row + RPP * i][col]) = va[i];
+    for (int i = 0; i < NA; ++i) *reinterpret_cast<vf4 *>(&As[buf][row + RPP * i][col]) = va[i];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) *reinterpret_cast<vf4 *>(&Bs[buf * TN + row + RPP * i][col]) = vb[i];
+    for (int i = 0; i < NB; ++i) *reinterpret_cast<vf4 *>(&Bs[buf][row + RPP * i][col]) = vb[i];
   };
   floatx16 acc[BI][BJ];
 #pragma unroll
@@ -1051,33 +1055,60 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArg
   stage(0);
   load(min(1, nk - 1));
   __syncthreads();
-#pragma unroll 1
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
-    const float(*as)[LD] = &As[cur * TM + wm * (TM / WM) + li];
-    const float(*bs)[LD] = &Bs[cur * TN + wn * (TN / WN) + li];
+    const float(*as)[LD] = &As[cur][wm * (TM / WM) + li];
+    const float(*bs)[LD] = &Bs[cur][wn * (TN / WN) + li];
+    vf4 a4[2][BI], b4[2][BJ];  // operands of the two halves of the k-tile
+    auto read = [&](int u) {
+#pragma unroll
+      for (int i = 0; i < BI; ++i) a4[u][i] = *reinterpret_cast<const vf4 *>(&as[i * 32][u * 8 + hf * 4]);
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) b4[u][j] = *reinterpret_cast<const vf4 *>(&bs[j * 32][u * 8 + hf * 4]);
+    };
+    read(0);
 #pragma unroll
     for (int u = 0; u < BKK / 8; ++u) {
-      vf4 a4[BI], b4[BJ];
-#pragma unroll
-      for (int i = 0; i < BI; ++i) a4[i] = *reinterpret_cast<const vf4 *>(&as[i * 32][u * 8 + hf * 4]);
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) b4[j] = *reinterpret_cast<const vf4 *>(&bs[j * 32][u * 8 + hf * 4]);
+      if (u == 0) read(1);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int i = 0; i < BI; ++i)
 #pragma unroll
-          for (int j = 0; j < BJ; ++j) acc[i][j] = mfma32x32x2(a4[i][r], b4[j][r], acc[i][j]);
+          for (int j = 0; j < BJ; ++j) acc[i][j] = mfma32x32x2(a4[u][i][r], b4[u][j][r], acc[i][j]);
     }
     // past the end both repeat the last tile into the idle buffer
     stage(cur ^ 1);
     load(min(kt + 2, nk - 1));
     __syncthreads();
   }
-  const TileOut out{P.c, args.ldc, P.bias, args.act, args.beta, false};
-  store_tile<BI, BJ, true, false>(args, out, acc, m0 + wm * (TM / WM), n0 + wn * (TN / WN), lane,
-                                  smem + wave * 32 * (32 * BJ + 4));
+
+  const int mw = m0 + wm * (TM / WM), nw = n0 + wn * (TN / WN);
+  float bias[BJ];
+#pragma unroll
+  for (int j = 0; j < BJ; ++j) {
+    const int n = nw + j * 32 + li;
+    bias[j] = P.bias && n < N ? P.bias[n] : 0.f;
+  }
+  // D[i][j] of a block sits at row 8 (r / 4) + 4 hf + r % 4, column li: 32 lanes
+  // store 32 consecutive columns of one row.  A launch here has no option but
+  // the pre-activation (cdml_linear_preact).
+  const bool whole = mw + TM / WM <= M && nw + TN / WN <= N;  // wave-uniform
+  float *cb = P.c + (size_t)(mw + 4 * hf) * args.ldc + nw + li;
+  float *pb = EPI ? args.pre + (size_t)(mw + 4 * hf) * args.ldpre + nw + li : nullptr;
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int d = i * 32 + 8 * (r >> 2) + (r & 3);
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) {
+        if (!whole && (mw + 4 * hf + d >= M || nw + j * 32 + li >= N)) continue;
+        const float z = acc[i][j][r] + bias[j];
+        if (EPI) pb[(size_t)d * args.ldpre + j * 32] = z;
+        cb[(size_t)d * args.ldc + j * 32] = activate(z, ACT);
+      }
+    }
 }
 
 // Few rows (decode steps, short batches: M <= MR), non-transposed operands,
@@ -1667,7 +1698,14 @@ void launch_f32_tile(GemmArgs &g, hipStream_t stream) {
   g.tiles_n = (g.N + TN - 1) / TN;
   g.total = g.tiles_m * g.tiles_n;
   g.padded = pad_to_xcd(g.total);
-  gemm_f32_kernel<TM, TN, WM, WN><<<dim3(g.padded), dim3(64 * WM * WN), 0, stream>>>(g);
+  const dim3 grid(g.padded), block(64 * WM * WN);
+  const bool relu = g.act != CDML_ACT_LEAKYRELU;
+  if (g.pre)
+    relu ? gemm_f32_kernel<TM, TN, WM, WN, CDML_ACT_RELU, true><<<grid, block, 0, stream>>>(g)
+         : gemm_f32_kernel<TM, TN, WM, WN, CDML_ACT_LEAKYRELU, true><<<grid, block, 0, stream>>>(g);
+  else
+    relu ? gemm_f32_kernel<TM, TN, WM, WN, kActReluMarked, false><<<grid, block, 0, stream>>>(g)
+         : gemm_f32_kernel<TM, TN, WM, WN, CDML_ACT_LEAKYRELU, false><<<grid, block, 0, stream>>>(g);
 }
 void launch_f32(GemmArgs &g, hipStream_t stream) {
   const long long big = (long long)((g.M + 255) / 256) * ((g.N + 127) / 128);
