@@ -988,6 +988,46 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_kernel(const BwdAr
                           a.rope_cs ? a.rope_cs + (size_t)qi * (a.hd >> 1) : nullptr, hf);
 }
 
+// Stores a 32-row block of dQ from accumulators that hold dQ[q][d] with d in the
+// lanes: register r of block db is row q0 + 8 (r / 4) + 4 hf + r % 4, column db * 32
+// + li, so 32 lanes write 128 contiguous bytes (lanes that hold 16 bytes of 32
+// different rows cost the pass 28 us of 320 at 256 x 511, 8 heads of 32).  x is
+// multiplied by scale and rotated back by the rows' pairs of rope_cs when
+// non-NULL; the partner of a column is in the neighbouring lane.
+template <int HD>
+struct RowStore {
+  static constexpr int NDB = HD / 32;
+  float2 cs[NDB][16];  // loaded before any store (a load issued after a store waits for it)
+  __device__ __forceinline__ void load(const BwdArgs &a, int q0, int li, int hf) {
+    if (!a.rope_cs) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float2 *row = a.rope_cs + (size_t)min(q0 + acc_row(r) + 4 * hf, a.lq - 1) * (HD / 2) + (li >> 1);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) cs[db][r] = row[db * 16];
+    }
+  }
+  __device__ __forceinline__ void store(const BwdArgs &a, const floatx16 (&x)[NDB], int b, int q0, int col0, int li,
+                                        int hf) const {
+#pragma clang fp contract(off)
+    float *base = a.dq + ((size_t)b * a.lq + q0) * a.lddq + col0 + li;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = acc_row(r) + 4 * hf;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) {
+        float y = x[db][r] * a.scale;
+        if (a.rope_cs) {  // rope_inverse_pair on (y, partner), in every lane
+          const float z = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y), 0xB1, 0xF, 0xF, false));
+          const float c = cs[db][r].x, s = -cs[db][r].y;
+          y = li & 1 ? z * s + y * c : y * c - z * s;
+        }
+        if (q0 + row < a.lq) base[(size_t)row * a.lddq + db * 32] = y;
+      }
+    }
+  }
+};
+
 // K^T tile of the stored-dS dQ kernel: BN keys of one head as 16-value rows of
 // dims (slab s holds keys 16 s .. 16 s + 15, key k of a slab at place
 // 8 (k % 2) + k / 2, the order of the stored dS operands), split into three bf16
@@ -999,13 +1039,28 @@ struct KtStage {
   static constexpr int SLAB = 4 * (CH * 32) + 256, PLANE = BN / 16 * SLAB, BYTES = 3 * PLANE;
   static_assert(NU >= 1 && CH * (BN / 2) % BW_THREADS == 0 && (BW_THREADS / 8) % CH == 0, "tile units");
   static __device__ __forceinline__ constexpr int cluster(int c) { return c * CH * 32 + (c & 1) * 16 + (c >> 1) * 128; }
+  // Keys row and row + 2 of unit (slab, dim group, sb), its place, and its pieces' stores.
+  static __device__ __forceinline__ int unit_row(int slab, int sb) { return 16 * slab + 4 * (sb >> 1) + (sb & 1); }
+  static __device__ __forceinline__ int unit_dst(int slab, int g, int sb) {
+    return slab * SLAB + g * 32 + ((sb & 1) * 4 + (sb >> 1)) * 4;
+  }
+  static __device__ __forceinline__ void put(char *d, int plane, const vf4 &r0, const vf4 &r1) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint32_t h, m, l;
+      split_bf16x3(r0[c], r1[c], h, m, l);
+      *reinterpret_cast<uint32_t *>(d + cluster(c)) = h;
+      *reinterpret_cast<uint32_t *>(d + cluster(c) + plane) = m;
+      *reinterpret_cast<uint32_t *>(d + cluster(c) + 2 * plane) = l;
+    }
+  }
   vf4 r[NU][2];
   int row, col, dst;
   __device__ __forceinline__ void init() {
     const int t = threadIdx.x, sb = t & 7, g = (t >> 3) % CH, slab = (t >> 3) / CH;
-    row = 16 * slab + 4 * (sb >> 1) + (sb & 1);  // and row + 2
+    row = unit_row(slab, sb);
     col = 4 * g;
-    dst = slab * SLAB + g * 32 + ((sb & 1) * 4 + (sb >> 1)) * 4;
+    dst = unit_dst(slab, g, sb);
   }
   __device__ __forceinline__ void load(const float *__restrict__ base, int ld, int row0, int nrows) {
     const float *tile = base + (size_t)row0 * ld;
@@ -1018,29 +1073,78 @@ struct KtStage {
   }
   __device__ __forceinline__ void store(char *lds) const {
 #pragma unroll
-    for (int i = 0; i < NU; ++i)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        uint32_t h, m, l;
-        split_bf16x3(r[i][0][c], r[i][1][c], h, m, l);
-        char *d = lds + dst + BW_THREADS / 8 / CH * SLAB * i + cluster(c);
-        *reinterpret_cast<uint32_t *>(d) = h;
-        *reinterpret_cast<uint32_t *>(d + PLANE) = m;
-        *reinterpret_cast<uint32_t *>(d + 2 * PLANE) = l;
-      }
+    for (int i = 0; i < NU; ++i) put(lds + dst + BW_THREADS / 8 / CH * SLAB * i, PLANE, r[i][0], r[i][1]);
   }
   static __device__ __forceinline__ int operand(int li, int hf) { return cluster(li & 3) + (li >> 2) * 32 + hf * 16; }
 };
 
+// One 32-key block of dQ = dS K: cur is this lane's dS operand, kt its K^T operand
+// of plane 0, first slab of the block.
+template <int HD>
+__device__ __forceinline__ void dq_block(const vf4 (&cur)[4], const char *kt, int plane, int slab,
+                                         floatx16 (&dq)[HD / 32], floatx16 (&dqc)[HD / 32]) {
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = cur[2 * st + (e >> 2)][e & 3];
+    bf16x8 ds[3];
+    split_operand(x, ds);
+#pragma unroll
+    for (int db = 0; db < HD / 32; ++db) {
+      bf16x8 k[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) k[p] = *reinterpret_cast<const bf16x8 *>(kt + p * plane + st * slab + db * 256);
+#pragma unroll
+      for (int i = 0; i < kSplitProducts; ++i) {
+        floatx16 &c = i == kSplitMain ? dq[db] : dqc[db];
+        c = mfma32x32x16(ds[kSplitA[i]], k[kSplitB[i]], c);
+      }
+    }
+  }
+}
+
+// Joins the two accumulators; whether some row came out non-finite (wave-uniform).
+template <int HD>
+__device__ __forceinline__ bool dq_finish(floatx16 (&dq)[HD / 32], const floatx16 (&dqc)[HD / 32]) {
+  float bad = 0.f;
+#pragma unroll
+  for (int db = 0; db < HD / 32; ++db) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dq[db][r] += dqc[db][r];
+    bad = nonfinite_sum(dq[db], bad);
+  }
+  return any_nonfinite(bad);
+}
+
+// Query block qi on the fp32 MFMA straight from memory (see the dK/dV kernel); dsw:
+// this lane's part of its dS blocks.
+template <int HD>
+__device__ __forceinline__ void dq_recompute(const BwdArgs &a, const float *kbase, const float *dsw, int qi, int li,
+                                             int hf, floatx16 (&dq)[HD / 32]) {
+#pragma unroll
+  for (int db = 0; db < HD / 32; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
+#pragma unroll 1
+  for (int j = 0; j <= qi; ++j)
+#pragma unroll 1
+    for (int s = 0; s < 16; ++s) {
+      const float x = dsw[(size_t)j * 1024 + s];
+      const float *krow = kbase + (size_t)min(32 * j + 2 * s + hf, a.lk - 1) * a.ldk;
+#pragma unroll
+      for (int db = 0; db < HD / 32; ++db) dq[db] = mfma32x32x2(x, krow[db * 32 + li], dq[db]);
+    }
+}
+
 // dQ from the dS blocks that the dK/dV kernel stored (causal, lq == lk, 16-byte
-// aligned rows): dQ^T = scale K^T dS^T, one product instead of recomputing S and
-// dP, on three bf16 pieces per fp32 operand (common.h).  Query-tile major with
+// aligned rows): dQ = scale dS K, one product instead of recomputing S and dP, on
+// three bf16 pieces per fp32 operand (common.h).  Query-tile major with
 // the heaviest tiles first, as the forward.  Wave w owns query block i = q0 / 32 +
 // w; for its key blocks j <= i the dS operand (dS[q][2s + c], s = 0..15, in lane
 // (q, c)) is 16 contiguous floats per lane, loaded two blocks ahead, and K^T
-// streams through double-buffered LDS.  A lane ends with one query's dims in
-// registers, so both halves of a rotary pair are in one lane and the stores are
-// 16 bytes wide.  The blocks' bytes bound it: 2.1 GB at 4 x 4096 x 16 heads.
+// streams through double-buffered LDS as the other operand.  The blocks' bytes
+// bound it: 2.1 GB at 4 x 4096 x 16 heads.
 template <int HD, int BN>
 __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const BwdArgs a) {
   constexpr int NKB = BN / 32;
@@ -1101,27 +1205,7 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
 #pragma unroll
         for (int i = 0; i < 4; ++i) n2[i] = *reinterpret_cast<const vf4 *>(dsw + (size_t)(j + 2) * 1024 + 4 * i);
       }
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = cur[2 * st + (e >> 2)][e & 3];
-        bf16x8 ds[3];
-        split_operand(x, ds);
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          bf16x8 k[3];
-#pragma unroll
-          for (int p = 0; p < 3; ++p)
-            k[p] = *reinterpret_cast<const bf16x8 *>(lds[lbuf] + ko + p * Stage::PLANE + (2 * kb + st) * Stage::SLAB +
-                                                     db * 256);
-#pragma unroll
-          for (int i = 0; i < kSplitProducts; ++i) {
-            floatx16 &c = i == kSplitMain ? dq[db] : dqc[db];
-            c = mfma32x32x16(k[kSplitA[i]], ds[kSplitB[i]], c);
-          }
-        }
-      }
+      dq_block<HD>(cur, lds[lbuf] + ko + 2 * kb * Stage::SLAB, Stage::PLANE, Stage::SLAB, dq, dqc);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         cur[i] = n1[i];
@@ -1132,32 +1216,88 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
     __syncthreads();
   }
 
-  float bad = 0.f;
+  if (last < 0) return;
+  if (dq_finish<HD>(dq, dqc)) dq_recompute<HD>(a, kbase, dsw, qi, li, hf, dq);
+  RowStore<HD> out;
+  out.load(a, qw0, li, hf);
+  out.store(a, dq, b, qw0, col0, li, hf);
+}
+
+// The same product, in the same order, for sequences of head dim 32 up to 32 *
+// kShortQB long: one workgroup per (sequence, head) stages the pieces of the head's
+// whole K^T once (flash_bwd_dq_ds_kernel's workgroups read K 2.5 times over at 512
+// queries: 1482 instead of 1276 MB for 2048 heads); wave w owns query blocks w and
+// nqb - 1 - w, so every wave has nqb + 1 key blocks of work (the middle block of an
+// odd count alone) and no barrier follows the staging.
+constexpr int kShortQB = 16;
+__global__ void __launch_bounds__(32 * kShortQB, 2) flash_bwd_dq_ds_short_kernel(const BwdArgs a) {
+  constexpr int HD = 32;
+  typedef KtStage<HD, 64> Stage;
+  constexpr int NDB = HD / 32, CH = HD / 4, PLANE = 2 * kShortQB * Stage::SLAB;
+  constexpr int PF = 4;
+  __shared__ __attribute__((aligned(16))) char lds[3 * PLANE];
+  const int bh = blockIdx.x;
+  const int b = bh / a.heads, h = bh % a.heads;
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 31, hf = lane >> 5;
+  const int nqb = (a.lq + 31) >> 5;
+  const int col0 = h * HD;
+  const float *__restrict__ kbase = a.k + (size_t)b * a.lk * a.ldk + col0;
+  const float *__restrict__ dsbh = a.ds + (size_t)bh * a.ds_bh + li * 32 + hf * 16;
+  // dS operands PF blocks ahead in a ring: block j lives in buf[j % PF] (the loop
+  // is unrolled by PF, so every index is a constant and no load in flight is ever
+  // copied), and the load of block j + PF goes into the buffer that block j has
+  // just left.  The second query block's first loads go out before the first
+  // one's stores.
+  vf4 buf[PF][4];
+  auto fetch = [&](vf4 (&x)[4], int qi, int j) {
+    if (j <= qi) {
 #pragma unroll
-  for (int db = 0; db < NDB; ++db) {
+      for (int i = 0; i < 4; ++i)
+        x[i] = *reinterpret_cast<const vf4 *>(dsbh + ((size_t)qi * (qi + 1) / 2 + j) * 1024 + 4 * i);
+    }
+  };
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dq[db][r] += dqc[db][r];
-    bad = nonfinite_sum(dq[db], bad);
+  for (int p = 0; p < PF; ++p) fetch(buf[p], nqb - 1 - wave, p);
+  // K rows [0, 32 nqb) of the head, rows past lk clamped (their dS is 0)
+  for (int e = t; e < nqb * 16 * CH; e += blockDim.x) {
+    const int sb = e & 7, g = (e >> 3) % CH, slab = (e >> 3) / CH;
+    const int row = Stage::unit_row(slab, sb);
+    const vf4 r0 = *reinterpret_cast<const vf4 *>(kbase + (size_t)min(row, a.lk - 1) * a.ldk + 4 * g);
+    const vf4 r1 = *reinterpret_cast<const vf4 *>(kbase + (size_t)min(row + 2, a.lk - 1) * a.ldk + 4 * g);
+    Stage::put(lds + Stage::unit_dst(slab, g, sb), PLANE, r0, r1);
   }
-  if (any_nonfinite(bad)) {  // on the fp32 MFMA straight from memory (see the dK/dV kernel)
+  __syncthreads();
+  const int ko = Stage::operand(li, hf);
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    const int qi = pass == 0 ? nqb - 1 - wave : wave;
+    if (pass == 1 && qi >= nqb - 1 - wave) break;  // the middle block ran in pass 0
+    floatx16 dq[NDB], dqc[NDB];                     // hh, and its corrections
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
-#pragma unroll 1
-    for (int j = 0; j <= last; ++j)
-#pragma unroll 1
-      for (int s = 0; s < 16; ++s) {
-        const float x = dsw[(size_t)j * 1024 + s];
-        const float *krow = kbase + (size_t)min(32 * j + 2 * s + hf, a.lk - 1) * a.ldk;
+      for (int r = 0; r < 16; ++r) dq[db][r] = dqc[db][r] = 0.f;
+    for (int j0 = 0; j0 <= qi; j0 += PF) {
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) dq[db] = mfma32x32x2(krow[db * 32 + li], x, dq[db]);
+      for (int u = 0; u < PF; ++u) {
+        const int j = j0 + u;
+        if (j > qi) break;
+        dq_block<HD>(buf[u], lds + ko + 2 * j * Stage::SLAB, PLANE, Stage::SLAB, dq, dqc);
+        fetch(buf[u], qi, j + PF);
       }
+    }
+    RowStore<HD> out;
+    out.load(a, 32 * qi, li, hf);
+    if (pass == 0 && wave < nqb - 1 - wave) {
+#pragma unroll
+      for (int p = 0; p < PF; ++p) fetch(buf[p], wave, p);
+    }
+    if (dq_finish<HD>(dq, dqc)) dq_recompute<HD>(a, kbase, dsbh + (size_t)qi * (qi + 1) / 2 * 1024, qi, li, hf, dq);
+    out.store(a, dq, b, 32 * qi, col0, li, hf);
   }
-  const int qrow = qw0 + li;
-  if (qrow < a.lq)
-    store_column<HD, true>(a, dq, a.dq + ((size_t)b * a.lq + qrow) * a.lddq + col0, a.scale,
-                          a.rope_cs ? a.rope_cs + (size_t)qrow * (a.hd >> 1) : nullptr, hf);
 }
 
 // Any head dim, any strides: one workgroup per (sequence, head) walks the
@@ -1287,7 +1427,14 @@ void launch_bwd(BwdArgs &a, hipStream_t st) {
     if constexpr (CAUSAL && !HAS_MASK && VEC) {
       if (a.ds) {  // dQ from the stored dS blocks
         flash_bwd_dkdv_split_kernel<HD, true, false, true, true><<<kgrid, kblock, 0, st>>>(a);
-        flash_bwd_dq_ds_kernel<HD, 64><<<qgrid, block, 0, st>>>(a);
+        // Whole K^T per (sequence, head) where that fills the device: us at 8 heads
+        // of 32, short / not: 256 x 511 313 / 358, 128 x 512 160 / 176, 64 x 512 81 /
+        // 86, 32 x 512 37 / 37, 64 x 400 58 / 60; at 384 keys and below the staged
+        // tile is half empty (128 x 300 79 / 74).
+        if (HD == 32 && a.lq > 384 && a.lq <= 32 * kShortQB && n_bh >= 2 * num_cus())
+          flash_bwd_dq_ds_short_kernel<<<dim3(n_bh), dim3(64 * ((a.lq + 63) / 64)), 0, st>>>(a);
+        else
+          flash_bwd_dq_ds_kernel<HD, 64><<<qgrid, block, 0, st>>>(a);
         return;
       }
     }

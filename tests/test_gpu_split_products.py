@@ -236,3 +236,40 @@ def test_attention_backward_values_outside_the_split(hd):
     want = backward64(q, k, v, dout, heads, scale, tril, per=2)  # what they reach is summed on the fp32 MFMA
     for stored in (False, True):
         check_backward(backward(q, k, v, dout, heads, scale, True, stored=stored), want, f"hd {hd} stored {stored}")
+
+
+def backward_saved(q, k, v, dout, batch, heads, rope):
+    """Causal cdml_sdpa_bwd_saved(_rope) of `batch` sequences, with room for the stored dS -> dQ, dK, dV."""
+    R, D = q.shape
+    L, hd, C = R // batch, D // heads, G.C
+    lib, st, scale = G.N.lib(), G.stream().handle, 1.0 / np.sqrt(D // heads)
+    bufs = [G.up(t) for t in (q, k, v, dout)]
+    o, lse, cs = G.N.DeviceBuffer(R * D * 4), G.N.DeviceBuffer(batch * heads * L * 4), G.N.DeviceBuffer(L * hd * 4)
+    grads = [G.N.DeviceBuffer(R * D * 4) for _ in range(3)]
+    qkv = [x for b in bufs[:3] for x in (b.ptr, D)]
+    outs = [x for g in grads for x in (g.ptr, D)]
+    G.N.check(lib.cdml_sdpa_fwd_lse(*qkv, o.ptr, D, lse.ptr, batch, L, L, D, heads, scale, 1, None, st))
+    G.N.check(lib.cdml_rope_table(cs.ptr, L, hd, 10000.0, st))
+    n = C.c_size_t(0)
+    G.N.check(lib.cdml_sdpa_bwd_saved_workspace_size(batch, L, L, D, heads, 1, C.byref(n)))
+    ws = G.N.DeviceBuffer(n.value)
+    args = [*qkv, o.ptr, D, lse.ptr, bufs[3].ptr, D, *outs, batch, L, L, D, heads, scale, 1, None]
+    if rope:
+        G.N.check(lib.cdml_sdpa_bwd_saved_rope(*args, cs.ptr, L, ws.ptr, n.value, st))
+    else:
+        G.N.check(lib.cdml_sdpa_bwd_saved(*args, ws.ptr, n.value, st))
+    return [G.down(g, (R, D)) for g in grads]
+
+
+# 13 to 16 query blocks, whole and ragged, of at least 512 (sequence, head) pairs take the kernel that stages a
+# head's whole K; a few sequences take the tiled one, which test_attention_backward checks
+@pytest.mark.parametrize("L", [385, 416, 447, 512])
+@pytest.mark.parametrize("rope", [False, True])
+def test_short_dq_has_the_bits_of_the_tiled_one(L, rope):
+    heads, few, copies = 4, 4, 32
+    q, k, v, dout = (synth.normal(i, (few * L, heads * 32)) for i in (1, 2, 3, 4))
+    dout[L + 5, 40] = np.inf  # one head's dQ is recomputed on the fp32 MFMA
+    want = backward_saved(q, k, v, dout, few, heads, rope)
+    got = backward_saved(*(np.tile(t, (copies, 1)) for t in (q, k, v, dout)), few * copies, heads, rope)
+    for g, w, name in zip(got, want, ("dQ", "dK", "dV")):
+        assert np.array_equal(g.view(np.uint32), np.tile(w, (copies, 1)).view(np.uint32)), name
