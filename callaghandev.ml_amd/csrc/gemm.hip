@@ -483,8 +483,7 @@ struct OpStage {
       }
     }
   }
-  // The last, ragged k-tile: k at or past kvalid read as zero (T = false:
-  // kvalid % 4 == 0).
+  // The last, ragged k-tile: k at or past kvalid are not read, they count as zero.
   __device__ __forceinline__ void load_tail(const float *__restrict__ base, int kvalid) {
     const vf4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -495,7 +494,13 @@ struct OpStage {
         if (2 * sb + 1 < kvalid) v[2 * i + 1] = *reinterpret_cast<const vf4 *>(base + off[i] + ldk);
       } else {
         v[i] = zero;
-        if (4 * sb < kvalid) v[i] = *reinterpret_cast<const vf4 *>(base + off[i]);
+        if (4 * sb + 3 < kvalid) {
+          v[i] = *reinterpret_cast<const vf4 *>(base + off[i]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            if (4 * sb + c < kvalid) v[i][c] = base[off[i] + c];
+        }
       }
     }
   }
@@ -714,8 +719,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &
   }
 }
 
-// Tiled kernel (16-byte aligned rows, element offsets below 2^32; K % 4 == 0
-// where an operand is [rows][K], rows % 4 == 0 where it is [K][rows]).  A
+// Tiled kernel (16-byte aligned rows, element offsets below 2^32; rows % 4 == 0
+// where an operand is [K][rows]).  A
 // workgroup of WM x WN waves computes a TM x TN tile of C, each wave a
 // (TM/WM) x (TN/WN) block of 32x32 tiles on the bf16 MFMA, both operands split
 // into three bf16 pieces on their way into LDS (common.h).  K advances by 16
@@ -1669,10 +1674,10 @@ int launch_tile(GemmArgs g, hipStream_t stream) {
 
 // Whether a [rows, K] (T = false) or [K, rows] (T = true) operand with row
 // stride ld and base p suits the tiled kernel's staging.
-bool stage_ok(const float *p, int rows, int K, int ld, bool T) {
+bool stage_ok(const float *p, int rows, int ld, bool T) {
   if (!aligned16(p) || ld % 4) return false;
   if (T) return rows % 4 == 0 && 16ull * (unsigned long long)ld + (unsigned long long)rows < (1ull << 32);
-  return K % 4 == 0 && (unsigned long long)rows * ld < (1ull << 32);
+  return (unsigned long long)rows * ld < (1ull << 32);
 }
 
 // 128 x 128 tiles (two workgroups per CU) where they give three quarters of
@@ -1749,11 +1754,11 @@ int launch_gemm(GemmArgs &g, bool ta, bool tb, hipStream_t stream, const char *w
     return fail(CDML_E_INVALID, "%s: matrix too large", what);
   bool fast = g.K > 0;
   for (int i = 0; i < g.nprob; ++i)
-    fast = fast && stage_ok(g.p[i].a, g.M, g.K, g.lda, ta) && stage_ok(g.p[i].w, g.N, g.K, g.ldb, tb);
+    fast = fast && stage_ok(g.p[i].a, g.M, g.lda, ta) && stage_ok(g.p[i].w, g.N, g.ldb, tb);
   if (g.kseg) {  // only the tiled input-gradient kernel reads K segments
     bool ok = !ta && tb && !has_epi(g) && g.nprob == 1 && g.ksplit <= 1 && g.kseg * 16 * 3 == g.K;
     for (int i = 0; ok && i < 3; ++i)
-      ok = stage_ok(g.p[i].a, g.M, g.kseg * 16, g.lda, false) && stage_ok(g.p[i].w, g.N, g.kseg * 16, g.ldb, true);
+      ok = stage_ok(g.p[i].a, g.M, g.lda, false) && stage_ok(g.p[i].w, g.N, g.ldb, true);
     if (!ok) return fail(CDML_E_INVALID, "%s: K segments need the tiled input-gradient kernel", what);
     fast = true;
   }
@@ -2160,7 +2165,7 @@ extern "C" int cdml_backprop_qkv(const float *x, const float *dq, const float *d
     const float *w[3] = {wq, wk, wv};
     bool fused = out_dim > 0 && out_dim % 16 == 0 && (long long)3 * out_dim <= INT32_MAX;
     for (int s = 0; fused && s < 3; ++s)
-      fused = stage_ok(d[s], rows, out_dim, out_dim, false) && stage_ok(w[s], in_dim, out_dim, in_dim, true);
+      fused = stage_ok(d[s], rows, out_dim, false) && stage_ok(w[s], in_dim, in_dim, true);
     if (fused) {
       GemmArgs g{};
       g.lda = out_dim;

@@ -51,6 +51,23 @@ def test_forward_and_gradients(rows, ind, out):
     check(bg[:, None], dy.T, np.ones((rows, 1), np.float32), "bias gradient", bg0.astype(np.float64)[:, None])
 
 
+# out (the product's K) with every remainder by 4 and by 16, in rows padded to the next multiple of 4
+@pytest.mark.parametrize("rows,ind,out", [(17, 8, 130), (65, 64, 17), (129, 132, 19), (300, 200, 31), (4099, 1024, 45)])
+def test_padded_rows_of_any_width(rows, ind, out):
+    """Input gradient and matrix product of rows with an aligned stride whose width is no multiple of 4: the padding
+    (NaN here) is not read into the sums."""
+    ld = -(-out // 4) * 4
+    dy, w = synth.normal(4, (rows, out)), synth.normal(2, (out, ind))
+    padded = np.full((rows, ld), np.nan, np.float32)
+    padded[:, :out] = dy
+    bdy, bw, dx = G.up(padded), G.up(w), G.N.DeviceBuffer(rows * ind * 4)
+    G.N.check(G.N.lib().cdml_linear_backward(None, ind, bdy.ptr, ld, bw.ptr, dx.ptr, ind, None, None, rows, ind, out, 0,
+                                             None, 0, G.stream().handle))
+    check(G.down(dx, (rows, ind)), dy, w, "input gradient")
+    G.N.check(G.N.lib().cdml_matmul(bdy.ptr, ld, bw.ptr, ind, dx.ptr, ind, rows, out, ind, G.stream().handle))
+    check(G.down(dx, (rows, ind)), dy, w, "matrix product")
+
+
 @pytest.mark.parametrize("rows,ind,out", [(70, 48, 72), (2100, 64, 1540)])
 def test_values_outside_the_split(rows, ind, out):
     """Infinities, NaNs and values above the largest bf16 give what the fp32
