@@ -572,6 +572,14 @@ __device__ __forceinline__ void recompute_blocks(const GemmArgs &args, int prob,
   }
 }
 
+// Orders the LDS accesses of a wave's lanes where they pass values to each other
+// without a workgroup barrier: the hardware keeps a wave's LDS accesses in order, and
+// this keeps the compiler from moving them past each other.  It emits no instruction.
+__device__ __forceinline__ void lds_handover() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Where a wave's blocks go: C (or a split-K partial, which takes neither bias
 // nor activation nor beta).
 struct TileOut {
@@ -649,6 +657,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &
   }
 #pragma unroll 1
   for (int i = 0; i < BI; ++i) {
+    if (i > 0) lds_handover();  // the band's last reads
 #pragma unroll
     for (int ii = 0; ii < BI; ++ii)
       if (ii == i) {  // the accumulators need constant indices, the loop's body only one copy
@@ -657,6 +666,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &
 #pragma unroll
           for (int r = 0; r < 16; ++r) lds[(8 * (r >> 2) + 4 * hf + (r & 3)) * PITCH + j * 32 + li] = acc[ii][j][r];
       }
+    lds_handover();
     auto rows = [&](auto full) {
       constexpr bool FULL = decltype(full)::value;  // every row and column exists, 16-byte accesses
 #pragma unroll 1
