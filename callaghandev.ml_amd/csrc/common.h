@@ -63,11 +63,15 @@ __device__ __forceinline__ floatx16 mfma32x32x2(float a, float b, floatx16 c) {
 
 // fp32 products on the bf16 matrix cores.  An fp32 value is the sum of three
 // bf16 values, h = bf16(x), m = bf16(x - h), l = x - h - m, each rounded to
-// nearest: 8 + 8 + 8 significant bits hold all 24, so the split loses nothing
-// (for |x| above 2^-110; below it l underflows).  Of the nine products of two
-// split operands, hh + hm + mh + mm + hl + lh are summed in fp32; ml, lm and ll
-// are below 2^-24 of |a b| together.  Six bf16 products take 6/16 of one fp32
-// product's matrix-core cycles.
+// nearest: 8 + 8 + 8 significant bits hold all 24.  Operands are multiplied by
+// kSplitScale = 2^16 on their way into the split, and the sums by 2^-32 at the end:
+// the last bit of the smallest fp32 value, 2^-149, then lies at 2^-133, the last
+// bit of the smallest bf16 value (the MFMA keeps subnormal operands and sums), so
+// the split loses nothing at all.  (Unscaled, l underflows below 2^-110: an operand
+// of rms 2^-118 had an error of 9e-6, one of 2^-124 6e-4.)  Of the nine products
+// of two split operands, hh + hm + mh + mm + hl + lh are summed in fp32; ml, lm
+// and ll are below 2^-24 of |a b| together.  Six bf16 products take 6/16 of one
+// fp32 product's matrix-core cycles.
 //
 // The bf16 MFMA adds eight products at a time to its accumulator, one rounding
 // each: with all six products in one accumulator a K of 16 takes 12 roundings
@@ -88,10 +92,11 @@ __device__ __forceinline__ floatx16 mfma32x32x2(float a, float b, floatx16 c) {
 // columns of the operands change their sign as they are split, at no cost),
 // which turns the drift round, and undo the sign at the end.
 //
-// An infinity, a NaN or a value above the largest bf16 leaves inf - inf in m,
-// so every result that it reaches comes out non-finite; the kernels test their
-// results for that (any_nonfinite) and recompute such blocks with
-// mfma32x32x2, whose infinities and NaNs are those of the fp32 sum.
+// An infinity, a NaN or a value of 2^112 and more (above the largest bf16 once
+// scaled) leaves inf - inf in m, and a sum of 2^96 and more overflows, so every
+// result that one reaches comes out non-finite; the kernels test their results for
+// that (any_nonfinite) and recompute such blocks with mfma32x32x2, whose
+// infinities and NaNs are those of the fp32 sum.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t vu2 __attribute__((ext_vector_type(2)));
 typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
@@ -99,6 +104,10 @@ constexpr int kSplitProducts = 6;
 constexpr int kSplitA[kSplitProducts] = {2, 0, 1, 1, 0, 0};  // piece of A (0 = h, 1 = m, 2 = l)
 constexpr int kSplitB[kSplitProducts] = {0, 2, 1, 0, 1, 0};  // piece of B
 constexpr int kSplitMain = 5;                                // hh; the others are its corrections
+
+constexpr float kSplitScale = 65536.f;             // 2^16, of either operand
+constexpr float kSplitUnscale = 1.f / 65536.f;     // of a sum with one scaled operand
+constexpr float kSplitUnscale2 = kSplitUnscale * kSplitUnscale;  // with two
 
 // (bf16(a), bf16(b)) in the low and high half, rounded to nearest even.
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
@@ -116,10 +125,10 @@ __device__ __forceinline__ void split_bf16x3(float a, float b, uint32_t &h, uint
 }
 
 // The three pieces of eight values as MFMA operands.
-__device__ __forceinline__ void split_operand(const float (&x)[8], bf16x8 (&p)[3]) {
+__device__ __forceinline__ void split_operand(const float (&x)[8], float scale, bf16x8 (&p)[3]) {
   uint32_t h[4], m[4], l[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) split_bf16x3(x[2 * i], x[2 * i + 1], h[i], m[i], l[i]);
+  for (int i = 0; i < 4; ++i) split_bf16x3(x[2 * i] * scale, x[2 * i + 1] * scale, h[i], m[i], l[i]);
   p[0] = __builtin_bit_cast(bf16x8, (vu4{h[0], h[1], h[2], h[3]}));
   p[1] = __builtin_bit_cast(bf16x8, (vu4{m[0], m[1], m[2], m[3]}));
   p[2] = __builtin_bit_cast(bf16x8, (vu4{l[0], l[1], l[2], l[3]}));

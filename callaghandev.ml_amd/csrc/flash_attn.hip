@@ -15,7 +15,9 @@
 //                   one swap between the two half-waves.
 //   online softmax  running max / sum per query in the exp2 domain
 //                   (scale * log2 e folded into Q), masked keys -inf.
-//   O^T += V^T P^T  accumulators 8 s .. 8 s + 7 of a lane hold the keys 16 s +
+//   O^T += V^T P^T  V is scaled for the split (common.h), the probabilities are not:
+//                   one below 2^-110 loses at most 2^-134, where exp2 itself drops
+//                   those below 2^-126.  Accumulators 8 s .. 8 s + 7 of a lane hold the keys 16 s +
 //                   {4 h .. 4 h + 3, 8 + 4 h .. 8 + 4 h + 3} (h = lane / 32): V is
 //                   staged transposed with its keys in that order, so the
 //                   probabilities are consumed in place.
@@ -166,7 +168,8 @@ struct KvStage {
         for (int c = 0; c < 4; ++c) {
           uint32_t h, m, l;
           const float x = r[2 * i][c], y = r[2 * i + 1][c];
-          split_bf16x3(c & 1 ? -x : x, c & 1 ? -y : y, h, m, l);
+          const float f = c & 1 ? -kSplitScale : kSplitScale;
+          split_bf16x3(x * f, y * f, h, m, l);
           char *d = lds + dst + vslabs(i) * VSLAB + vgroups(i) * 32 + vcluster(c);
           *reinterpret_cast<uint32_t *>(d) = h;
           *reinterpret_cast<uint32_t *>(d + VPLANE) = m;
@@ -221,9 +224,14 @@ constexpr float kFastSumLimit = 4294967296.0f;  // 2^32
 
 // Q^T operand of a wave: the three bf16 pieces of q[qi][16 s + 8 hf + 0..7] times
 // scale_log2.  Rows past lq read row lq - 1: they are computed but never stored.
+// Scores start from the row's reference, so neither Q nor K takes the split's scale:
+// what a component below 2^-110 loses (2^-134) reaches a score only through a
+// component of 2^100 and more on the other side.  Returns whether Q holds one or
+// the other (wave-uniform); such rows are recomputed on the fp32 MFMA.
 template <int HD, bool VEC>
-__device__ __forceinline__ void load_q(bf16x8 (&q)[HD / 16][3], const FlashArgs &a, int b, int col0, int qi, int hf) {
+__device__ __forceinline__ bool load_q(bf16x8 (&q)[HD / 16][3], const FlashArgs &a, int b, int col0, int qi, int hf) {
   const float *qrow = a.q + ((size_t)b * a.lq + min(qi, a.lq - 1)) * a.ldq + col0;
+  float most = 0.f, least = 1.f;
 #pragma unroll
   for (int s = 0; s < HD / 16; ++s) {
     float x[8];
@@ -239,8 +247,14 @@ __device__ __forceinline__ void load_q(bf16x8 (&q)[HD / 16][3], const FlashArgs 
         for (int r = 0; r < 4; ++r) x[4 * g + r] = d + r < a.hd ? qrow[d + r] * a.scale_log2 : 0.f;
       }
     }
-    split_operand(x, q[s]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      most = fmaxf(most, fabsf(x[e]));
+      least = fminf(least, x[e] == 0.f ? 1.f : fabsf(x[e]));
+    }
+    split_operand(x, 1.f, q[s]);
   }
+  return __builtin_amdgcn_ballot_w64(most >= 0x1p100f || least < 0x1p-110f) != 0;
 }
 
 // The online softmax of one wave's 32 query rows (one per lane % 32) over
@@ -299,7 +313,7 @@ struct OnlineRows {
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = p[8 * s + e];
       bf16x8 pp[3];
-      split_operand(x, pp);
+      split_operand(x, 1.f, pp);
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
         bf16x8 v[3];
@@ -422,8 +436,8 @@ struct OnlineRows {
     for (int db = 0; db < NDB; ++db) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float o = oacc[db][r] + ocor[db][r];
-        oacc[db][r] = r & 1 ? -o : o;
+        // (adding 0 keeps the zeros of a row without a key positive)
+        oacc[db][r] = fmaf(oacc[db][r] + ocor[db][r], r & 1 ? -kSplitUnscale : kSplitUnscale, 0.f);
       }
       bad = nonfinite_sum(oacc[db], bad);
     }
@@ -431,8 +445,8 @@ struct OnlineRows {
   }
 
   // The wave's rows on the fp32 MFMA straight from memory: only for rows that
-  // came out non-finite (an infinity or NaN in Q, K or V, or a product that
-  // overflows), so that they hold what the fp32 products give.
+  // came out non-finite (common.h) or whose Q is out of the split's range (load_q),
+  // so that they hold what the fp32 products give.
   __device__ __forceinline__ void recompute(const FlashArgs &a, int b, int col0, int qi, int li, int hf, int kend,
                                             int key_last, const uint8_t *mrow) {
     init();
@@ -516,7 +530,7 @@ __global__ void __launch_bounds__(FA_THREADS, HD <= 32 ? 3 : (HD <= 64 ? 2 : 1))
   st.init(a.ldk, a.ldv);
   st.load(kbase, vbase, a.ldk, a.ldv, 0, a.lk, a.hd);
   bf16x8 q[HD / 16][3];
-  load_q<HD, VEC>(q, a, b, col0, qi, hf);
+  const bool wide = load_q<HD, VEC>(q, a, b, col0, qi, hf);
   st.store(lds[0]);
   __syncthreads();
 
@@ -568,7 +582,7 @@ __global__ void __launch_bounds__(FA_THREADS, HD <= 32 ? 3 : (HD <= 64 ? 2 : 1))
     st.store(lds[cur ^ 1]);
     __syncthreads();
   }
-  if (rows.finish() && qw0 < a.lq)
+  if ((rows.finish() || wide) && qw0 < a.lq)
     rows.recompute(a, b, col0, qi, li, hf, CAUSAL ? min(qw0 + 32, a.lk) : a.lk, key_last, mrow);
   rows.store(a, bh, b, qi, col0, hf);
 }

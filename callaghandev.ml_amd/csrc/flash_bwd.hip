@@ -470,8 +470,8 @@ struct QgStage {
       uint32_t w[3][4];  // [piece][dim]: query `row` in the low half, `row + 1` in the high half
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const float x = r[i][0][c], y = r[i][1][c];
-        split_bf16x3(c & 1 ? -x : x, c & 1 ? -y : y, w[0][c], w[1][c], w[2][c]);
+        const float f = c & 1 ? -kSplitScale : kSplitScale;
+        split_bf16x3(r[i][0][c] * f, r[i][1][c] * f, w[0][c], w[1][c], w[2][c]);
       }
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
@@ -511,6 +511,9 @@ struct QgStage {
 // 2.33 -> 1.93 ms (this kernel 1.40 -> 1.05 ms), bound by the exponentials and splits
 // between the products: vector ALU 48% of the cycles, matrix pipes 34%.
 //
+// All operands but P carry the split's scale; a probability below 2^-110 loses at
+// most 2^-134, where exp2 itself drops those below 2^-126.
+//
 // S and dP of odd keys are computed negated, so that the drift of the bf16 MFMA
 // (common.h) cancels in a query's sum of dS over its keys, which has to be zero.
 //
@@ -549,12 +552,12 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
 
   // B operands of S = Q K^T and / or dP = dO V^T: the pieces of K[key][16 s + 8 hf
   // + 0..7] and of V, odd dims negated as in the staged tiles, and odd keys.
+  const float sgn = li & 1 ? -1.f : 1.f;
   bf16x8 kv[NT][NS][3];
 #pragma unroll
   for (int x = 0; x < NT; ++x) {
     const size_t kr = (size_t)b * a.lk + min(key, a.lk - 1);
     const float *row = (PAIRED ? role_p : x == 0) ? a.k + kr * a.ldk + col0 : a.v + kr * a.ldv + col0;
-    const uint32_t odd_key = (uint32_t)(li & 1) << 31;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       float f[8];
@@ -562,9 +565,9 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       for (int e = 0; e < 8; ++e) {
         const int d = 16 * s + 8 * hf + e;
         const float v = VEC || d < a.hd ? row[d] : 0.f;
-        f[e] = __uint_as_float(__float_as_uint(e & 1 ? -v : v) ^ odd_key);
+        f[e] = e & 1 ? -v : v;
       }
-      split_operand(f, kv[x][s]);
+      split_operand(f, sgn * kSplitScale, kv[x][s]);
     }
   }
 
@@ -584,7 +587,7 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       for (int r = 0; r < 16; ++r) acc[x][db][r] = cor[x][db][r] = 0.f;
 
   // P = exp2(S scale log2 e - lse) in place; scale_log2 carries the sign of an
-  // odd key.  l4(g): lse of query rows 8 g + 4 hf + 0..3 of the sub-block.
+  // odd key and undoes the split's scale.  l4(g): lse of query rows 8 g + 4 hf + 0..3 of the sub-block.
   auto probabilities = [&](floatx16 &s, float scale_log2, int qb0, auto l4) {
     // (the masked and the unmasked forms are separate branches: a select
     // per element would run the mask arithmetic on every sub-block)
@@ -612,13 +615,13 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       }
     }
   };
-  // dS = P (sgn dP - D) in place of dP, and the dS store.
-  auto score_gradients = [&](const floatx16 &p, floatx16 &dp, float sgn, int qb0, auto d4) {
+  // dS = P (f dP - D) in place of dP, and the dS store.
+  auto score_gradients = [&](const floatx16 &p, floatx16 &dp, float f, int qb0, auto d4) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const vf4 d = d4(g);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) dp[4 * g + c] = p[4 * g + c] * fmaf(sgn, dp[4 * g + c], -d[c]);
+      for (int c = 0; c < 4; ++c) dp[4 * g + c] = p[4 * g + c] * fmaf(f, dp[4 * g + c], -d[c]);
     }
     if constexpr (STORE_DS) {
       // The stored dS blocks of this (sequence, head) as a buffer resource (the
@@ -658,15 +661,16 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
     for (int r = 0; r < 16; ++r) m[r] += c[r];
     return m;
   };
-  // acc[n] += (the staged transposed rows of one tensor) x w, w the 32 x 32 P or dS.
-  auto column_product = [&](const char *cols, const floatx16 &w, int n) {
+  // acc[n] += (the staged transposed rows of one tensor) x w, w the 32 x 32 P or dS
+  // times ws.
+  auto column_product = [&](const char *cols, const floatx16 &w, float ws, int n) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       float x[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = w[8 * st + e];
       bf16x8 wp[3];
-      split_operand(x, wp);
+      split_operand(x, ws, wp);
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
         bf16x8 g[3];
@@ -684,7 +688,9 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
   // Sub-blocks wholly before these keys contribute nothing, and keys that all
   // lie past lk take nothing.
   auto active = [&](int qb0) { return kw0 < a.lk && !(CAUSAL && qb0 + 31 < kw0); };
-  const float sgn = li & 1 ? -1.f : 1.f;
+  // Both operands of S and dP carry the split's scale.
+  const float s_scale = sgn * kSplitUnscale2 * a.scale_log2, dp_scale = sgn * kSplitUnscale2;
+  constexpr float p_scale = 1.f, ds_scale = kSplitScale;
 
   auto lse4 = [&](int buf) {
     return [&, buf](int g) { return *reinterpret_cast<const vf4 *>(&Ls[buf][8 * g + 4 * hf]); };
@@ -727,20 +733,20 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       if (active(qb0)) {
         p = row_product(lds[cur], kv[0]);
         if constexpr (PAIRED) {
-          probabilities(p, sgn * a.scale_log2, qb0, lse4(cur));
+          probabilities(p, s_scale, qb0, lse4(cur));
 #pragma unroll
           for (int g = 0; g < 4; ++g) Ps[pair][g][lane] = vf4{p[4 * g], p[4 * g + 1], p[4 * g + 2], p[4 * g + 3]};
         } else {
           floatx16 dp = row_product(lds[cur] + Stage::TENSOR, kv[NT - 1]);
-          probabilities(p, sgn * a.scale_log2, qb0, lse4(cur));
-          column_product(lds[cur] + Stage::TENSOR, p, 0);
-          score_gradients(p, dp, sgn, qb0, delta4(cur));
-          column_product(lds[cur], dp, NT - 1);
+          probabilities(p, s_scale, qb0, lse4(cur));
+          column_product(lds[cur] + Stage::TENSOR, p, p_scale, 0);
+          score_gradients(p, dp, dp_scale, qb0, delta4(cur));
+          column_product(lds[cur], dp, ds_scale, NT - 1);
         }
       }
       if constexpr (PAIRED) {
         __syncthreads();
-        if (active(qb0)) column_product(lds[cur] + Stage::TENSOR, p, 0);  // dV^T += dO^T P
+        if (active(qb0)) column_product(lds[cur] + Stage::TENSOR, p, p_scale, 0);  // dV^T += dO^T P
       }
       stage(cur ^ 1);
       __syncthreads();
@@ -760,8 +766,8 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
 #pragma unroll
           for (int c = 0; c < 4; ++c) p[4 * g + c] = x[c];
         }
-        score_gradients(p, dp, sgn, qb0, delta4(cur));
-        column_product(lds[cur], dp, 0);  // dK^T += Q^T dS
+        score_gradients(p, dp, dp_scale, qb0, delta4(cur));
+        column_product(lds[cur], dp, ds_scale, 0);  // dK^T += Q^T dS
       }
       __syncthreads();
     }
@@ -771,13 +777,12 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
   float bad = 0.f;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
+    const bool of_v = PAIRED ? role_p : n == 0;
+    const float f = kSplitUnscale / (of_v ? p_scale : ds_scale);
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float x = acc[n][db][r] + cor[n][db][r];
-        acc[n][db][r] = r & 1 ? -x : x;
-      }
+      for (int r = 0; r < 16; ++r) acc[n][db][r] = (acc[n][db][r] + cor[n][db][r]) * (r & 1 ? -f : f);
       bad = nonfinite_sum(acc[n][db], bad);
     }
   }
@@ -1048,7 +1053,7 @@ struct KtStage {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       uint32_t h, m, l;
-      split_bf16x3(r0[c], r1[c], h, m, l);
+      split_bf16x3(r0[c] * kSplitScale, r1[c] * kSplitScale, h, m, l);
       *reinterpret_cast<uint32_t *>(d + cluster(c)) = h;
       *reinterpret_cast<uint32_t *>(d + cluster(c) + plane) = m;
       *reinterpret_cast<uint32_t *>(d + cluster(c) + 2 * plane) = l;
@@ -1089,7 +1094,7 @@ __device__ __forceinline__ void dq_block(const vf4 (&cur)[4], const char *kt, in
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = cur[2 * st + (e >> 2)][e & 3];
     bf16x8 ds[3];
-    split_operand(x, ds);
+    split_operand(x, kSplitScale, ds);
 #pragma unroll
     for (int db = 0; db < HD / 32; ++db) {
       bf16x8 k[3];
@@ -1111,7 +1116,7 @@ __device__ __forceinline__ bool dq_finish(floatx16 (&dq)[HD / 32], const floatx1
 #pragma unroll
   for (int db = 0; db < HD / 32; ++db) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dq[db][r] += dqc[db][r];
+    for (int r = 0; r < 16; ++r) dq[db][r] = (dq[db][r] + dqc[db][r]) * kSplitUnscale2;
     bad = nonfinite_sum(dq[db], bad);
   }
   return any_nonfinite(bad);

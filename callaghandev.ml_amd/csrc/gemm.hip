@@ -420,7 +420,8 @@ __global__ void __launch_bounds__(NTHREADS) gemm_nt_kernel(const GemmArgs args) 
 //   T = false: the source is [rows][K] (k contiguous, row stride ld): a unit
 //     is four k of one row, one 16-byte load and an 8-byte store per plane; a
 //     thread's units come in pairs of neighbouring rows, one in each of NC = 2
-//     clusters, so the stores of a wave cover 512 contiguous bytes.
+//     clusters, so the stores of a wave cover 512 contiguous bytes (with one unit
+//     per thread, NP = 1, a wave's rows fall in both clusters).
 //   T = true:  the source is [K][rows] (rows contiguous, k-row stride ld): a
 //     unit is four rows of two k, two 16-byte loads and per row (NC = 4) a
 //     4-byte store per plane, 256 contiguous bytes for eight units.
@@ -445,7 +446,7 @@ struct OpStage {
   static constexpr int NV = T ? 2 * NP : NP;               // their loads
   static constexpr int SPLITS = 2 * NV;                    // split_bf16x3 calls
   static constexpr int STORES = T ? 12 * NP : 3 * NP;
-  static_assert(NP >= 1 && ROWS * (T ? 2 : 4) % NT == 0 && (T || NP % 2 == 0), "staging shape");
+  static_assert(NP >= 1 && ROWS * (T ? 2 : 4) % NT == 0 && (T || NP % 2 == 0 || NP == 1), "staging shape");
   uint32_t off[NP];
   vf4 v[NV];
   int sa, sb;  // T = false: (row pair, first k / 4); T = true: (row group, k / 2)
@@ -453,7 +454,8 @@ struct OpStage {
 
   // First tile row of unit i.
   __device__ __forceinline__ int unit_row(int i) const {
-    return T ? 4 * (sa + NT / 8 * i) : 2 * sa + (i & 1) + NT / 2 * (i >> 1);
+    if (T) return 4 * (sa + NT / 8 * i);
+    return NP == 1 ? sa : 2 * sa + (i & 1) + NT / 2 * (i >> 1);
   }
   __device__ __forceinline__ void init(int row0, int rows, int ld) {
     const int t = threadIdx.x;
@@ -504,13 +506,9 @@ struct OpStage {
       }
     }
   }
-  // FLIP: the values also change their sign bit with `flip` (0 or 1 << 31).
-  template <bool FLIP>
-  __device__ __forceinline__ void store(char *lds, uint32_t flip) const {
-    auto signed_value = [&](float x, bool neg) {
-      if (FLIP) x = __uint_as_float(__float_as_uint(x) ^ flip);
-      return neg ? -x : x;
-    };
+  // scale: kSplitScale or its negative.
+  __device__ __forceinline__ void store(char *lds, float scale) const {
+    auto scaled = [&](float x, bool neg) { return x * (neg ? -scale : scale); };
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       if constexpr (T) {
@@ -518,16 +516,19 @@ struct OpStage {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           uint32_t h, m, l;
-          split_bf16x3(signed_value(v[2 * i][c], c & 1), signed_value(v[2 * i + 1][c], c & 1), h, m, l);
+          split_bf16x3(scaled(v[2 * i][c], c & 1), scaled(v[2 * i + 1][c], c & 1), h, m, l);
           *reinterpret_cast<uint32_t *>(d + cluster(c)) = h;
           *reinterpret_cast<uint32_t *>(d + cluster(c) + PLANE) = m;
           *reinterpret_cast<uint32_t *>(d + cluster(c) + 2 * PLANE) = l;
         }
       } else {
-        char *d = lds + cluster(i & 1) + (sa + NT / 4 * (i >> 1)) * 32 + sb * 8;
+        const bool odd = NP == 1 ? sa & 1 : i & 1;
+        const int place = NP == 1 ? sa >> 1 : sa + NT / 4 * (i >> 1);
+        char *d = lds + cluster(odd) + place * 32 + sb * 8;
+        const float f = odd ? -scale : scale;
         uint32_t h0, m0, l0, h1, m1, l1;
-        split_bf16x3(signed_value(v[i][0], i & 1), signed_value(v[i][1], i & 1), h0, m0, l0);
-        split_bf16x3(signed_value(v[i][2], i & 1), signed_value(v[i][3], i & 1), h1, m1, l1);
+        split_bf16x3(v[i][0] * f, v[i][1] * f, h0, m0, l0);
+        split_bf16x3(v[i][2] * f, v[i][3] * f, h1, m1, l1);
         *reinterpret_cast<vu2 *>(d) = vu2{h0, h1};
         *reinterpret_cast<vu2 *>(d + PLANE) = vu2{m0, m1};
         *reinterpret_cast<vu2 *>(d + 2 * PLANE) = vu2{l0, l1};
@@ -542,9 +543,8 @@ struct OpStage {
 
 // A wave's BI x BJ blocks recomputed on the fp32 MFMA straight from memory,
 // one block after the other: only for blocks whose split products came out
-// non-finite (an infinity, a NaN, a value above the largest bf16, or a sum that
-// overflows), so that they hold what the fp32 sum gives.  k runs over [k0, k1)
-// of each of nseg operand pairs.
+// non-finite (common.h), so that they hold what the fp32 sum gives.  k runs over
+// [k0, k1) of each of nseg operand pairs.
 template <int BI, int BJ, bool TA, bool TB>
 __device__ __forceinline__ void recompute_blocks(const GemmArgs &args, int prob, int nseg, int k0, int k1, int mw,
                                                  int nw, int li, int hf, floatx16 (&acc)[BI][BJ]) {
@@ -843,11 +843,10 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
   };
   // Split-K chunks take turns in the sign of opA: the drift of the partial
   // sums (common.h) would otherwise add up over the chunks.
-  constexpr bool FLIP = TA && TB;
-  const uint32_t flip = FLIP ? (uint32_t)(chunk & 1) << 31 : 0;
+  const float scale_a = TA && TB && (chunk & 1) ? -kSplitScale : kSplitScale;
   auto stage = [&](int buf) {
-    sa.template store<FLIP>(As + buf * StageA::BYTES, flip);
-    sb.template store<false>(Bs + buf * StageB::BYTES, 0);
+    sa.store(As + buf * StageA::BYTES, scale_a);
+    sb.store(Bs + buf * StageB::BYTES, kSplitScale);
   };
   const int ao = StageA::operand(wm * (TM / WM), li, hf), bo = StageB::operand(wn * (TN / WN), li, hf);
   bf16x8 a[3][BI], b[3][BJ];
@@ -918,7 +917,9 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
         read_b(0, nxt);
         constexpr int NM = kSplitProducts * BI * BJ;
         constexpr int NR = 2 * (BI + BJ);  // reads between the first MFMAs, then the stores
-        constexpr int VALU = (11 * (StageA::SPLITS + StageB::SPLITS) + NM - 1) / NM + 1;
+// Spreads a k-tile's VALU instructions (104 of the splits) over its 24 MFMAs; us with
+        // 4 / 6 of them per MFMA: forward 16384 x 4096 -> 1024 702 / 710, its dW 737 / 727.
+        constexpr int VALU = TA || TB ? 6 : 4;
         constexpr int STORES = StageA::STORES + StageB::STORES;
         constexpr int AT_ONCE = (STORES + NM - NR - 1) / (NM - NR);
         constexpr int EVERY = STORES > (NM - NR) / 2 ? 1 : 2;
@@ -951,15 +952,14 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
   }
   {
     // rows and columns of odd index were negated (rows 8 (r / 4) + 4 hf + r % 4)
-    const uint32_t s0 = ((uint32_t)(li & 1) << 31) ^ flip, s1 = s0 ^ (1u << 31);
+    const float s0 = (li & 1) != (scale_a < 0.f) ? -kSplitUnscale2 : kSplitUnscale2;
     float bad = 0.f;
 #pragma unroll
     for (int i = 0; i < BI; ++i)
 #pragma unroll
       for (int j = 0; j < BJ; ++j) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[i][j][r] = __uint_as_float(__float_as_uint(acc[i][j][r] + cor[i][j][r]) ^ (r & 1 ? s1 : s0));
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = (acc[i][j][r] + cor[i][j][r]) * (r & 1 ? -s0 : s0);
         bad = nonfinite_sum(acc[i][j], bad);
       }
     if (any_nonfinite(bad)) {
@@ -1691,9 +1691,9 @@ bool stage_ok(const float *p, int rows, int ld, bool T) {
 }
 
 // 128 x 128 tiles (two workgroups per CU) where they give three quarters of
-// the CUs one, 64 x 64 otherwise, four times as many (fwd / dX, us): 4096 x 1024
-// x 1024, 256 tiles of 128 x 128: 56 / 64 against 67 / 69; 2048 x 1024 x 1024, 128
-// tiles: 50 / 62 against 49 / 54; 512 x 1024 x 1024: 44 / 54 against 36 / 44.
+// the CUs one, 64 x 64 otherwise, four times as many (dX, us): 4096 x 1024 x 1024, 256
+// tiles of 128 x 128: 64 against 69; 2048 x 1024 x 1024, 128 tiles: 62 against 54;
+// 512 x 1024 x 1024: 54 against 44.
 // (256 x 128 with eight waves, one workgroup per CU, is 1-3% faster than 128 x
 // 128 forward and 2-8% slower in both gradients, whose short k-loops and long
 // epilogues another workgroup has to cover.)
@@ -1701,6 +1701,10 @@ template <bool TA, bool TB>
 int launch_tiled(GemmArgs &g, hipStream_t stream) {
   const long long tiles = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.nprob * std::max(g.ksplit, 1);
   if (4 * tiles >= 3LL * num_cus()) return launch_tile<128, 128, 2, 2, 2, 3, TA, TB>(g, stream);
+  // Four waves forward: a launch of few workgroups is bound by the splits between a
+  // wave's products (520 x 512 -> 512 21.5 -> 16.3 us, 200 x 1024 -> 1024 37.4 -> 27.6).
+  // A transposed operand has units for two waves only.
+  if constexpr (!TA && !TB) return launch_tile<64, 64, 2, 2, 3, 2, TA, TB>(g, stream);
   return launch_tile<64, 64, 2, 1, 3, 2, TA, TB>(g, stream);
 }
 

@@ -17,12 +17,12 @@ from cdml import synth
 pytestmark = pytest.mark.gpu
 
 
-def check(got, a, b, what, extra=0.0):
-    """got against a [M, K] @ b [K, N] (+ extra) in float64."""
+def check(got, a, b, what, extra=0.0, floor=2.0 ** -149):
+    """got against a [M, K] @ b [K, N] (+ extra) in float64; floor: what sums of subnormals may be off by."""
     with np.errstate(all="ignore"):
         A, B = a.astype(np.float64), b.astype(np.float64)
         want = A @ B + extra
-        bound = (a.shape[1] / 8 + 8) * 2.0 ** -24 * (np.abs(A) @ np.abs(B) + np.abs(extra))
+        bound = (a.shape[1] / 8 + 8) * 2.0 ** -24 * (np.abs(A) @ np.abs(B) + np.abs(extra)) + floor
     fine = np.isfinite(want) & (np.abs(want) < np.finfo(np.float32).max)
     assert np.array_equal(np.isnan(got), np.isnan(want)), f"{what}: NaNs elsewhere"
     inf = ~fine & ~np.isnan(want)
@@ -49,6 +49,18 @@ def test_forward_and_gradients(rows, ind, out):
     check(dx, dy, w, "input gradient")
     check(wg, dy.T, x, "weight gradient", wg0.astype(np.float64))
     check(bg[:, None], dy.T, np.ones((rows, 1), np.float32), "bias gradient", bg0.astype(np.float64)[:, None])
+
+
+@pytest.mark.parametrize("sx,sw", [(-124, 0), (0, -124), (-60, -60), (90, -110)])
+@pytest.mark.parametrize("rows,ind,out", [(70, 48, 72), (300, 100, 200), (2100, 64, 1540)])
+def test_small_operands(rows, ind, out, sx, sw):
+    """The split keeps all bits of operands down to the smallest normal floats."""
+    x, w = synth.normal(1, (rows, ind)) * np.float32(2.0 ** sx), synth.normal(2, (out, ind)) * np.float32(2.0 ** sw)
+    dy = synth.normal(4, (rows, out)) * np.float32(2.0 ** (min(sx, 0) if sw else 0))
+    check(G.linear(x, w, None), x, w.T, "forward")
+    wg, _, dx = G.linear_backward(x, dy, w, np.zeros((out, ind), np.float32), np.zeros(out, np.float32))
+    check(dx, dy, w, "input gradient")
+    check(wg, dy.T, x, "weight gradient", floor=2.0 ** -149 * 64)  # a sum of up to 64 chunks
 
 
 # out (the product's K) with every remainder by 4 and by 16, in rows padded to the next multiple of 4
@@ -149,6 +161,18 @@ def test_attention_values_outside_the_split(hd):
     check_attention(got, q, k, v, heads, 1.0 / np.sqrt(hd), False, f"hd {hd} infinite value")
 
 
+@pytest.mark.parametrize("hd", [32, 40, 64, 128])
+def test_attention_small_operands(hd):
+    """V of the smallest normal floats, and Q and K at opposite ends of the range."""
+    L, heads, scale = 130, 2, 1.0 / np.sqrt(hd)
+    q, k, v = (synth.normal(i, (L, heads * hd)) for i in (4, 5, 6))
+    up, down = np.float32(2.0 ** 112), np.float32(2.0 ** -112)
+    for a, b, c, what in ((q, k, v * np.float32(2.0 ** -122), "V"), (q * up, k * down, v, "K"), (q * down, k * up, v, "Q")):
+        for causal in (False, True):
+            check_attention(G.sdpa(a, b, c, heads, causal=causal, scale=scale), a, b, c, heads, scale, causal,
+                            f"small {what}, hd {hd} causal {causal}")
+
+
 def backward(q, k, v, dout, heads, scale, causal, mask=None, stored=False):
     """cdml_sdpa_bwd; stored: with the workspace that lets the dK/dV pass store dS."""
     L, D = q.shape
@@ -206,15 +230,15 @@ def backward64(q, k, v, dout, heads, scale, allowed, per=8):
     return out
 
 
-def check_backward(got, want, what):
+def check_backward(got, want, what, floor=2.0 ** -126):
+    """floor: values under the smallest normal float may be flushed."""
     for g, (w, bound), name in zip(got, want, ("dQ", "dK", "dV")):
         assert np.array_equal(np.isnan(g), np.isnan(w)), f"{what} {name}: NaNs elsewhere"
         inf = np.isinf(w)
         assert np.array_equal(g[inf], w[inf]), f"{what} {name}: infinities"
         fine = np.isfinite(w)
-        # values under the smallest normal float may be flushed
         with np.errstate(invalid="ignore"):
-            over = np.abs(g.astype(np.float64) - np.where(fine, w, 0.0)) - bound - 2.0 ** -126
+            over = np.abs(g.astype(np.float64) - np.where(fine, w, 0.0)) - bound - floor
         assert np.all(over[fine] <= 0), f"{what} {name}: {np.max(over[fine]):.3g} over the bound"
 
 
@@ -253,6 +277,20 @@ def test_attention_backward_values_outside_the_split(hd):
     want = backward64(q, k, v, dout, heads, scale, tril, per=2)  # what they reach is summed on the fp32 MFMA
     for stored in (False, True):
         check_backward(backward(q, k, v, dout, heads, scale, True, stored=stored), want, f"hd {hd} stored {stored}")
+
+
+@pytest.mark.parametrize("hd", [20, 32, 40, 64])
+def test_attention_backward_small_operands(hd):
+    """Gradients of the smallest normal floats, and V, Q and K of such, keep all their bits."""
+    L, heads, scale = 130, 2, 1.0 / np.sqrt(hd)
+    t = [synth.normal(i, (L, heads * hd)) for i in (1, 2, 3, 4)]
+    tril = np.tril(np.ones((L, L), bool))
+    for small in ((3,), (2,), (0,), (1,)):
+        q, k, v, dout = (x * np.float32(2.0 ** -120) if i in small else x for i, x in enumerate(t))
+        want = backward64(q, k, v, dout, heads, scale, tril)
+        for stored in (False, True):
+            check_backward(backward(q, k, v, dout, heads, scale, True, stored=stored), want,
+                           f"hd {hd} small {'QKVG'[small[0]]} stored {stored}", floor=2.0 ** -149 * L)
 
 
 def backward_saved(q, k, v, dout, batch, heads, rope):
