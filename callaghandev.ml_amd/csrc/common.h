@@ -88,9 +88,11 @@ __device__ __forceinline__ floatx16 mfma32x32x2(float a, float b, floatx16 c) {
 // 1e-8 of its size: nothing next to an element's own rounding error, but the
 // same sign in every element, which a column sum over many rows collects (a
 // bias gradient over 130816 rows had 5.8e-6 instead of 4.5e-7).  The kernels
-// therefore compute every other row and column of a product negated (rows and
-// columns of the operands change their sign as they are split, at no cost),
-// which turns the drift round, and undo the sign at the end.
+// therefore compute every other row and column of a product negated (the operands
+// change their sign as they are split, at no cost), which turns the drift round,
+// and undo the sign at the end; along the queries of the attention output and the
+// keys of dV, whose other operand, the probabilities, is not scaled, every other
+// workgroup does.
 //
 // An infinity, a NaN or a value of 2^112 and more (above the largest bf16 once
 // scaled) leaves inf - inf in m, and a sum of 2^96 and more overflows, so every

@@ -149,7 +149,9 @@ struct KvStage {
     }
   }
 
-  __device__ __forceinline__ void store(char *lds) const {
+  // vscale: the split's scale of V, negative where the workgroup's outputs are
+  // computed negated.
+  __device__ __forceinline__ void store(char *lds, float vscale) const {
     if (kside) {
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
@@ -168,7 +170,7 @@ struct KvStage {
         for (int c = 0; c < 4; ++c) {
           uint32_t h, m, l;
           const float x = r[2 * i][c], y = r[2 * i + 1][c];
-          const float f = c & 1 ? -kSplitScale : kSplitScale;
+          const float f = c & 1 ? -vscale : vscale;
           split_bf16x3(x * f, y * f, h, m, l);
           char *d = lds + dst + vslabs(i) * VSLAB + vgroups(i) * 32 + vcluster(c);
           *reinterpret_cast<uint32_t *>(d) = h;
@@ -231,7 +233,7 @@ constexpr float kFastSumLimit = 4294967296.0f;  // 2^32
 template <int HD, bool VEC>
 __device__ __forceinline__ bool load_q(bf16x8 (&q)[HD / 16][3], const FlashArgs &a, int b, int col0, int qi, int hf) {
   const float *qrow = a.q + ((size_t)b * a.lq + min(qi, a.lq - 1)) * a.ldq + col0;
-  float most = 0.f, least = 1.f;
+  uint32_t most = 0, least = ~0u;  // of |x|, and of 2 |x| - 1 as integers, which leaves zeros out
 #pragma unroll
   for (int s = 0; s < HD / 16; ++s) {
     float x[8];
@@ -249,12 +251,12 @@ __device__ __forceinline__ bool load_q(bf16x8 (&q)[HD / 16][3], const FlashArgs 
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      most = fmaxf(most, fabsf(x[e]));
-      least = fminf(least, x[e] == 0.f ? 1.f : fabsf(x[e]));
+      most = max(most, __float_as_uint(x[e]) & 0x7fffffffu);
+      least = min(least, (__float_as_uint(x[e]) << 1) - 1u);
     }
     split_operand(x, 1.f, q[s]);
   }
-  return __builtin_amdgcn_ballot_w64(most >= 0x1p100f || least < 0x1p-110f) != 0;
+  return __builtin_amdgcn_ballot_w64(most >= (100u + 127u) << 23 || least < (17u << 24) - 1u) != 0;  // 2^100, 2^-110
 }
 
 // The online softmax of one wave's 32 query rows (one per lane % 32) over
@@ -428,16 +430,16 @@ struct OnlineRows {
     warm = !__builtin_amdgcn_ballot_w64(m_run == -INFINITY);
   }
 
-  // Joins the two accumulators and undoes the sign of the odd dims; whether
-  // some row came out non-finite (wave-uniform).
-  __device__ __forceinline__ bool finish() {
+  // Joins the two accumulators and undoes V's scale (unscale) and the sign of the
+  // odd dims; whether some row came out non-finite (wave-uniform).
+  __device__ __forceinline__ bool finish(float unscale) {
     float bad = (l_a + l_b) * 0.f;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         // (adding 0 keeps the zeros of a row without a key positive)
-        oacc[db][r] = fmaf(oacc[db][r] + ocor[db][r], r & 1 ? -kSplitUnscale : kSplitUnscale, 0.f);
+        oacc[db][r] = fmaf(oacc[db][r] + ocor[db][r], r & 1 ? -unscale : unscale, 0.f);
       }
       bad = nonfinite_sum(oacc[db], bad);
     }
@@ -531,7 +533,9 @@ __global__ void __launch_bounds__(FA_THREADS, HD <= 32 ? 3 : (HD <= 64 ? 2 : 1))
   st.load(kbase, vbase, a.ldk, a.ldv, 0, a.lk, a.hd);
   bf16x8 q[HD / 16][3];
   const bool wide = load_q<HD, VEC>(q, a, b, col0, qi, hf);
-  st.store(lds[0]);
+  // Every other workgroup along a head's rows computes its outputs negated (common.h).
+  const float sign = (qt + b) & 1 ? -1.f : 1.f, vscale = sign * kSplitScale;
+  st.store(lds[0], vscale);
   __syncthreads();
 
   const int kend = CAUSAL ? min(q0 + FA_BM, a.lk) : a.lk;
@@ -579,10 +583,10 @@ __global__ void __launch_bounds__(FA_THREADS, HD <= 32 ? 3 : (HD <= 64 ? 2 : 1))
       }
       if (!done) rows.consume(sacc, vop, hf, masked, last_vis, mrow, kb0, a.lk - 1, qi < a.lq);
     }
-    st.store(lds[cur ^ 1]);
+    st.store(lds[cur ^ 1], vscale);
     __syncthreads();
   }
-  if ((rows.finish() || wide) && qw0 < a.lq)
+  if ((rows.finish(sign * kSplitUnscale) || wide) && qw0 < a.lq)
     rows.recompute(a, b, col0, qi, li, hf, CAUSAL ? min(qw0 + 32, a.lk) : a.lk, key_last, mrow);
   rows.store(a, bh, b, qi, col0, hf);
 }

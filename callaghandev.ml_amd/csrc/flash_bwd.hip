@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(BW_THREADS, HD <= 64 ? 2 : 1) flash_bwd_dkdv_k
 //               order in which the score accumulators hold them; four clusters by
 //               d % 4.
 // Odd dims are negated in both (common.h); K and V carry the same sign in the
-// wave's registers, and the stores undo it.  A unit is four dims of two queries:
+// wave's registers, and the stores undo it, as that of dO (gscale).  A unit is four dims of two queries:
 // its pieces are packed along the queries as they are split and repacked along
 // the dims by byte permutes.
 template <int HD, bool VEC>
@@ -463,14 +463,15 @@ struct QgStage {
       }
     }
   }
-  __device__ __forceinline__ void store(char *lds) const {
+  __device__ __forceinline__ void store(char *lds, float gscale) const {
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
+      const float scale = (NU == 1 ? gside : i == 1) ? gscale : kSplitScale;
       char *base = lds + (NU == 1 ? (gside ? TENSOR : 0) : i * TENSOR);
       uint32_t w[3][4];  // [piece][dim]: query `row` in the low half, `row + 1` in the high half
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const float f = c & 1 ? -kSplitScale : kSplitScale;
+        const float f = c & 1 ? -scale : scale;
         split_bf16x3(r[i][0][c] * f, r[i][1][c] * f, w[0][c], w[1][c], w[2][c]);
       }
 #pragma unroll
@@ -515,7 +516,9 @@ struct QgStage {
 // most 2^-134, where exp2 itself drops those below 2^-126.
 //
 // S and dP of odd keys are computed negated, so that the drift of the bf16 MFMA
-// (common.h) cancels in a query's sum of dS over its keys, which has to be zero.
+// (common.h) cancels in a query's sum of dS over its keys, which has to be zero;
+// dK and dV alternate their sign along the keys as well as the dims for the column
+// sums that bias gradients take of them.
 //
 // With STORE_DS (causal, lq == lk) the kernel also writes every dS sub-block
 // it forms, for flash_bwd_dq_ds_kernel: block (query block i, key block j),
@@ -688,9 +691,12 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
   // Sub-blocks wholly before these keys contribute nothing, and keys that all
   // lie past lk take nothing.
   auto active = [&](int qb0) { return kw0 < a.lk && !(CAUSAL && qb0 + 31 < kw0); };
-  // Both operands of S and dP carry the split's scale.
-  const float s_scale = sgn * kSplitUnscale2 * a.scale_log2, dp_scale = sgn * kSplitUnscale2;
-  constexpr float p_scale = 1.f, ds_scale = kSplitScale;
+  // Both operands of S and dP carry the split's scale.  dK of odd keys, and dV of
+  // every other workgroup along a head's rows (through dO), are summed negated.
+  const float gsgn = (kt + b) & 1 ? -1.f : 1.f;
+  const float s_scale = sgn * kSplitUnscale2 * a.scale_log2, dp_scale = sgn * gsgn * kSplitUnscale2;
+  const float ds_scale = sgn * kSplitScale;
+  constexpr float p_scale = 1.f;
 
   auto lse4 = [&](int buf) {
     return [&, buf](int g) { return *reinterpret_cast<const vf4 *>(&Ls[buf][8 * g + 4 * hf]); };
@@ -715,7 +721,7 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       }
     };
     auto stage = [&](int buf) {
-      sg.store(lds[buf]);
+      sg.store(lds[buf], gsgn * kSplitScale);
       if (t < BQ) {
         Ls[buf][t] = lreg;
         Ds[buf][t] = dreg;
@@ -778,7 +784,7 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
     const bool of_v = PAIRED ? role_p : n == 0;
-    const float f = kSplitUnscale / (of_v ? p_scale : ds_scale);
+    const float f = of_v ? gsgn * kSplitUnscale : sgn * kSplitUnscale2;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
 #pragma unroll
@@ -1053,7 +1059,8 @@ struct KtStage {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       uint32_t h, m, l;
-      split_bf16x3(r0[c] * kSplitScale, r1[c] * kSplitScale, h, m, l);
+      const float f = c & 1 ? -kSplitScale : kSplitScale;
+      split_bf16x3(r0[c] * f, r1[c] * f, h, m, l);
       *reinterpret_cast<uint32_t *>(d + cluster(c)) = h;
       *reinterpret_cast<uint32_t *>(d + cluster(c) + plane) = m;
       *reinterpret_cast<uint32_t *>(d + cluster(c) + 2 * plane) = l;
@@ -1084,9 +1091,10 @@ struct KtStage {
 };
 
 // One 32-key block of dQ = dS K: cur is this lane's dS operand, kt its K^T operand
-// of plane 0, first slab of the block.
+// of plane 0, first slab of the block.  Odd queries and odd dims are computed
+// negated (common.h).
 template <int HD>
-__device__ __forceinline__ void dq_block(const vf4 (&cur)[4], const char *kt, int plane, int slab,
+__device__ __forceinline__ void dq_block(const vf4 (&cur)[4], float ds_scale, const char *kt, int plane, int slab,
                                          floatx16 (&dq)[HD / 32], floatx16 (&dqc)[HD / 32]) {
 #pragma unroll
   for (int st = 0; st < 2; ++st) {
@@ -1094,7 +1102,7 @@ __device__ __forceinline__ void dq_block(const vf4 (&cur)[4], const char *kt, in
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = cur[2 * st + (e >> 2)][e & 3];
     bf16x8 ds[3];
-    split_operand(x, kSplitScale, ds);
+    split_operand(x, ds_scale, ds);
 #pragma unroll
     for (int db = 0; db < HD / 32; ++db) {
       bf16x8 k[3];
@@ -1109,14 +1117,17 @@ __device__ __forceinline__ void dq_block(const vf4 (&cur)[4], const char *kt, in
   }
 }
 
-// Joins the two accumulators; whether some row came out non-finite (wave-uniform).
+// Joins the two accumulators and undoes scale and signs (register r holds a query of
+// r's parity, lane li a dim of li's); whether some row came out non-finite
+// (wave-uniform).
 template <int HD>
-__device__ __forceinline__ bool dq_finish(floatx16 (&dq)[HD / 32], const floatx16 (&dqc)[HD / 32]) {
+__device__ __forceinline__ bool dq_finish(floatx16 (&dq)[HD / 32], const floatx16 (&dqc)[HD / 32], int li) {
+  const float f = li & 1 ? -kSplitUnscale2 : kSplitUnscale2;
   float bad = 0.f;
 #pragma unroll
   for (int db = 0; db < HD / 32; ++db) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dq[db][r] = (dq[db][r] + dqc[db][r]) * kSplitUnscale2;
+    for (int r = 0; r < 16; ++r) dq[db][r] = (dq[db][r] + dqc[db][r]) * (r & 1 ? -f : f);
     bad = nonfinite_sum(dq[db], bad);
   }
   return any_nonfinite(bad);
@@ -1198,6 +1209,7 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
   __syncthreads();
 
   const int ko = Stage::operand(li, hf);
+  const float ds_scale = li & 1 ? -kSplitScale : kSplitScale;
   for (int kt = 0; kt < n_kt; ++kt) {
     const int lbuf = kt & 1;
     const int k0 = kt * BN;
@@ -1210,7 +1222,7 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
 #pragma unroll
         for (int i = 0; i < 4; ++i) n2[i] = *reinterpret_cast<const vf4 *>(dsw + (size_t)(j + 2) * 1024 + 4 * i);
       }
-      dq_block<HD>(cur, lds[lbuf] + ko + 2 * kb * Stage::SLAB, Stage::PLANE, Stage::SLAB, dq, dqc);
+      dq_block<HD>(cur, ds_scale, lds[lbuf] + ko + 2 * kb * Stage::SLAB, Stage::PLANE, Stage::SLAB, dq, dqc);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         cur[i] = n1[i];
@@ -1222,7 +1234,7 @@ __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const Bw
   }
 
   if (last < 0) return;
-  if (dq_finish<HD>(dq, dqc)) dq_recompute<HD>(a, kbase, dsw, qi, li, hf, dq);
+  if (dq_finish<HD>(dq, dqc, li)) dq_recompute<HD>(a, kbase, dsw, qi, li, hf, dq);
   RowStore<HD> out;
   out.load(a, qw0, li, hf);
   out.store(a, dq, b, qw0, col0, li, hf);
@@ -1276,6 +1288,7 @@ __global__ void __launch_bounds__(32 * kShortQB, 2) flash_bwd_dq_ds_short_kernel
   }
   __syncthreads();
   const int ko = Stage::operand(li, hf);
+  const float ds_scale = li & 1 ? -kSplitScale : kSplitScale;
 #pragma unroll 1
   for (int pass = 0; pass < 2; ++pass) {
     const int qi = pass == 0 ? nqb - 1 - wave : wave;
@@ -1290,7 +1303,7 @@ __global__ void __launch_bounds__(32 * kShortQB, 2) flash_bwd_dq_ds_short_kernel
       for (int u = 0; u < PF; ++u) {
         const int j = j0 + u;
         if (j > qi) break;
-        dq_block<HD>(buf[u], lds + ko + 2 * j * Stage::SLAB, PLANE, Stage::SLAB, dq, dqc);
+        dq_block<HD>(buf[u], ds_scale, lds + ko + 2 * j * Stage::SLAB, PLANE, Stage::SLAB, dq, dqc);
         fetch(buf[u], qi, j + PF);
       }
     }
@@ -1300,7 +1313,7 @@ __global__ void __launch_bounds__(32 * kShortQB, 2) flash_bwd_dq_ds_short_kernel
 #pragma unroll
       for (int p = 0; p < PF; ++p) fetch(buf[p], wave, p);
     }
-    if (dq_finish<HD>(dq, dqc)) dq_recompute<HD>(a, kbase, dsbh + (size_t)qi * (qi + 1) / 2 * 1024, qi, li, hf, dq);
+    if (dq_finish<HD>(dq, dqc, li)) dq_recompute<HD>(a, kbase, dsbh + (size_t)qi * (qi + 1) / 2 * 1024, qi, li, hf, dq);
     out.store(a, dq, b, 32 * qi, col0, li, hf);
   }
 }

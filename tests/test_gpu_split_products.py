@@ -328,3 +328,35 @@ def test_short_dq_has_the_bits_of_the_tiled_one(L, rope):
     got = backward_saved(*(np.tile(t, (copies, 1)) for t in (q, k, v, dout)), few * copies, heads, rope)
     for g, w, name in zip(got, want, ("dQ", "dK", "dV")):
         assert np.array_equal(g.view(np.uint32), np.tile(w, (copies, 1)).view(np.uint32)), name
+
+
+def drift(err, sign):
+    """Mean of sign * err over the errors' root mean square, in units of what independent errors give."""
+    return abs((err * sign).mean()) / np.sqrt((err ** 2).mean()) * np.sqrt(err.size)
+
+
+def test_errors_do_not_add_up_over_rows():
+    """The bf16 MFMA rounds down; the kernels alternate the signs of rows and columns so that its drift does not
+    collect in sums over rows (bias gradients).  Independent errors give a normal deviate; without the alternation
+    along the rows the drift of dQ is 10 and that of O, alternating with the column, 11."""
+    rows, ind, out = 32768, 64, 64
+    x, w = synth.normal(1, (rows, ind)), synth.normal(2, (out, ind))
+    err = G.linear(x, w, None) - x.astype(np.float64) @ w.astype(np.float64).T
+    alternating = np.where(np.arange(out) % 2, -1.0, 1.0)
+    assert drift(err, 1.0) < 5 and drift(err, alternating) < 5
+    batch, heads, hd, L = 256, 4, 32, 128
+    D, scale = heads * hd, 1.0 / np.sqrt(hd)
+    q, k, v, dout = (synth.normal(i, (batch * L, D)) for i in (1, 2, 3, 4))
+    dq, dk, _ = backward_saved(q, k, v, dout, batch, heads, False)
+    o = G.sdpa(q, k, v, heads, causal=True, scale=scale, batch=batch)
+    Q, K, V, W = (t.reshape(batch, L, heads, hd).transpose(0, 2, 1, 3).astype(np.float64) for t in (q, k, v, dout))
+    s = np.where(np.tril(np.ones((L, L), bool)), Q @ K.swapaxes(2, 3) * scale, -np.inf)
+    p = np.exp(s - s.max(3, keepdims=True))
+    p /= p.sum(3, keepdims=True)
+    O = p @ V
+    ds = p * (W @ V.swapaxes(2, 3) - (W * O).sum(3, keepdims=True))
+    flat = lambda t: t.transpose(0, 2, 1, 3).reshape(-1, D)
+    alternating = np.where(np.arange(D) % 2, -1.0, 1.0)
+    for got, want, name in ((dq, ds @ K * scale, "dQ"), (dk, ds.swapaxes(2, 3) @ Q * scale, "dK"), (o, O, "O")):
+        err = got - flat(want)
+        assert drift(err, 1.0) < 5 and drift(err, alternating) < 5, name
