@@ -1,10 +1,13 @@
 """GPU tests of the products that run as three bf16 pieces per fp32 operand.
 
-Bound: the kernels add eight products per rounding, so a sum over K has at most
-K / 8 + a few roundings of partial sums that never exceed sum |a b|, and the
-left-out products are below 2^-24 of it: |got - exact| <= (K / 8 + 8) 2^-24
-sum |a b|.  A lost third piece (2^-17), a wrong index or a wrong sign is far
-outside it at these K.
+Bounds: the kernels add eight products per rounding, so a sum over K has n = K / 8
+and a few roundings of partial sums that never exceed sum |a b|, and the left-out
+products are below 2^-24 of it: |got - exact| <= (K / 8 + 8) 2^-24 sum |a b|, where
+a wrong index or sign is far outside.  Of operands with independent signs the
+partial sums grow like sqrt(i / n) and the roundings are independent, each at most
+2^-24 / sqrt(3) of its sum in the mean square: the 2-norm of all errors is at most
+2^-24 (sqrt(n / 6) + 2) of the results', which a lost third piece (2^-18) exceeds
+at every shape here (test_split_bounds.py).
 """
 from __future__ import annotations
 
@@ -29,6 +32,9 @@ def check(got, a, b, what, extra=0.0, floor=2.0 ** -149):
     assert np.array_equal(got[inf], np.sign(want[inf]) * np.float32(np.inf)), f"{what}: infinities"
     err = np.abs(got[fine].astype(np.float64) - want[fine])
     assert np.all(err <= bound[fine]), f"{what}: {np.max(err / bound[fine]):.3g} of the bound"
+    if fine.all():
+        part = np.linalg.norm(err) / np.linalg.norm(want) / (2.0 ** -24 * (np.sqrt(a.shape[1] / 48) + 2))
+        assert part <= 1, f"{what}: {part:.3g} of the bound on the 2-norm"
 
 
 # rows, in, out: one tile and its neighbours (63 .. 65, 127 .. 129), ragged k-tiles (K % 16 = 4, 8, 12; K below
@@ -63,6 +69,27 @@ def test_small_operands(rows, ind, out, sx, sw):
     check(wg, dy.T, x, "weight gradient", floor=2.0 ** -149 * 64)  # a sum of up to 64 chunks
 
 
+@pytest.mark.parametrize("rows,ind,hid", [(300, 64, 256), (4099, 256, 512)])
+def test_relu_block_gradients(rows, ind, hid):
+    """A training ReLU block's backward against float64 with the derivatives that the kernel's own output marks, so
+    that no bound has to allow for a pre-activation on either side of 0."""
+    x, w1, b1 = synth.normal(1, (rows, ind)), synth.xavier_uniform(2, hid, ind), synth.normal(3, (hid,))
+    dy, w2 = synth.normal(4, (rows, ind)), synth.xavier_uniform(5, ind, hid)
+    z2, z1 = np.zeros((ind, hid), np.float32), np.zeros((hid, ind), np.float32)
+    h = G.linear_preact_output_only(x, w1, b1, 3)
+    dh, gw2, gb2 = G.linear_backward_act(h, dy, w2, z2, z2[:, 0].copy(), dz=h, act=3 | 0x100)
+    check(gw2, dy.T, h, "second layer's weights")
+    check(gb2[:, None], dy.T, np.ones((rows, 1), np.float32), "second layer's bias")
+    on = ~np.signbit(h)
+    assert not dh[~on].any()
+    exact = (dy.astype(np.float64) @ w2.astype(np.float64)).astype(np.float32)
+    check(np.where(on, dh, exact), dy, w2, "hidden deltas")
+    dx, gw1, gb1 = G.linear_backward_act(x, dh, w1, z1, z1[:, 0].copy())
+    check(dx, dh, w1, "input gradient")
+    check(gw1, dh.T, x, "first layer's weights")
+    check(gb1[:, None], dh.T, np.ones((rows, 1), np.float32), "first layer's bias")
+
+
 # out (the product's K) with every remainder by 4 and by 16, in rows padded to the next multiple of 4
 @pytest.mark.parametrize("rows,ind,out", [(17, 8, 130), (65, 64, 17), (129, 132, 19), (300, 200, 31), (4099, 1024, 45)])
 def test_padded_rows_of_any_width(rows, ind, out):
@@ -94,6 +121,42 @@ def test_values_outside_the_split(rows, ind, out):
     wg, bg, dx = G.linear_backward(x, dy, w, np.zeros((out, ind), np.float32), np.zeros(out, np.float32))
     check(dx, dy, w, "input gradient")
     check(wg, dy.T, x, "weight gradient")
+
+
+# the K-segmented input gradient, on both tile sizes
+@pytest.mark.parametrize("rows,ind,out", [(70, 48, 64), (2100, 1540, 16)])
+def test_backprop_qkv_values_outside_the_split(rows, ind, out):
+    d = [synth.normal(1 + i, (rows, out)) for i in range(3)]
+    w = [synth.normal(4 + i, (out, ind)) for i in range(3)]
+    d[0][3, 5], d[1][9, 0], d[2][20, 7], d[2][41, 11] = np.inf, -np.inf, np.nan, 3.4e38
+    w[2][11] *= np.float32(1e-30)
+    zeros = [t for _ in range(3) for t in (np.zeros((out, ind), np.float32), np.zeros(out, np.float32))]
+    got = G.backprop_qkv(synth.normal(7, (rows, ind)), *d, *w, *zeros)[0]
+    check(got, np.hstack(d), np.vstack(w), "input gradient")
+
+
+@pytest.mark.parametrize("rows,dim,hd", [(70, 64, 16), (2048, 512, 64)])
+def test_rotary_values_outside_the_split(rows, dim, hd):
+    """Q and K are the rotation of what the fp32 sums give, infinities and NaNs included, V the sums."""
+    x = synth.normal(1, (rows, dim))
+    w = [synth.normal(2 + i, (dim, dim)) for i in range(3)]
+    b = [synth.normal(5 + i, (dim,)) for i in range(3)]
+    x[3, 5], x[9, 0], x[20, 7], x[41, 11] = np.inf, -np.inf, np.nan, 3.4e38
+    for t in w:
+        t[:, 11] *= np.float32(1e-30)
+    got = G.project_qkv_rope(x, w[0], b[0], w[1], b[1], w[2], b[2], hd)
+    check(got[2], x, w[2].T, "V", b[2].astype(np.float64))
+    for i in range(2):
+        with np.errstate(all="ignore"):
+            X, W = x.astype(np.float64), w[i].T.astype(np.float64)
+            z = X @ W + b[i]
+            lim = (dim / 8 + 8) * 2.0 ** -24 * (np.abs(X) @ np.abs(W) + np.abs(b[i])) + 2.0 ** -22 * np.abs(z)
+        want = G.rope(z.astype(np.float32), num_heads=dim // hd, head_dim=hd)
+        lim = np.repeat(lim.reshape(rows, -1, 2).sum(2), 2, axis=1)  # the rotation mixes a pair's errors
+        assert np.array_equal(np.isnan(got[i]), np.isnan(want)), "QK"[i]
+        inf, fine = np.isinf(want), np.isfinite(want)
+        assert np.array_equal(got[i][inf], want[inf]), "QK"[i]
+        assert np.all(np.abs(got[i][fine].astype(np.float64) - want[fine]) <= lim[fine]), "QK"[i]
 
 
 def attention64(q, k, v, heads, scale, causal):
@@ -273,10 +336,16 @@ def test_attention_backward_values_outside_the_split(hd):
     dout[31, 3] = np.inf
     dout[70, hd + 5] = 3.4e38  # above the largest bf16
     v[:, hd + 5] *= np.float32(1e-30)
-    tril = np.tril(np.ones((L, L), bool))
-    want = backward64(q, k, v, dout, heads, scale, tril, per=2)  # what they reach is summed on the fp32 MFMA
-    for stored in (False, True):
-        check_backward(backward(q, k, v, dout, heads, scale, True, stored=stored), want, f"hd {hd} stored {stored}")
+    tril, full = np.tril(np.ones((L, L), bool)), np.ones((L, L), bool)
+    drop = synth.uniform(9, L * L).reshape(L, L) < 0.7
+    drop[:, 0] = drop[31] = True  # every query sees a key, and query 31 all that it may
+    for causal, mask in ((True, None), (False, None), (False, drop), (True, drop)):
+        allowed = (tril if causal else full) & (drop if mask is not None else full)
+        # what they reach is summed on the fp32 MFMA
+        want = backward64(q, k, v, dout, heads, scale, allowed, per=2)
+        for stored in (False, True):
+            check_backward(backward(q, k, v, dout, heads, scale, causal, mask, stored=stored and mask is None), want,
+                           f"hd {hd} causal {causal} mask {mask is not None} stored {stored}")
 
 
 @pytest.mark.parametrize("hd", [20, 32, 40, 64])
