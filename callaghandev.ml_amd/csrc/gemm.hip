@@ -87,8 +87,8 @@ __device__ __forceinline__ float swap_pair(float y) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y), 0xB1, 0xF, 0xF, false));
 }
 
-// Epilogue of both forward GEMM kernels with the rotary embedding of
-// AccelerationCPU.cs:4947-4975 folded in.  A lane holds column n of rows
+// Epilogue of the fallback forward kernel (gemm_nt_kernel) with the rotary embedding
+// of AccelerationCPU.cs:4947-4975 folded in.  A lane holds column n of rows
 // mrow0 + 32 i + 8 (r / 4) + 4 hf + r % 4, so the pair partner of column n
 // (n ^ 1; head dims are even) sits in lane li ^ 1 of the same register: one
 // lane swap gives each lane both halves of its pair.  The swap runs in every
@@ -139,14 +139,11 @@ __device__ __forceinline__ void store_rope(const GemmArgs &args, const GemmProbl
     const int pb = seg > 0 ? mb % seg : mb;    // position of row mb in its segment
     if (seg <= 0 || pb + 31 < seg) {
       if (full) {
-        // A whole block inside one segment: positions pos0 + pb + dr (every
-        // one inside the table, which the entry point checks), no predicates,
-        // and per row only wave-uniform offsets from the lane's bases.
-        // The table entries of four rows are loaded before any of their
-        // stores: a load issued after a store waits for it (the memory
-        // counter covers both), which serialised one round trip per element.
-        // (Loading a group ahead, or eight rows at once, takes the kernel past
-        // 128 VGPRs and one of its two workgroups per CU.)
+        // A whole block inside one segment: positions pos0 + pb + dr (every one inside
+        // the table, which the entry point checks), no predicates, and per row only
+        // wave-uniform offsets from the lane's bases.  The table entries of four rows
+        // are loaded before any of their stores: a load issued after a store waits
+        // for it (the memory counter covers both).
         const float2 *__restrict__ csb = args.rope_cs + (size_t)(args.rope_pos0 + pb + 4 * hf) * pairs;
         float *__restrict__ cb = P.c + (size_t)(mb + 4 * hf) * args.ldc;
 #pragma unroll
@@ -1003,8 +1000,8 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
 // rounding of 0 moves a whole row of the layer below's gradient by up to a
 // tenth of its rms when its last bits change; above 16 rows these products keep
 // the bits they have always had.  fp32-equivalent TFLOP/s with z / without:
-// 130816 x 256 -> 1024 112 / 124, 16380 x 1024 -> 4096 136 / 137 (the split
-// kernel has 160-199).
+// 130816 x 256 -> 1024 118 / 127, 16380 x 1024 -> 4096 137 / 138 (the split
+// kernel has 147-195).
 //
 // Both operand tiles sit in LDS as [rows][16] with pitch 20 floats, double
 // buffered; lanes read 16-byte operands that feed four v_mfma_f32_32x32x2_f32
@@ -1012,9 +1009,10 @@ __global__ void __launch_bounds__(64 * WM * WN, MINB) gemm_tile_kernel(const Gem
 // the second half of a k-tile are read while the MFMAs of the first run.  The
 // rows of a wave's 16 are stored in the order 0, 4, 8, 12, 1, 5, ..., whose
 // 64-byte pieces fall in disjoint banks.  The activation is a template argument
-// and the epilogue stores from the accumulators: with a run-time activation
-// behind store_tile, and without the read-ahead, the kernel took 696 instead of
-// 552 us for 130816 x 256 -> 1024 and 92 instead of 79 us for 16384 x 512 -> 512.
+// and the epilogue stores from the accumulators, whole wave blocks without a
+// predicate: with a run-time activation behind store_tile, and without the
+// read-ahead, the kernel took 697 instead of 541 us for 130816 x 256 -> 1024 and 90
+// instead of 78 us for 16384 x 512 -> 512.
 template <int TM, int TN, int WM, int WN, int ACT, bool EPI>
 __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArgs args) {
   constexpr int NT = 64 * WM * WN, BKK = 16, LD = BKK + 4;
@@ -1108,22 +1106,25 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) gemm_f32_kernel(const GemmArg
   // D[i][j] of a block sits at row 8 (r / 4) + 4 hf + r % 4, column li: 32 lanes
   // store 32 consecutive columns of one row.  A launch here has no option but
   // the pre-activation (cdml_linear_preact).
-  const bool whole = mw + TM / WM <= M && nw + TN / WN <= N;  // wave-uniform
   float *cb = P.c + (size_t)(mw + 4 * hf) * args.ldc + nw + li;
   float *pb = EPI ? args.pre + (size_t)(mw + 4 * hf) * args.ldpre + nw + li : nullptr;
+  auto store = [&](auto whole) {
 #pragma unroll
-  for (int i = 0; i < BI; ++i)
+    for (int i = 0; i < BI; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = i * 32 + 8 * (r >> 2) + (r & 3);
+      for (int r = 0; r < 16; ++r) {
+        const int d = i * 32 + 8 * (r >> 2) + (r & 3);
 #pragma unroll
-      for (int j = 0; j < BJ; ++j) {
-        if (!whole && (mw + 4 * hf + d >= M || nw + j * 32 + li >= N)) continue;
-        const float z = acc[i][j][r] + bias[j];
-        if (EPI) pb[(size_t)d * args.ldpre + j * 32] = z;
-        cb[(size_t)d * args.ldc + j * 32] = activate(z, ACT);
+        for (int j = 0; j < BJ; ++j) {
+          if (!decltype(whole)::value && (mw + 4 * hf + d >= M || nw + j * 32 + li >= N)) continue;
+          const float z = acc[i][j][r] + bias[j];
+          if (EPI) pb[(size_t)d * args.ldpre + j * 32] = z;
+          cb[(size_t)d * args.ldc + j * 32] = activate(z, ACT);
+        }
       }
-    }
+  };
+  if (mw + TM / WM <= M && nw + TN / WN <= N) store(std::true_type{});  // wave-uniform
+  else store(std::false_type{});
 }
 
 // Few rows (decode steps, short batches: M <= MR), non-transposed operands,
