@@ -98,7 +98,10 @@ __device__ __forceinline__ floatx16 mfma32x32x2(float a, float b, floatx16 c) {
 // scaled) leaves inf - inf in m, and a sum of 2^96 and more overflows, so every
 // result that one reaches comes out non-finite; the kernels test their results for
 // that (any_nonfinite) and recompute such blocks with mfma32x32x2, whose
-// infinities and NaNs are those of the fp32 sum.
+// infinities and NaNs are those of the fp32 sum.  That walks K serially from memory:
+// one NaN takes a 16384 x 1024 -> 4096 product from 0.79 to 1.5 ms, its input gradient
+// from 0.78 to 2.8, its weight gradient from 0.71 to 6.3, and an attention backward of
+// 4 x 4096 from 2.3 to 9.3.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t vu2 __attribute__((ext_vector_type(2)));
 typedef uint32_t vu4 __attribute__((ext_vector_type(4)));

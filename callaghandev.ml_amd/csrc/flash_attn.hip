@@ -15,12 +15,14 @@
 //                   one swap between the two half-waves.
 //   online softmax  running max / sum per query in the exp2 domain
 //                   (scale * log2 e folded into Q), masked keys -inf.
-//   O^T += V^T P^T  V is scaled for the split (common.h), the probabilities are not:
-//                   one below 2^-110 loses at most 2^-134, where exp2 itself drops
-//                   those below 2^-126.  Accumulators 8 s .. 8 s + 7 of a lane hold the keys 16 s +
+//   O^T += V^T P^T  accumulators 8 s .. 8 s + 7 of a lane hold the keys 16 s +
 //                   {4 h .. 4 h + 3, 8 + 4 h .. 8 + 4 h + 3} (h = lane / 32): V is
 //                   staged transposed with its keys in that order, so the
-//                   probabilities are consumed in place.
+//                   probabilities are consumed in place.  V carries the split's
+//                   scale (common.h), the probabilities do not (16 more VALU
+//                   instructions per sub-block, 1-5% of the kernel): one below
+//                   2^-110 loses at most 2^-134, where exp2 itself drops those
+//                   below 2^-126.
 //
 // Causal: tiles entirely above the diagonal are never loaded; a wave skips
 // MFMA work for its 32-key sub-blocks that lie wholly in its future; heavy
@@ -28,12 +30,11 @@
 // with sum 0 and is written as 0 (AccelerationCPU.cs:1908-1911).
 //
 // What bounds it: at head dim 64 a 32 x 32 sub-block costs a wave 48 MFMAs
-// (1536 cycles of the matrix pipe) and about 250 VALU instructions (half of them
-// the two splits), at head dim 32 half the MFMAs and 210: the vector units there.
-// Measured on MI355X: the causal layer 4 x 4096, 16 heads of 64, of which this
-// kernel is half, 1750 -> 1560 us against the same kernel on the fp32 MFMA; the
-// matrix pipes are busy 61% of its cycles at head dim 64 and 45% at 32 (vector
-// units 55% and 73%).
+// (1536 cycles of the matrix pipe) and some 290 other VALU instructions, half of
+// them the splits (5.96 per MFMA at 4 x 4096); at head dim 32 half the MFMAs and 280
+// (11.8 per MFMA): the vector units there.  Measured on MI355X at 4 x 4096, 16 heads
+// of 64: 0.69 ms (1.05 ms on the fp32 MFMA), matrix pipes 57% busy; 256 x 512, 8 heads
+// of 32: 0.25 ms, 39%.  LDS bank conflicts take 11% of the active cycles at 4 x 4096.
 #include <cfloat>
 
 #include "common.h"

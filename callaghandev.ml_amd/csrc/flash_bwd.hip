@@ -207,8 +207,9 @@ __device__ __forceinline__ void store_column(const BwdArgs &a, const floatx16 (&
 // wave's keys need 384 registers there.  Workgroup i takes (sequence, head)
 // i % n_bh and key tile i / n_bh: under the causal rule the first key tiles are
 // seen by the most queries, so the heaviest tiles go out first on every XCD.
-template <int HD, int BQ, bool CAUSAL, bool HAS_MASK, bool VEC>
-__global__ void __launch_bounds__(BW_THREADS, HD <= 64 ? 2 : 1) flash_bwd_dkdv_kernel(const BwdArgs a) {
+template <int HD, bool CAUSAL, bool HAS_MASK, bool VEC>
+__global__ void __launch_bounds__(BW_THREADS, 1) flash_bwd_dkdv_kernel(const BwdArgs a) {
+  constexpr int BQ = 32;
   constexpr int NQB = BQ / 32;  // 32-query sub-blocks per tile
   constexpr int NDB = HD / 32;  // 32-wide head-dim blocks of dK^T / dV^T
   constexpr int NKG = HD / 8;   // 8-dim groups of the Q.K and dO.V products
@@ -415,9 +416,9 @@ __global__ void __launch_bounds__(BW_THREADS, HD <= 64 ? 2 : 1) flash_bwd_dkdv_k
 //               order in which the score accumulators hold them; four clusters by
 //               d % 4.
 // Odd dims are negated in both (common.h); K and V carry the same sign in the
-// wave's registers, and the stores undo it, as that of dO (gscale).  A unit is four dims of two queries:
-// its pieces are packed along the queries as they are split and repacked along
-// the dims by byte permutes.
+// wave's registers, and the stores undo it, as that of dO (gscale).  A unit is four
+// dims of two queries: its pieces are packed along the queries as they are split and
+// repacked along the dims by byte permutes.
 template <int HD, bool VEC>
 struct QgStage {
   static constexpr int CH = HD / 4;
@@ -502,15 +503,16 @@ struct QgStage {
 // Head dim 64: a pair of waves owns 32 keys.  Wave w (0..3) holds K's pieces,
 // forms S and P and sums dV; wave w + 4 holds V's, forms dP, takes P through LDS,
 // forms and stores dS and sums dK.  A pair shares a SIMD, so one wave's
-// exponentials and splits run under the other's products, and each needs 221
+// exponentials and splits run under the other's products, and each needs 224
 // registers (one wave for both needs 470 and is alone on its SIMD: 35% of the
-// cycles in the matrix pipes, paired 47%).  Per 32-query tile, two barriers: P is
+// cycles in the matrix pipes, paired 45%).  Per 32-query tile, two barriers: P is
 // written before the first, read after it.  Head dim 32: one wave does both in
-// 246 registers, two workgroups to a CU; pairs took 31% longer there, half the
+// 250 registers, two workgroups to a CU; pairs took 31% longer there, half the
 // products per barrier.
-// 4 x 4096 x 16 heads x 64, whole backward: 5.13 -> 3.92 ms; 511 x 256 x 8 x 32:
-// 2.33 -> 1.93 ms (this kernel 1.40 -> 1.05 ms), bound by the exponentials and splits
-// between the products: vector ALU 48% of the cycles, matrix pipes 34%.
+// Measured on MI355X: 4 x 4096, 16 heads of 64, 1.69 ms (2.19 on the fp32 MFMA); 256 x
+// 511, 8 heads of 32, 0.65 ms (0.77).  Bound by the exponentials and splits between
+// the products: 5.1 and 10.2 VALU instructions beside each MFMA, matrix pipes 45% and
+// 30% busy.
 //
 // All operands but P carry the split's scale; a probability below 2^-110 loses at
 // most 2^-134, where exp2 itself drops those below 2^-126.
@@ -1160,7 +1162,7 @@ __device__ __forceinline__ void dq_recompute(const BwdArgs &a, const float *kbas
 // w; for its key blocks j <= i the dS operand (dS[q][2s + c], s = 0..15, in lane
 // (q, c)) is 16 contiguous floats per lane, loaded two blocks ahead, and K^T
 // streams through double-buffered LDS as the other operand.  The blocks' bytes
-// bound it: 2.1 GB at 4 x 4096 x 16 heads.
+// bound it: 2.1 GB in 0.60 ms at 4 x 4096, 16 heads of 64.
 template <int HD, int BN>
 __global__ void __launch_bounds__(BW_THREADS, 2) flash_bwd_dq_ds_kernel(const BwdArgs a) {
   constexpr int NKB = BN / 32;
@@ -1434,7 +1436,7 @@ int zero_rows(float *p, long long rows, int cols, int ld, hipStream_t st) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-template <int HD, int BQ, int BN, bool CAUSAL, bool HAS_MASK, bool VEC>
+template <int HD, int BN, bool CAUSAL, bool HAS_MASK, bool VEC>
 void launch_bwd(BwdArgs &a, hipStream_t st) {
   const int n_bh = a.batch * a.heads;
   const int kt = (a.lk + BW_TILE - 1) / BW_TILE;
@@ -1458,27 +1460,27 @@ void launch_bwd(BwdArgs &a, hipStream_t st) {
     }
     flash_bwd_dkdv_split_kernel<HD, CAUSAL, HAS_MASK, VEC, false><<<kgrid, kblock, 0, st>>>(a);
   } else {
-    flash_bwd_dkdv_kernel<HD, BQ, CAUSAL, HAS_MASK, VEC><<<kgrid, block, 0, st>>>(a);
+    flash_bwd_dkdv_kernel<HD, CAUSAL, HAS_MASK, VEC><<<kgrid, block, 0, st>>>(a);
   }
   flash_bwd_dq_kernel<HD, BN, CAUSAL, HAS_MASK, VEC><<<qgrid, block, 0, st>>>(a);
 }
 
-template <int HD, int BQ, int BN, bool VEC>
+template <int HD, int BN, bool VEC>
 void launch_bwd_mode(BwdArgs &a, bool causal, hipStream_t st) {
   if (causal) {
-    if (a.mask) launch_bwd<HD, BQ, BN, true, true, VEC>(a, st);
-    else launch_bwd<HD, BQ, BN, true, false, VEC>(a, st);
+    if (a.mask) launch_bwd<HD, BN, true, true, VEC>(a, st);
+    else launch_bwd<HD, BN, true, false, VEC>(a, st);
   } else if (a.mask) {
-    launch_bwd<HD, BQ, BN, false, true, VEC>(a, st);
+    launch_bwd<HD, BN, false, true, VEC>(a, st);
   } else {
-    launch_bwd<HD, BQ, BN, false, false, VEC>(a, st);
+    launch_bwd<HD, BN, false, false, VEC>(a, st);
   }
 }
 
-template <int HD, int BQ, int BN>
+template <int HD, int BN>
 void launch_bwd_hd(BwdArgs &a, bool causal, bool vec, hipStream_t st) {
-  if (vec) launch_bwd_mode<HD, BQ, BN, true>(a, causal, st);
-  else launch_bwd_mode<HD, BQ, BN, false>(a, causal, st);
+  if (vec) launch_bwd_mode<HD, BN, true>(a, causal, st);
+  else launch_bwd_mode<HD, BN, false>(a, causal, st);
 }
 
 }  // namespace
@@ -1660,9 +1662,9 @@ int sdpa_bwd_impl(const float *q, int ldq, const float *k, int ldk, const float 
       a.ds_bh = (long long)(extra / sizeof(float) / bh);
     }
   }
-  if (hd_pad == 32) launch_bwd_hd<32, 64, 64>(a, causal != 0, vec, st);
-  else if (hd_pad == 64) launch_bwd_hd<64, 64, 32>(a, causal != 0, vec, st);
-  else launch_bwd_hd<128, 32, 32>(a, causal != 0, vec, st);
+  if (hd_pad == 32) launch_bwd_hd<32, 64>(a, causal != 0, vec, st);
+  else if (hd_pad == 64) launch_bwd_hd<64, 32>(a, causal != 0, vec, st);
+  else launch_bwd_hd<128, 32>(a, causal != 0, vec, st);
   return check_launch("flash_bwd_dkdv_kernel / flash_bwd_dq_kernel");
 }
 

@@ -739,13 +739,13 @@ __device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &
 // barrier, and the split (VALU) and LDS instructions are spread between the
 // MFMAs by scheduling groups; with NB = 2 (small tiles) several workgroups per
 // CU hide each other's staging.  Measured on MI355X, 128 x 128 tiles
-// (fp32-equivalent TFLOP/s, forward, dX and dW of 16384 x 4096 x 1024): 194, 182
-// and 183, where the fp32 MFMA form that this replaces had 138, 128 and 131.  The
+// (fp32-equivalent TFLOP/s, forward, dX and dW of 16384 x 4096 x 1024): 190, 183
+// and 193, where the fp32 MFMA form that this replaces had 138, 128 and 131.  The
 // library's own bf16 product reaches 1170-1340 TFLOP/s, a sixth of which is
 // 195-223: the power of the matrix cores bounds both (a loop of MFMAs alone on
-// random data runs at 1.8 of 2.4 GHz; on zeros this kernel takes 274).  256 x 256
-// tiles would take 208-229 with one accumulator (see common.h); the registers do
-// not hold two.
+// random data runs at 1.8 of 2.4 GHz); matrix pipes 58-63% busy forward, 5.4-5.6
+// VALU instructions beside each MFMA.  256 x 256 tiles would take 208-229 with one
+// accumulator (see common.h); the registers do not hold two.
 //
 // With TA and a bias-gradient pointer, the workgroups of the first column
 // tile also sum the opA values that they stage (every k once) and add the row

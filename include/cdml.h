@@ -158,8 +158,10 @@ int cdml_project_qkv(const float *x, const float *wq, const float *bq,
  * x [rows, in_dim] with row stride ldx; w [out_dim, in_dim]; b [out_dim] or
  * NULL; y [rows, out_dim] with row stride ldy; activation CDML_ACT_*.
  * Matrix products here and below take fp32 operands as three bf16 pieces each
- * (24 bits, exact) and sum six products in fp32, at no larger error than fp32
- * sums; infinities, NaNs and overflows come out as in fp32. */
+ * (all 24 bits, down to the smallest floats) and sum six products in fp32, at
+ * no larger error than fp32 sums; infinities, NaNs and overflows come out as
+ * in fp32.  Blocks that one of these, a value of 2^112 or a sum of 2^96
+ * reaches are computed a second time in fp32, several times slower. */
 int cdml_linear(const float *x, int ldx, const float *w, const float *b,
                 float *y, int ldy, int rows, int in_dim, int out_dim,
                 int activation, cdml_stream stream);

@@ -48,7 +48,7 @@ import bench  # noqa: E402  (TRAFFIC_SOURCES, source_digest)
 
 PROFILES = os.path.join(ROOT, "profiles")
 PASSES = ("trace", "traffic", "counters", "trainc5", "backward", "train", "c1")
-COUNTERS_A = ("GRBM_GUI_ACTIVE SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES SQ_INSTS_VALU_MFMA_F32 "
+COUNTERS_A = ("GRBM_GUI_ACTIVE SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES SQ_INSTS_MFMA "
               "SQ_INSTS_VALU SQ_INSTS_VALU_TRANS_F32 SQ_INSTS_LDS SQ_LDS_BANK_CONFLICT")
 COUNTERS_B = ("GRBM_GUI_ACTIVE SQ_WAVES SQ_WAVE_CYCLES SQ_WAIT_ANY SQ_WAIT_INST_ANY SQ_ACTIVE_INST_VALU "
               "SQ_ACTIVE_INST_LDS SQ_WAIT_INST_LDS")
@@ -249,7 +249,7 @@ def counter_table(out, tag, bench_args, keep, with_traffic=False):
         ca, cb = a[key], b.get(key, {})
         act = mean(ca["GRBM_GUI_ACTIVE"]) / N_XCC
         busy = mean(ca["SQ_VALU_MFMA_BUSY_CYCLES"]) / N_SIMD
-        mf = mean(ca["SQ_INSTS_VALU_MFMA_F32"])
+        mf = mean(ca["SQ_INSTS_MFMA"])
         valu = mean(ca["SQ_INSTS_VALU"]) - mf
         trans = mean(ca["SQ_INSTS_VALU_TRANS_F32"])
         lds = mean(ca["SQ_INSTS_LDS"])
@@ -269,8 +269,8 @@ def counter_table(out, tag, bench_args, keep, with_traffic=False):
 
 
 COUNTER_NOTE = ("`GRBM_GUI_ACTIVE` is summed over the 8 XCCs (divided by 8); `SQ_VALU_MFMA_BUSY_CYCLES` is "
-                "summed over the 1024 SIMDs (divided by 1024) and reads 64 cycles per "
-                "`v_mfma_f32_32x32x2_f32`; `SQ_INSTS_VALU` includes the MFMAs, which are subtracted; "
+                "summed over the 1024 SIMDs (divided by 1024) and reads 32 cycles per "
+                "`v_mfma_f32_32x32x16_bf16`, 64 per `v_mfma_f32_32x32x2_f32`; `SQ_INSTS_VALU` includes the MFMAs, which are subtracted; "
                 "`SQ_WAIT_INST_ANY` / `SQ_WAVE_CYCLES` is the share of a wave's life spent with an "
                 "instruction waiting to issue (other waves hold the SIMD, or a dependency).  Durations are "
                 "under counter collection, which lengthens them.")
@@ -319,6 +319,10 @@ def pass_backward(out):
             f"and {rc.get('ms')} ms.")
     write("mha_backward_c3_kernel_stats.md",
           header("Kernel durations: c3 MHA layer backward", [cmd], note) + "\n" + stats_table(read_stats(d)) + "\n")
+    cmds, rows = counter_table(out, "bwdc3", ["--only", "c3_mha_layer_backward"], ["flash_bwd", "bwd_delta", "gemm_"])
+    write("mha_backward_c3_counters.md",
+          header("Counters of the c3 MHA layer backward", cmds, "Per dispatch of the kernels of the same leg.  " +
+                 COUNTER_NOTE) + "\n" + "\n".join(rows) + "\n")
 
 
 TRAIN_LEGS = {
