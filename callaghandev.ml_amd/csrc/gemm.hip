@@ -738,9 +738,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &
 // multiplied, so the operands of its first product are read before the
 // barrier, and the split (VALU) and LDS instructions are spread between the
 // MFMAs by scheduling groups; with NB = 2 (small tiles) several workgroups per
-// CU hide each other's staging.  Measured on MI355X, 128 x 128 tiles
-// (fp32-equivalent TFLOP/s, forward, dX and dW of 16384 x 4096 x 1024): 190, 183
-// and 193, where the fp32 MFMA form that this replaces had 138, 128 and 131.  The
+// CU hide each other's staging.  Measured on MI355X (fp32-equivalent TFLOP/s,
+// forward, dX and dW of 16384 x 4096 x 1024): 199, 183 and 193, where the fp32 MFMA form that this replaces had 138, 128 and 131.  The
 // library's own bf16 product reaches 1170-1340 TFLOP/s, a sixth of which is
 // 195-223: the power of the matrix cores bounds both (a loop of MFMAs alone on
 // random data runs at 1.8 of 2.4 GHz); matrix pipes 58-63% busy forward, 5.4-5.6
@@ -1691,16 +1690,27 @@ bool stage_ok(const float *p, int rows, int ld, bool T) {
   return (unsigned long long)rows * ld < (1ull << 32);
 }
 
-// 128 x 128 tiles (two workgroups per CU) where they give three quarters of
-// the CUs one, 64 x 64 otherwise, four times as many (dX, us): 4096 x 1024 x 1024, 256
-// tiles of 128 x 128: 64 against 69; 2048 x 1024 x 1024, 128 tiles: 62 against 54;
-// 512 x 1024 x 1024: 54 against 44.
-// (256 x 128 with eight waves, one workgroup per CU, is 1-3% faster than 128 x
-// 128 forward and 2-8% slower in both gradients, whose short k-loops and long
-// epilogues another workgroup has to cover.)
+// Forward products of many rows take 256 x 128 tiles (eight waves, one workgroup per
+// CU), which split a quarter less per product: us against 128 x 128, 16384 x 1024 ->
+// 4096 690 / 726, 16384 x 512 -> 512 50.6 / 53.7, 130816 x 256 -> 1024 453 / 459.  A last
+// round that is less than three quarters full costs more than that until it is one
+// of seven (5000 x 1000 -> 2000, 1.25 rounds: 148 / 133).  Both gradients are 2-8%
+// slower so: their short k-loops and long epilogues want another workgroup beside.
+inline bool wide_tiles(const GemmArgs &g) {
+  const int cus = num_cus();
+  const long long tiles = (long long)((g.M + 255) / 256) * ((g.N + 127) / 128) * g.nprob, rest = tiles % cus;
+  return g.M >= 2048 && tiles > 0 && (rest == 0 || 4 * rest >= 3LL * cus || tiles >= 6LL * cus);
+}
+
+// Else 128 x 128 tiles (two workgroups per CU) where they give three quarters of the
+// CUs one, 64 x 64 otherwise, four times as many (dX, us): 4096 x 1024 x 1024, 256 tiles
+// of 128 x 128: 64 against 69; 2048 x 1024 x 1024, 128 tiles: 62 against 54; 512 x 1024 x
+// 1024: 54 against 44.
 template <bool TA, bool TB>
 int launch_tiled(GemmArgs &g, hipStream_t stream) {
   const long long tiles = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.nprob * std::max(g.ksplit, 1);
+  if constexpr (!TA && !TB)
+    if (wide_tiles(g)) return launch_tile<256, 128, 4, 2, 2, 3, TA, TB>(g, stream);
   if (4 * tiles >= 3LL * num_cus()) return launch_tile<128, 128, 2, 2, 2, 3, TA, TB>(g, stream);
   // Four waves forward: a launch of few workgroups is bound by the splits between a
   // wave's products (520 x 512 -> 512 21.5 -> 16.3 us, 200 x 1024 -> 1024 37.4 -> 27.6).

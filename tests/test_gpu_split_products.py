@@ -57,6 +57,34 @@ def test_forward_and_gradients(rows, ind, out):
     check(bg[:, None], dy.T, np.ones((rows, 1), np.float32), "bias gradient", bg0.astype(np.float64)[:, None])
 
 
+def test_wide_tiles():
+    """512 tiles of 256 x 128, two whole rounds of 256 CUs, with ragged rows, columns and last k-tile; a few more rows
+    make a short third round and leave the product to 128 x 128 tiles, which have the same bits."""
+    rows, ind, out = 16300, 36, 1000
+    x, w, b = synth.normal(1, (rows, ind)), synth.normal(2, (out, ind)), synth.normal(3, (out,))
+    y = G.linear(x, w, b)
+    check(y, x, w.T, "forward", b.astype(np.float64))
+    z, h = G.linear_preact(x, w, b, 5)  # swish, with its pre-activation
+    assert np.array_equal(z, y)
+    more = G.linear(np.vstack([x, x[:300]]), w, b)
+    assert np.array_equal(more[:rows], y)
+
+
+def test_wide_tiles_rotary():
+    """252 tiles of 256 x 128 (one round) against the same rows in three launches of smaller tiles."""
+    rows, dim, hd, seg = 10700, 256, 32, 1070
+    x = synth.normal(1, (rows, dim))
+    w = [synth.normal(2 + i, (dim, dim)) for i in range(3)]
+    b = [synth.normal(5 + i, (dim,)) for i in range(3)]
+    args = (w[0], b[0], w[1], b[1], w[2], b[2], hd)
+    got = G.project_qkv_rope(x, *args, seg_len=seg)
+    check(got[2], x, w[2].T, "V", b[2].astype(np.float64))
+    for i in (0, 4280, 9630):
+        part = G.project_qkv_rope(x[i:i + seg], *args)
+        for g, p in zip(got, part):
+            assert np.array_equal(g[i:i + seg], p)
+
+
 @pytest.mark.parametrize("sx,sw", [(-124, 0), (0, -124), (-60, -60), (90, -110)])
 @pytest.mark.parametrize("rows,ind,out", [(70, 48, 72), (300, 100, 200), (2100, 64, 1540)])
 def test_small_operands(rows, ind, out, sx, sw):
