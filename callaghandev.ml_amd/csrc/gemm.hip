@@ -742,8 +742,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &args, const TileOut &
 // forward, dX and dW of 16384 x 4096 x 1024): 199, 183 and 193, where the fp32 MFMA form that this replaces had 138, 128 and 131.  The
 // library's own bf16 product reaches 1170-1340 TFLOP/s, a sixth of which is
 // 195-223: the power of the matrix cores bounds both (a loop of MFMAs alone on
-// random data runs at 1.8 of 2.4 GHz); matrix pipes 58-63% busy forward, 5.4-5.6
-// VALU instructions beside each MFMA.  256 x 256 tiles would take 208-229 with one
+// random data runs at 1.8 of 2.4 GHz); matrix pipes 60-64% busy forward, 4.3-4.5
+// VALU instructions beside each MFMA (128 x 128 tiles 58-63%, 5.4-5.6).  256 x 256 tiles would take 208-229 with one
 // accumulator (see common.h); the registers do not hold two.
 //
 // With TA and a bias-gradient pointer, the workgroups of the first column
