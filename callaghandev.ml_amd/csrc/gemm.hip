@@ -421,7 +421,8 @@ __global__ void __launch_bounds__(NTHREADS) gemm_nt_kernel(const GemmArgs args) 
 //     per thread, NP = 1, a wave's rows fall in both clusters).
 //   T = true:  the source is [K][rows] (rows contiguous, k-row stride ld): a
 //     unit is four rows of two k, two 16-byte loads and per row (NC = 4) a
-//     4-byte store per plane, 256 contiguous bytes for eight units.
+//     4-byte store per plane, 256 contiguous bytes for eight units.  Where a
+//     tile has fewer units than threads, the first UNITS threads stage it.
 // The clusters start 16, 128 and 144 bytes past a multiple of 256, so that
 // the 16-byte pieces of sixteen lanes of an operand read fall in different
 // banks.  Each thread's offsets are fixed for the whole K loop; rows past the
@@ -439,11 +440,12 @@ struct OpStage {
   static constexpr int PLANE = NC * ROWB + (T ? 256 : 64);  // bytes of one piece
   static constexpr int BYTES = 3 * PLANE;
   static constexpr int BLOCK = 32 / NC * 32;               // bytes between 32-row blocks
-  static constexpr int NP = ROWS * (T ? 2 : 4) / NT;       // units per thread
+  static constexpr int UNITS = ROWS * (T ? 2 : 4);
+  static constexpr int NP = UNITS < NT ? 1 : UNITS / NT;   // units per thread, of the first UNITS threads
   static constexpr int NV = T ? 2 * NP : NP;               // their loads
   static constexpr int SPLITS = 2 * NV;                    // split_bf16x3 calls
   static constexpr int STORES = T ? 12 * NP : 3 * NP;
-  static_assert(NP >= 1 && ROWS * (T ? 2 : 4) % NT == 0 && (T || NP % 2 == 0 || NP == 1), "staging shape");
+  static_assert(UNITS < NT ? T && UNITS % 64 == 0 : UNITS % NT == 0 && (T || NP % 2 == 0 || NP == 1), "staging shape");
   uint32_t off[NP];
   vf4 v[NV];
   int sa, sb;  // T = false: (row pair, first k / 4); T = true: (row group, k / 2)
@@ -466,6 +468,11 @@ struct OpStage {
       else
         off[i] = (uint32_t)min(row0 + unit_row(i), rows - 1) * (uint32_t)ld + 4 * sb;
     }
+  }
+  // Whether this wave has units.  One without loads rows past the tile (clamped) and
+  // stores nothing: a conditional load would put the staging registers into scratch.
+  static __device__ __forceinline__ bool staging() {
+    return UNITS >= NT || __builtin_amdgcn_readfirstlane(threadIdx.x) < UNITS;
   }
   // First element of k-tile kt.
   static __device__ __forceinline__ const float *tile(const float *x, int kt, int ld) {
@@ -506,6 +513,7 @@ struct OpStage {
   // scale: kSplitScale or its negative.
   __device__ __forceinline__ void store(char *lds, float scale) const {
     auto scaled = [&](float x, bool neg) { return x * (neg ? -scale : scale); };
+    if (!staging()) return;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       if constexpr (T) {
@@ -1712,10 +1720,11 @@ int launch_tiled(GemmArgs &g, hipStream_t stream) {
   if constexpr (!TA && !TB)
     if (wide_tiles(g)) return launch_tile<256, 128, 4, 2, 2, 3, TA, TB>(g, stream);
   if (4 * tiles >= 3LL * num_cus()) return launch_tile<128, 128, 2, 2, 2, 3, TA, TB>(g, stream);
-  // Four waves forward: a launch of few workgroups is bound by the splits between a
-  // wave's products (520 x 512 -> 512 21.5 -> 16.3 us, 200 x 1024 -> 1024 37.4 -> 27.6).
-  // A transposed operand has units for two waves only.
-  if constexpr (!TA && !TB) return launch_tile<64, 64, 2, 2, 3, 2, TA, TB>(g, stream);
+  // Four waves where A runs along K: a launch of few workgroups is bound by the splits
+  // between a wave's products (520 x 512 -> 512 forward 21.5 -> 16.3 us, dX 24.8 -> 19.8;
+  // 200 x 1024 -> 1024 37.4 -> 27.6 and 44 -> 34).  A transposed operand has units for two
+  // of them only.
+  if constexpr (!TA) return launch_tile<64, 64, 2, 2, 3, 2, TA, TB>(g, stream);
   return launch_tile<64, 64, 2, 1, 3, 2, TA, TB>(g, stream);
 }
 
