@@ -459,12 +459,17 @@ struct QgStage {
           r[i][x] = *reinterpret_cast<const vf4 *>(p);
         } else {
 #pragma unroll
-          for (int c = 0; c < 4; ++c) r[i][x][c] = col + c < hd ? p[c] : 0.f;
+          for (int c = 0; c < 4; ++c) r[i][x][c] = p[min(c, hd - 1 - col)];
         }
       }
     }
   }
-  __device__ __forceinline__ void store(char *lds, float gscale) const {
+  // Without VEC, columns at or past hd were read from column hd - 1 and count as zero
+  // through their factor: a select at the load, with the factor behind it, is scheduled
+  // beside the load and waits for it (42 x 3528, one head of 40: 943 against 820 us
+  // causal, 1843 against 1544 not). A column hd - 1 that is not finite makes NaN of them,
+  // in a row whose own pieces hold NaN already: the recompute below reads them as zeros.
+  __device__ __forceinline__ void store(char *lds, float gscale, int hd) const {
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
       const float scale = (NU == 1 ? gside : i == 1) ? gscale : kSplitScale;
@@ -472,7 +477,7 @@ struct QgStage {
       uint32_t w[3][4];  // [piece][dim]: query `row` in the low half, `row + 1` in the high half
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const float f = c & 1 ? -scale : scale;
+        const float f = VEC || col + c < hd ? (c & 1 ? -scale : scale) : 0.f;
         split_bf16x3(r[i][0][c] * f, r[i][1][c] * f, w[0][c], w[1][c], w[2][c]);
       }
 #pragma unroll
@@ -723,7 +728,7 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       }
     };
     auto stage = [&](int buf) {
-      sg.store(lds[buf], gsgn * kSplitScale);
+      sg.store(lds[buf], gsgn * kSplitScale, a.hd);
       if (t < BQ) {
         Ls[buf][t] = lreg;
         Ds[buf][t] = dreg;

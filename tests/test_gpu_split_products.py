@@ -353,15 +353,16 @@ def test_attention_backward(hd, L):
             check_backward(backward(q, k, v, dout, heads, scale, causal, stored=True), want, what + " stored dS")
 
 
-@pytest.mark.parametrize("hd", [32, 64])
-def test_attention_backward_values_outside_the_split(hd):
+# the scalar loads of head dims 20 and 40 read the last column for those past it
+@pytest.mark.parametrize("hd,col", [(32, 3), (64, 3), (20, 19), (40, 39)])
+def test_attention_backward_values_outside_the_split(hd, col):
     """An infinite and a huge output gradient: the keys they reach get what the fp32 products give, the others
     their values."""
     L, heads, scale = 130, 2, 1.0 / np.sqrt(hd)
     q, k, v, dout = (synth.normal(i, (L, heads * hd)) for i in (1, 2, 3, 4))
     # Query 31 sees all of the first 32 keys, in the first head.  (A masked pair of the same 32 x 32 block has weight
     # 0, and 0 * inf is a NaN in fp32 too.)
-    dout[31, 3] = np.inf
+    dout[31, col] = np.inf
     dout[70, hd + 5] = 3.4e38  # above the largest bf16
     v[:, hd + 5] *= np.float32(1e-30)
     tril, full = np.tril(np.ones((L, L), bool)), np.ones((L, L), bool)
