@@ -459,17 +459,17 @@ struct QgStage {
           r[i][x] = *reinterpret_cast<const vf4 *>(p);
         } else {
 #pragma unroll
-          for (int c = 0; c < 4; ++c) r[i][x][c] = p[min(c, hd - 1 - col)];
+          for (int c = 0; c < 4; ++c) r[i][x][c] = col + c < hd ? p[c] : 0.f;
         }
       }
     }
   }
-  // Without VEC, columns at or past hd were read from column hd - 1 and count as zero
-  // through their factor: a select at the load, with the factor behind it, is scheduled
-  // beside the load and waits for it (42 x 3528, one head of 40: 943 against 820 us
-  // causal, 1843 against 1544 not). A column hd - 1 that is not finite makes NaN of them,
-  // in a row whose own pieces hold NaN already: the recompute below reads them as zeros.
-  __device__ __forceinline__ void store(char *lds, float gscale, int hd) const {
+  // Without VEC the scaling would be scheduled beside the guarded loads and wait for them:
+  // the values pass through an empty asm here first (42 x 3528, one head of 40: 943 -> 832 us
+  // causal, 1843 -> 1524 not).  Zeroing the padding through the factor instead takes as long
+  // but holds a dozen registers more: 200 against 172 us, 8 x 1024 with four heads of 20 under
+  // a mask, where it spilled.
+  __device__ __forceinline__ void store(char *lds, float gscale) const {
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
       const float scale = (NU == 1 ? gside : i == 1) ? gscale : kSplitScale;
@@ -477,8 +477,10 @@ struct QgStage {
       uint32_t w[3][4];  // [piece][dim]: query `row` in the low half, `row + 1` in the high half
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const float f = VEC || col + c < hd ? (c & 1 ? -scale : scale) : 0.f;
-        split_bf16x3(r[i][0][c] * f, r[i][1][c] * f, w[0][c], w[1][c], w[2][c]);
+        const float f = c & 1 ? -scale : scale;
+        float r0 = r[i][0][c], r1 = r[i][1][c];
+        if constexpr (!VEC) asm volatile("" : "+v"(r0), "+v"(r1));
+        split_bf16x3(r0 * f, r1 * f, w[0][c], w[1][c], w[2][c]);
       }
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
@@ -728,7 +730,7 @@ __global__ void __launch_bounds__(paired_keys(HD) ? 2 * BW_THREADS : BW_THREADS,
       }
     };
     auto stage = [&](int buf) {
-      sg.store(lds[buf], gsgn * kSplitScale, a.hd);
+      sg.store(lds[buf], gsgn * kSplitScale);
       if (t < BQ) {
         Ls[buf][t] = lreg;
         Ds[buf][t] = dreg;

@@ -353,7 +353,7 @@ def test_attention_backward(hd, L):
             check_backward(backward(q, k, v, dout, heads, scale, causal, stored=True), want, what + " stored dS")
 
 
-# the scalar loads of head dims 20 and 40 read the last column for those past it
+# head dims 20 and 40: scalar loads, the last column beside those that count as zero
 @pytest.mark.parametrize("hd,col", [(32, 3), (64, 3), (20, 19), (40, 39)])
 def test_attention_backward_values_outside_the_split(hd, col):
     """An infinite and a huge output gradient: the keys they reach get what the fp32 products give, the others
